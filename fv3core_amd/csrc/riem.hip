@@ -4,28 +4,30 @@
 // Reference: fv3core/stencils/sim1_solver.py:11-101 (two tridiagonal
 // solves, for the pressure perturbation and for w, plus the dz update),
 // riem_solver_c.py:13-165 and riem_solver3.py:24-242 (precompute / sim1 /
-// finalize stencils).  Here each solver is one kernel: one thread owns one
-// column, always in FP64, and lanes of a wave own neighbouring i, so each
-// k-indexed access is coalesced.
+// finalize stencils).  Each solver is one kernel, always in FP64, that reads
+// every input level once (pt, cappa and w a second time at the end, which
+// frees their registers in between) and keeps all intermediates on chip.
 //
-// The stencils' ten FORWARD/BACKWARD passes become six sweeps: precompute,
-// the pe evaluation and the pp forward elimination run as one upward sweep;
-// then the pp back substitution (down), the w forward elimination (up), the
-// w back substitution (down), the pe update with the finalize of pe / pk /
-// ppe (up) and the dz update with the height integration (down).  Of the
-// two column arrays a sweep hands to the next one in the opposite
-// direction, one (pp, then w) lives in LDS, 40 KB per wave at 80 levels so
-// that four waves fit a CU and every wave of a C96 cube is resident at once,
-// and the other (gam, aa, the w factors, the new pe) in one workspace slab;
-// dm, dz, pem and pk3 are recomputed from the inputs wherever a sweep needs
-// them (by the same operations, so with the same bits), and pem / pm, which
-// only an upward running sum produces, go to two more slabs.
+// What bounds it: nearly all of the ~1000 instructions a column-level takes
+// are the logs, exps and divisions of pressures and coefficients, which
+// depend on their own level only; what one level hands to the next is two
+// division chains and a few sums.  One thread per column (as these kernels
+// were) runs everything in sequence, at less than one wave per SIMD on a C96
+// cube, and reads the inputs again in each of six sweeps.  Here a column's
+// levels are spread over a workgroup: RC columns by sets of LV levels, two
+// sets to a wave.  Every thread forms the independent part of its levels in
+// registers, and the recurrences run as chains: the waves take turns, each
+// carrying the running values through its levels and handing them on through
+// LDS.  Sums and recurrences keep the order of the stencils' sweeps, so the
+// results are those of the one-thread form bit for bit.
 //
-// A C96 cube has ~55k columns, under one wave per SIMD, so every sweep
-// walks k in chunks of KC levels: the chunk's loads (which never depend on
-// the values the sweep carries from level to level) are issued together
-// into registers, then the recurrence runs on them and the results are
-// stored.  Each chunk waits for memory once instead of once per level.
+// Measured (RiemannSolver3, last call, 79 levels, one MI355X; one thread per
+// column -> levels spread): six C12 tiles 224 -> 45 us, six C51 193 -> 66 us,
+// six C96 303 -> 240 us, six C128 628 -> 404 us, 96 C48 tiles with FP32
+// inputs 1246 -> 1013 us.  One workgroup takes about 104 k cycles, of which
+// the chains take 60 k; with two to a CU one's chains run beside the other's
+// independent parts.  64 columns by 10 levels (a whole wave per set, one
+// workgroup per CU) measured 342 us on six C96 tiles.
 #include "common.hpp"
 #include "timing.hpp"
 
@@ -34,10 +36,37 @@ namespace fv3 {
 constexpr double kRdgas = 287.05;
 constexpr double kGrav = 9.80665;
 constexpr double kCpAir = 1004.6;
-constexpr int KC = 8;       // levels per chunk of a column sweep
-constexpr int RW = 64;      // columns per workgroup (one wave)
+constexpr int RC = 32;      // columns per workgroup (half a wave)
 
 __device__ __forceinline__ double gm_of(double cp3) { return 1.0 / (1.0 - cp3); }
+
+// A refined reciprocal and the quotients by it: the Newton steps and the
+// final residual correction (Markstein) of the compiler's own division, so a
+// quotient has the bits of a / b wherever neither operand nor quotient is
+// near the ends of the exponent range (here: ratios of layer masses and
+// pressures).  Chains that divide twice by one value share the reciprocal.
+struct Recip {
+  double b, y;
+  __device__ __forceinline__ explicit Recip(double v) : b(v) {
+    const double y0 = __builtin_amdgcn_rcp(v);
+    const double y1 = fma(y0, fma(-v, y0, 1.0), y0);
+    y = fma(y1, fma(-v, y1, 1.0), y1);
+  }
+  __device__ __forceinline__ double quot(double a) const {
+    const double q = a * y;
+    return fma(fma(-b, q, a), y, q);
+  }
+};
+
+// The low (hi = false) or high half-wave's value in both halves.
+__device__ __forceinline__ double half_bcast(double v, bool hi) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)u, up = (unsigned)(u >> 32);
+  const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(up, up, false, false);
+  return __builtin_bit_cast(double, hi ? ((unsigned long long)b[1] << 32) | a[1]
+                                       : ((unsigned long long)b[0] << 32) | a[0]);
+}
 
 struct Box2 {
   int i1, j1, nib, njb;
@@ -64,37 +93,56 @@ struct RiemFields {
   S* w;
   double* pef;                                  // C only
   double *delz, *pe, *ppe, *pk3, *pk, *peln;    // 3 only
-  double* work;
-  int64_t slab;
 };
+
+constexpr int kRiemMaxLevels = 128;
 
 // C = true: RiemannSolverC (riem_solver_c.py:13-64); false: RiemannSolver3
 // (riem_solver3.py:24-103).  The sim1 arithmetic (sim1_solver.py:11-101) is
 // shared and evaluated in the stencils' order.
-template <bool C, typename S>
-__global__ void __launch_bounds__(RW)
+//
+// Thread (x, y) holds column x & 31 and, as set 2 y + (x >> 5), the layers
+// k0 .. k0 + LV - 1 of it (k0 = set LV); layers at and past nz compute on
+// clamped loads and reach no store.  slot[] passes a chain's carried values
+// from one wave to the next; xch[] a set's first or last level to its
+// neighbours.  At most five column arrays are alive at a time (2 LV registers
+// each), so that two workgroups fit a CU: gm, gr and w are formed or loaded a
+// second time instead of kept.
+template <bool C, typename S, typename OFF, int LV, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV <= 5 ? 4 : 2)))
     riem_kernel(Dom d, Box2 bx, Riem3Opts o, double dt, double p_fac, RiemFields<S> f) {
-  extern __shared__ double lds_y[];
-  const int64_t n = (int64_t)blockIdx.x * RW + threadIdx.x;
-  if (n >= (int64_t)bx.nib * bx.njb) return;
-  const int i = bx.i1 + (int)(n % bx.nib), j = bx.j1 + (int)(n / bx.nib);
+  extern __shared__ double lds[];
+  const int col = threadIdx.x & (RC - 1), half = threadIdx.x >> 5, nwave = blockDim.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int set = 2 * wave + half;
+  double* const slot = lds;                 // 2 x 2 x RC
+  double* const bot = slot + 4 * RC;        // pp at the surface
+  double* const xch = bot + RC;             // 2 x (2 nwave + 2) x RC
+  // pm waits in LDS until the end (each thread its own entries)
+  double* const pm = xch + 2 * (2 * nwave + 2) * RC + set * LV * RC + col;
+  auto sl = [&](int v, int w) -> double& { return slot[(v * 2 + (w & 1)) * RC + col]; };
+  auto xc = [&](int v, int w) -> double& { return xch[(v * (2 * nwave + 2) + w + 1) * RC + col]; };
+
+  const int ncol = bx.nib * bx.njb;
+  const int n0 = (int)blockIdx.x * RC + col;
+  const bool keep = n0 < ncol;  // columns past the box: clamped loads, no stores
+  const int n = keep ? n0 : ncol - 1;
+  const int i = bx.i1 + n % bx.nib, j = bx.j1 + n / bx.nib;
   const int t = blockIdx.y;
-  const int64_t c = (int64_t)t * d.st + (int64_t)j * d.sj + i;
   const int64_t c2 = (int64_t)t * d.st2 + (int64_t)j * d.sj2 + i;
-  const int64_t sk = d.sk;
-  const int nk = d.nk, nz = nk - 1;
-  auto at = [sk](int k) { return (int64_t)k * sk; };
-  double* const Y = lds_y + threadIdx.x;  // Y[k * RW]: pp, then w
-  auto y = [Y](int k) -> double& { return Y[k * RW]; };
-  double* const X = f.work + c;                 // gam / aa / gam2 / new pe
-  double* const PEM = f.work + f.slab + c;      // pem (interfaces)
-  double* const PM = f.work + 2 * f.slab + c;   // pm (layers)
-  const S* const CP = f.cappa + c;
-  const S* const QC = f.qc + c;
-  const S* const DP = f.dp + c;
-  const S* const PT = f.pt + c;
-  double* const Z = f.z + c;
-  S* const W = f.w + c;
+  const int nz = d.nk - 1;
+  const int k0 = set * LV;
+  // fields are addressed as a tile's uniform base plus the lane's offset in
+  // elements, layers past the bottom clamped to it
+  const int64_t tb = (int64_t)t * d.st;
+  const OFF sk = (OFF)d.sk;
+  const OFF c = (OFF)j * (OFF)d.sj + (OFF)i;
+  auto ptr = [tb](auto* base, OFF e) {
+    typedef decltype(base) P;
+    return (P)((const char*)(base + tb) + (size_t)(OFF)(e * (OFF)sizeof(*base)));
+  };
+  auto lay = [&](int u) -> OFF { return c + (OFF)min(k0 + u, nz - 1) * sk; };
+  auto itf = [&](int u) -> OFF { return c + (OFF)min(k0 + u, nz) * sk; };
   const double ptop = o.ptop;
   const double t1g = 2.0 * dt * dt;
   const double rdt = 1.0 / dt;
@@ -105,294 +153,344 @@ __global__ void __launch_bounds__(RW)
     else
       return dpk * rgrav;
   };
+  // The waves exchange through LDS only, so a barrier waits for LDS alone
+  // (__syncthreads would also wait for every load and store in flight).
+  auto barrier = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  // A chain up (down) the column: the waves take turns, each its lower (upper)
+  // set first, on the values v0, v1 the one before left.  Every wave passes
+  // nwave barriers.
+  auto chain = [&](bool up, double v0, double v1, auto body) {
+    const int turn = up ? wave : nwave - 1 - wave;
+    for (int w = 0; w < turn; ++w) barrier();
+    if (turn > 0) {
+      v0 = sl(0, turn);
+      v1 = sl(1, turn);
+    }
+    if (half == (up ? 0 : 1)) body(v0, v1);
+    v0 = half_bcast(v0, !up);
+    v1 = half_bcast(v1, !up);
+    if (half == (up ? 1 : 0)) {
+      body(v0, v1);
+      sl(0, turn + 1) = v0;
+      sl(1, turn + 1) = v1;
+    }
+    for (int w = turn; w < nwave; ++w) barrier();
+  };
 
-  // ---- S1 (up): precompute, pe = exp(gm log(-dm/dz Rd pt)) - pm, and the pp
-  // forward elimination, which lags one level behind (it needs pe and dm of
-  // the level below)
-  double z_k = Z[0];
-  double pem_k = ptop, peg_k = ptop, pelng_k = o.peln1;
-  PEM[0] = ptop;
-  double gr_prev = 0.0, bet_prev = 2.0, pp_k = 0.0, dm_k = 0.0, pe_k = 0.0;
-  y(0) = 0.0;
-  for (int k0 = 0; k0 < nz; k0 += KC) {
-    double dp[KC], qc[KC], z1[KC], pt[KC], cp[KC];
+  // ---- inputs, then chain A (up): the interface sums pem (of dp) and peg
+  // (of the dry part); entry u holds the interface below layer k0 + u
+  double dm[LV], pem[LV], dz[LV], g[LV], p[LV];
+  double pem0 = ptop, peg0 = ptop;  // the set's top interface
 #pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      const int k = min(k0 + u, nz - 1);
-      dp[u] = DP[at(k)];
-      qc[u] = QC[at(k)];
-      z1[u] = Z[at(k + 1)];
-      pt[u] = PT[at(k)];
-      cp[u] = CP[at(k)];
+  for (int u = 0; u < LV; ++u) {
+    const double dp = *ptr(f.dp, lay(u)), qc = *ptr(f.qc, lay(u));
+    const bool in = k0 + u < nz;  // layers past the bottom add nothing
+    pem[u] = in ? dp : 0.0;
+    g[u] = in ? dp * (1.0 - qc) : 0.0;
+    dm[u] = dm_of(dp);
+  }
+  {
+    double z = *ptr(f.z, itf(0));
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const double zn = *ptr(f.z, itf(u + 1));
+      dz[u] = zn - z;
+      z = zn;
+    }
+  }
+  chain(true, ptop, ptop, [&](double& a, double& b) {
+    pem0 = a;
+    peg0 = b;
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      a = a + pem[u];
+      b = b + g[u];
+      pem[u] = a;
+      g[u] = b;
+    }
+  });
+  // ---- precompute: pm and pe = exp(gm log(-dm/dz Rd pt)) - pm (into p)
+  {
+    double pg = peg0, lg = 0.0;
+    if constexpr (!C) lg = k0 == 0 ? o.peln1 : log(pg);
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      double pmk;
+      if constexpr (C) {
+        pmk = (g[u] - pg) / log(g[u] / pg);
+      } else {
+        const double ln = log(g[u]);
+        pmk = (g[u] - pg) / (ln - lg);
+        lg = ln;
+      }
+      pg = g[u];
+      pm[u * RC] = pmk;
+      const double pt = *ptr(f.pt, lay(u)), cp = *ptr(f.cappa, lay(u));
+      p[u] = exp(gm_of(cp) * log(-dm[u] / dz[u] * kRdgas * pt)) - pmk;
+    }
+  }
+  xc(0, set) = dm[0];
+  xc(1, set) = p[0];
+  barrier();
+  // ---- chain B (up): pp forward elimination (sim1_solver.py:42-56) of
+  // bb = 2 (1 + gr), dd = 3 (pe_k + gr pe_k+1); gr (in g) becomes gam, dd (in
+  // p) pp of the layer's top interface
+  double ppn = 0.0;  // pp at the set's bottom interface
+  {
+    const double dmn = xc(0, set + 1), pen = xc(1, set + 1);
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const bool last = k0 + u >= nz - 1;
+      const double dm1 = u + 1 < LV ? dm[u + 1 < LV ? u + 1 : u] : dmn;
+      const double pe1 = u + 1 < LV ? p[u + 1 < LV ? u + 1 : u] : pen;
+      g[u] = last ? 0.0 : dm[u] / dm1;
+      p[u] = last ? 3.0 * p[u] : 3.0 * (p[u] + g[u] * pe1);
+    }
+    chain(true, 0.0, 0.0, [&](double& pk, double& gk) {
+#pragma unroll
+      for (int u = 0; u < LV; ++u) {
+        const double gr = g[u], dd = p[u];
+        g[u] = gk;
+        p[u] = pk;
+        const Recip r(2.0 * (1.0 + gr) - gk);  // gr = 0 in the bottom layer
+        pk = r.quot(dd - pk);
+        gk = r.quot(gr);  // the next layer's gam = gr_k / bet_k
+        if (k0 + u == nz - 1) bot[col] = pk;
+      }
+    });
+    // layers past the bottom hand pp of interface nz up unchanged
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      if (k0 + u >= nz) {
+        p[u] = 0.0;
+        g[u] = -1.0;
+      }
+    }
+  }
+  // ---- chain C (down): pp back substitution; from the surface
+  chain(false, bot[col], 0.0, [&](double& pk, double&) {
+    ppn = pk;  // pp at the bottom interface (nz, where the layers end)
+#pragma unroll
+    for (int u = LV - 1; u >= 0; --u) {
+      p[u] = p[u] - g[u] * pk;  // gam = 0 in layer 0
+      pk = p[u];
+    }
+  });
+  // ---- aa of layers 1 .. nz - 1 (sim1_solver.py:57-66, into g) and the
+  // surface's p1, then the right-hand sides of w (into p)
+  double ab = 0.0;  // aa below the set's last layer
+  {
+    const double gml = gm_of(*ptr(f.cappa, lay(LV - 1)));
+    xc(0, set) = gml;
+    xc(1, set) = dz[LV - 1];
+    barrier();
+    double gm0 = xc(0, set - 1), dz0 = xc(1, set - 1);
+    double pe0 = pem0;
+    const double wsr = f.wsd[c2];
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const int k = k0 + u;
+      const double gmk = u + 1 < LV ? gm_of(*ptr(f.cappa, lay(u))) : gml;
+      const double pn = u + 1 < LV && k + 1 < nz ? p[u + 1 < LV ? u + 1 : u] : ppn;
+      const double w1 = *ptr(f.w, lay(u));
+      g[u] = k == 0 ? 0.0 : t1g * 0.5 * (gm0 + gmk) / (dz0 + dz[u]) * (pe0 + p[u]);
+      const double rhs = k == 0 ? dm[u] * w1 + dt * pn : dm[u] * w1 + dt * (pn - p[u]);
+      gm0 = gmk;
+      dz0 = dz[u];
+      pe0 = pem[u];
+      if (k == nz - 1) {
+        // dz of the bottom layer makes room for p1, which takes aa's place below it
+        dz[u] = t1g * gmk / dz[u] * (pem[u] + pn);
+        p[u] = rhs - dz[u] * wsr;
+        ab = dz[u];
+      } else {
+        p[u] = rhs;
+      }
+    }
+    barrier();
+    xc(0, set) = g[0];
+    barrier();
+    if (k0 + LV < nz) ab = xc(0, set + 1);
+  }
+  // ---- chain D (up): w forward elimination; aa (in g) becomes the back
+  // substitution's factor, the right-hand side (in p) w
+  chain(true, 1.0, 0.0, [&](double& bet, double& wp) {
+    // aa = 0 in layer 0: gam = 0, bet = dm - an there
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const double an = u + 1 < LV && k0 + u != nz - 1 ? g[u + 1 < LV ? u + 1 : u] : ab;
+      const Recip r(bet);
+      const double gam = r.quot(g[u]);
+      bet = dm[u] - (g[u] + an + g[u] * gam);
+      wp = (p[u] - g[u] * wp) / bet;
+      p[u] = wp;
+      g[u] = gam;
+    }
+  });
+#pragma unroll
+  for (int u = 0; u < LV; ++u)
+    if (k0 + u >= nz) p[u] = g[u] = 0.0;
+  // ---- chain E (down): w back substitution; carries gam_k+1 w_k+1
+  chain(false, 0.0, 0.0, [&](double& gw, double&) {
+#pragma unroll
+    for (int u = LV - 1; u >= 0; --u) {
+      p[u] = p[u] - gw;
+      gw = g[u] * p[u];
+    }
+  });
+  // ---- chain F (up): pe from the change of w (into p), of the interface
+  // below
+#pragma unroll
+  for (int u = 0; u < LV; ++u) {
+    const double w1 = *ptr(f.w, lay(u));
+    const double wk = p[u];
+    p[u] = k0 + u < nz ? dm[u] * (wk - w1) * rdt : 0.0;
+    if constexpr (!C) {
+      if (keep && k0 + u < nz) *ptr(f.w, lay(u)) = (S)wk;
+    }
+  }
+  double pet = 0.0;  // the set's top interface
+  chain(true, 0.0, 0.0, [&](double& a, double&) {
+    pet = a;
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      a = a + p[u];
+      p[u] = a;
+    }
+  });
+  // ---- finalize of the interface pressures
+  if (keep) {
+    if (set == 0) {
+      if constexpr (C) {
+        *ptr(f.pef, c) = ptop;
+      } else {
+        const double pk3k = o.use_logp ? o.peln1 : o.ptk;
+        *ptr(f.pk3, c) = pk3k;
+        *ptr(f.ppe, c) = o.beta < -0.1 ? 0.0 + ptop : 0.0;  // new pe is 0 at the top
+        if (o.last_call) {
+          *ptr(f.peln, c) = o.peln1;
+          *ptr(f.pk, c) = pk3k;
+          *ptr(f.pe, c) = ptop;
+        }
+      }
     }
 #pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      const int m = k0 + u;
-      if (m < nz) {
-        const double dmk = dp[u];
-        const double dm = dm_of(dmk);
-        const double dz = z1[u] - z_k;
-        const double peg_n = peg_k + dmk * (1.0 - qc[u]);
-        double pm;
+    for (int u = 0; u < LV; ++u) {
+      if (k0 + u < nz) {
+        const OFF ob = itf(u + 1);
         if constexpr (C) {
-          pm = (peg_n - peg_k) / log(peg_n / peg_k);
-          pem_k = pem_k + dmk;
+          *ptr(f.pef, ob) = p[u] + pem[u];
         } else {
-          const double pem_n = pem_k + dmk;
-          const double pelng_n = log(peg_n);
-          pm = (peg_n - peg_k) / (pelng_n - pelng_k);
-          pem_k = pem_n;
-          pelng_k = pelng_n;
-        }
-        peg_k = peg_n;
-        PEM[at(m + 1)] = pem_k;
-        PM[at(m)] = pm;
-        z_k = z1[u];
-        const double pe = exp(gm_of(cp[u]) * log(-dm / dz * kRdgas * pt[u])) - pm;
-        // pp forward elimination for level m - 1 (sim1_solver.py:42-56)
-        if (m == 0) {
-          dm_k = dm;
-          pe_k = pe;
-        } else if (m == 1) {
-          gr_prev = dm_k / dm;
-          bet_prev = 2.0 * (1.0 + gr_prev);
-          pp_k = 3.0 * (pe_k + gr_prev * pe) / bet_prev;
-          y(1) = pp_k;
-          dm_k = dm;
-          pe_k = pe;
-        } else {
-          const int k = m - 1;
-          const double g = gr_prev / bet_prev;
-          X[at(k)] = g;
-          const double gr = dm_k / dm;
-          const double bb = 2.0 * (1.0 + gr);
-          const double dd = 3.0 * (pe_k + gr * pe);
-          const double bet_k = bb - g;
-          pp_k = (dd - pp_k) / bet_k;
-          y(k + 1) = pp_k;
-          bet_prev = bet_k;
-          gr_prev = gr;
-          dm_k = dm;
-          pe_k = pe;
-        }
-      }
-    }
-  }
-  {
-    // last level of the elimination (bb = 2, dd = 3 pe)
-    const int k = nz - 1;
-    const double g = gr_prev / bet_prev;
-    X[at(k)] = g;
-    const double bet_k = 2.0 - g;
-    pp_k = (3.0 * pe_k - pp_k) / bet_k;
-    y(k + 1) = pp_k;
-  }
-
-  // ---- S2 (down): pp back substitution and aa (k = nz-1 .. 1)
-  {
-    double pp_next = y(nz);
-    double cpk = CP[at(nz - 1)];
-    double zk = Z[at(nz - 1)];
-    double dzk = Z[at(nz)] - zk;
-    for (int k0 = nz - 1; k0 >= 1; k0 -= KC) {
-      double gam[KC], cpm[KC], zm[KC], pem[KC];
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = max(k0 - u, 1);
-        gam[u] = X[at(k)];
-        cpm[u] = CP[at(k - 1)];
-        zm[u] = Z[at(k - 1)];
-        pem[u] = PEM[at(k)];
-      }
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = k0 - u;
-        if (k >= 1) {
-          const double dzm = zk - zm[u];
-          const double ppk = y(k) - gam[u] * pp_next;
-          y(k) = ppk;
-          X[at(k)] = t1g * 0.5 * (gm_of(cpm[u]) + gm_of(cpk)) / (dzm + dzk) * (pem[u] + ppk);
-          pp_next = ppk;
-          cpk = cpm[u];
-          zk = zm[u];
-          dzk = dzm;
-        }
-      }
-    }
-  }
-
-  // ---- S3 (up): w forward elimination (w1 = w on entry, gam into X)
-  const double wsr = f.wsd[c2];
-  double w_prev;
-  {
-    double aa_k = X[at(1)];
-    double pp_c = y(1);
-    const double dm0 = dm_of(DP[at(0)]);
-    double bet = dm0 - aa_k;
-    w_prev = (dm0 * W[at(0)] + dt * pp_c) / bet;
-    y(0) = w_prev;
-    for (int k0 = 1; k0 < nz; k0 += KC) {
-      double aan[KC], dp[KC], w1[KC];
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = min(k0 + u, nz - 1);
-        aan[u] = X[at(min(k + 1, nz - 1))];
-        dp[u] = DP[at(k)];
-        w1[u] = W[at(k)];
-      }
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = k0 + u;
-        if (k < nz) {
-          const double dm = dm_of(dp[u]);
-          const double ppn = y(k + 1);
-          const double g = aa_k / bet;
-          X[at(k)] = g;
-          double wk, b;
-          if (k < nz - 1) {
-            b = dm - (aa_k + aan[u] + aa_k * g);
-            wk = (dm * w1[u] + dt * (ppn - pp_c) - aa_k * w_prev) / b;
-          } else {
-            const double dzl = Z[at(k + 1)] - Z[at(k)];
-            const double p1 = t1g * gm_of(CP[at(k)]) / dzl * (PEM[at(k + 1)] + ppn);
-            b = dm - (aa_k + p1 + aa_k * g);
-            wk = (dm * w1[u] + dt * (ppn - pp_c) - p1 * wsr - aa_k * w_prev) / b;
-          }
-          y(k) = wk;
-          w_prev = wk;
-          bet = b;
-          pp_c = ppn;
-          if (k + 1 < nz) aa_k = aan[u];
-        }
-      }
-    }
-  }
-
-  // ---- S4 (down): w back substitution (k = nz-2 .. 0)
-  {
-    double w_next = w_prev;  // w[nz-1]
-    for (int k0 = nz - 2; k0 >= 0; k0 -= KC) {
-      double gam[KC];
-#pragma unroll
-      for (int u = 0; u < KC; ++u) gam[u] = X[at(max(k0 - u, 0) + 1)];
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = k0 - u;
-        if (k >= 0) {
-          w_next = y(k) - gam[u] * w_next;
-          y(k) = w_next;
-        }
-      }
-    }
-  }
-
-  // ---- S5 (up): pe from the change of w (new pe into X), and the finalize
-  // of the interface pressures; pem is re-summed as the precompute summed it
-  {
-    double pe_run = 0.0;
-    X[at(0)] = 0.0;
-    double pem = ptop;
-    if constexpr (C) {
-      f.pef[c] = ptop;
-    } else {
-      const double pk3k = o.use_logp ? o.peln1 : o.ptk;
-      f.pk3[c] = pk3k;
-      f.ppe[c] = 0.0;  // new pe is 0 at the top; beta < -0.1 adds pem
-      if (o.beta < -0.1) f.ppe[c] = 0.0 + pem;
-      if (o.last_call) {
-        f.peln[c] = o.peln1;
-        f.pk[c] = pk3k;
-        f.pe[c] = pem;
-      }
-    }
-    for (int k0 = 1; k0 < nk; k0 += KC) {
-      double dp[KC], w1[KC];
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = min(k0 + u, nk - 1);
-        dp[u] = DP[at(k - 1)];
-        w1[u] = W[at(k - 1)];
-      }
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = k0 + u;
-        if (k < nk) {
-          const double wk = y(k - 1);
-          pe_run = pe_run + dm_of(dp[u]) * (wk - w1[u]) * rdt;
-          X[at(k)] = pe_run;
-          pem = pem + dp[u];
-          if constexpr (C) {
-            f.pef[c + at(k)] = pe_run + pem;
-          } else {
-            W[at(k - 1)] = (S)wk;
-            const double peln_run = log(pem);
-            const double pk3k = o.use_logp ? peln_run : exp(o.kappa * peln_run);
-            f.pk3[c + at(k)] = pk3k;
-            f.ppe[c + at(k)] = o.beta < -0.1 ? pe_run + pem : pe_run;
-            if (o.last_call) {
-              f.peln[c + at(k)] = peln_run;
-              f.pk[c + at(k)] = pk3k;
-              f.pe[c + at(k)] = pem;
-            }
+          const double peln = log(pem[u]);
+          const double pk3k = o.use_logp ? peln : exp(o.kappa * peln);
+          *ptr(f.pk3, ob) = pk3k;
+          *ptr(f.ppe, ob) = o.beta < -0.1 ? p[u] + pem[u] : p[u];
+          if (o.last_call) {
+            *ptr(f.peln, ob) = peln;
+            *ptr(f.pk, ob) = pk3k;
+            *ptr(f.pe, ob) = pem[u];
           }
         }
       }
     }
   }
-
-  // ---- S6 (down): p1 and the dz update (sim1_solver.py:90-101), then the
+  // ---- chain G (down): p1 (sim1_solver.py:90-96, into p), its own-level
+  // part first; gr formed again
+  xc(0, set) = p[0];
+  xc(1, set) = dm[0];
+  barrier();
+  {
+    const double pen = xc(0, set + 1), dmn = xc(1, set + 1);
+    double pa = pet;
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const bool last = k0 + u >= nz - 1;
+      const double pc = u + 1 < LV ? p[u + 1 < LV ? u + 1 : u] : pen;
+      const double dm1 = u + 1 < LV ? dm[u + 1 < LV ? u + 1 : u] : dmn;
+      const double pb = p[u];
+      g[u] = last ? 0.0 : dm[u] / dm1;
+      p[u] = last ? (pa + 2.0 * pb) * 1.0 / 3.0
+                  : (pa + 2.0 * (1.0 + g[u]) * pb + g[u] * pc) * 1.0 / 3.0;
+      pa = pb;
+    }
+  }
+  chain(false, 0.0, 0.0, [&](double& a, double&) {
+#pragma unroll
+    for (int u = LV - 1; u >= 0; --u) {
+      p[u] = p[u] - g[u] * a;  // gr = 0 in the bottom layer
+      a = p[u];
+    }
+  });
+  // ---- the dz update (sim1_solver.py:97-101), then chain H (down): the
   // height / geopotential integration from the surface
-  {
-    double p1_next = 0.0;
-    double pe1 = X[at(nz)], pe2 = 0.0, dm1 = 0.0;
-    double zsum = f.surf[c2];
-    Z[at(nz)] = zsum;
-    for (int k0 = nz - 1; k0 >= 0; k0 -= KC) {
-      double pe0[KC], dp[KC], pm[KC], pt[KC], cp[KC];
 #pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = max(k0 - u, 0);
-        pe0[u] = X[at(k)];
-        dp[u] = DP[at(k)];
-        pm[u] = PM[at(k)];
-        pt[u] = PT[at(k)];
-        cp[u] = CP[at(k)];
-      }
-#pragma unroll
-      for (int u = 0; u < KC; ++u) {
-        const int k = k0 - u;
-        if (k >= 0) {
-          const double dm0 = dm_of(dp[u]);
-          double p1;
-          if (k == nz - 1) {
-            p1 = (pe0[u] + 2.0 * pe1) * 1.0 / 3.0;
-          } else {
-            const double gr = dm0 / dm1;
-            const double bb = 2.0 * (1.0 + gr);
-            p1 = (pe0[u] + bb * pe1 + gr * pe2) * 1.0 / 3.0 - gr * p1_next;
-          }
-          p1_next = p1;
-          const double maxp = p_fac * dm0 > p1 + pm[u] ? p_fac * pm[u] : p1 + pm[u];
-          const double dz = -dm0 * kRdgas * pt[u] * exp((cp[u] - 1.0) * log(maxp));
-          if constexpr (C) {
-            zsum = zsum - dz * kGrav;
-          } else {
-            f.delz[c + at(k)] = dz;
-            zsum = zsum - dz;
-          }
-          Z[at(k)] = zsum;
-          pe2 = pe1;
-          pe1 = pe0[u];
-          dm1 = dm0;
-        }
-      }
+  for (int u = 0; u < LV; ++u) {
+    const double pt = *ptr(f.pt, lay(u)), cp = *ptr(f.cappa, lay(u));
+    const double pmk = pm[u * RC];
+    const double maxp = p_fac * dm[u] > p[u] + pmk ? p_fac * pmk : p[u] + pmk;
+    const double dzn = -dm[u] * kRdgas * pt * exp((cp - 1.0) * log(maxp));
+    if constexpr (!C) {
+      if (keep && k0 + u < nz) *ptr(f.delz, lay(u)) = dzn;
     }
+    g[u] = k0 + u < nz ? (C ? dzn * kGrav : dzn) : 0.0;
+  }
+  const double surf = f.surf[c2];
+  chain(false, surf, 0.0, [&](double& a, double&) {
+#pragma unroll
+    for (int u = LV - 1; u >= 0; --u) {
+      a = a - g[u];
+      g[u] = a;
+    }
+  });
+  if (keep) {
+    if (set == 0) *ptr(f.z, c + (OFF)nz * sk) = surf;
+#pragma unroll
+    for (int u = 0; u < LV; ++u)
+      if (k0 + u < nz) *ptr(f.z, lay(u)) = g[u];
   }
 }
 
-// one column array of RW columns per wave in LDS: 64 KB at most
-constexpr int kRiemMaxLevels = 128;
-static size_t riem_lds_bytes(int nk) { return (size_t)nk * RW * sizeof(double); }
+template <int LV>
+int riem_waves(int nk) {
+  return (nk - 1 + 2 * LV - 1) / (2 * LV);
+}
+template <int LV>
+size_t riem_lds_bytes(int nk) {
+  const int nw = riem_waves<LV>(nk);
+  return (size_t)(5 + 2 * (2 * nw + 2) + 2 * nw * LV) * RC * sizeof(double);
+}
+
+// every byte offset in a tile fits 32 bits
+static bool riem_narrow(const fv3_domain* dom) {
+  return ((int64_t)dom->nk * dom->sk) * (int64_t)sizeof(double) < (int64_t)1 << 32;
+}
+
+template <bool C, typename S, typename OFF, int LV, int NW>
+void riem_launch_as(const fv3_domain* dom, hipStream_t s, const Dom& d, Box2 bx,
+                    const Riem3Opts& o, double dt, double p_fac, const RiemFields<S>& f) {
+  const dim3 grid((unsigned)((bx.nib * bx.njb + RC - 1) / RC), (unsigned)d.ntiles);
+  hipLaunchKernelGGL((riem_kernel<C, S, OFF, LV, NW>), grid, dim3(64, riem_waves<LV>(dom->nk)),
+                     riem_lds_bytes<LV>(dom->nk), s, d, bx, o, dt, p_fac, f);
+}
+
+template <bool C, typename S>
+void riem_launch(const fv3_domain* dom, hipStream_t s, const Dom& d, Box2 bx, const Riem3Opts& o,
+                 double dt, double p_fac, const RiemFields<S>& f) {
+  // 5 levels a thread up to 80 layers: 8 waves of 128 registers, two
+  // workgroups to a CU.  Above that 8 levels a thread (up to 128 layers), one
+  // workgroup to a CU: 100 layers on six C96 tiles 594 us with one thread per
+  // column, 454 us so, 639 us squeezed into 128 registers.
+  if (!riem_narrow(dom))
+    riem_launch_as<C, S, int64_t, 8, 8>(dom, s, d, bx, o, dt, p_fac, f);
+  else if (riem_waves<5>(dom->nk) <= 8)
+    riem_launch_as<C, S, uint32_t, 5, 8>(dom, s, d, bx, o, dt, p_fac, f);
+  else
+    riem_launch_as<C, S, uint32_t, 8, 8>(dom, s, d, bx, o, dt, p_fac, f);
+}
 
 static int check_riem(const fv3_domain* dom, const char* who, int i1, int i2, int j1, int j2,
                       int64_t slab, int nslabs) {
@@ -439,15 +537,11 @@ int riem_solver_c(const fv3_domain* dom, double dt2, double ptop, double p_fac, 
   f.z = gz;
   f.w = const_cast<S*>(w3);  // read only in this solver
   f.pef = pef;
-  f.work = work;
-  f.slab = work_slab;
-  dim3 grid((unsigned)(((int64_t)bx.nib * bx.njb + RW - 1) / RW), d.ntiles);
   // cappa, ptc, q_con, delpc, gz, w3 read; gz, pef written (per cell-level)
   TimedLaunch timed("riem_c_kernel", as_stream(stream),
                     (4.0 * sizeof(S) + 4.0 * sizeof(double)) * bx.nib * bx.njb *
                         (double)dom->nk * d.ntiles);
-  hipLaunchKernelGGL((riem_kernel<true, S>), grid, dim3(RW), riem_lds_bytes(dom->nk),
-                     as_stream(stream), d, bx, o, dt2, p_fac, f);
+  riem_launch<true, S>(dom, as_stream(stream), d, bx, o, dt2, p_fac, f);
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }
@@ -499,16 +593,12 @@ int riem_solver3(const fv3_domain* dom, int last_call, double dt, double ptop, d
   f.pk3 = pk3;
   f.pk = pk;
   f.peln = peln;
-  f.work = work;
-  f.slab = work_slab;
-  dim3 grid((unsigned)(((int64_t)bx.nib * bx.njb + RW - 1) / RW), d.ntiles);
   // cappa, q_con, delp, pt, zh, w read; zh, ppe, pk3, delz, w written, plus
   // pe, pk and peln on the last call (per cell-level)
   TimedLaunch timed("riem3_kernel", as_stream(stream),
                     ((5.0 * sizeof(S) + (6.0 + 3.0 * o.last_call) * sizeof(double))) * bx.nib * bx.njb *
                         (double)dom->nk * d.ntiles);
-  hipLaunchKernelGGL((riem_kernel<false, S>), grid, dim3(RW), riem_lds_bytes(dom->nk),
-                     as_stream(stream), d, bx, o, dt, p_fac, f);
+  riem_launch<false, S>(dom, as_stream(stream), d, bx, o, dt, p_fac, f);
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }

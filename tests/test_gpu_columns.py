@@ -120,3 +120,113 @@ def test_riem_solver3_parity(last_call, use_logp, beta):
     for name, g, rr in zip(names, got, ref):
         assert_close(to_np(g)[sl], rr, 1e-12, near_zero=1e-12, what=name,
                      scale_floor=floors.get(name, 0.0))
+
+
+class _OneUlp:
+    """numpy with every exp and log result moved by one ulp, up or down."""
+
+    def __init__(self, seed):
+        self._rng = np.random.default_rng(seed)
+
+    def __getattr__(self, name):
+        return getattr(np, name)
+
+    def _moved(self, a):
+        return np.nextafter(a, self._rng.choice([-np.inf, np.inf], size=np.shape(a)))
+
+    def exp(self, a):
+        return self._moved(np.exp(a))
+
+    def log(self, a):
+        return self._moved(np.log(a))
+
+
+# Columns of 3 layers up to the most a workgroup holds: one thread's levels,
+# one more than whole sets, the last layer alone in its set, and both sides
+# of the change from 5 to 8 levels a thread (80 / 81).
+@pytest.mark.parametrize("nz", [3, 5, 6, 10, 11, 41, 80, 81, 127])
+@pytest.mark.parametrize("n", [5, 9])
+def test_riem_solvers_level_counts(nz, n, monkeypatch):
+    from fv3core_amd import workloads
+
+    monkeypatch.setattr(workloads, "hybrid_coefficients", workloads.synthetic_hybrid)
+    r = riemann_inputs(n, nz, workload=90 + nz)
+    factory, gi = _factory(n, nz)
+    t = {k: to_storage(v) for k, v in r.items() if isinstance(v, np.ndarray) and v.ndim >= 2}
+    gz, pef = t["gz"].clone(), utils.zeros(gi.max_shape)
+    RiemannSolverC(factory, 0.05)(r["dt"] / 2, t["cappa"], r["ptop"], t["hs"], t["ws"], t["pt"],
+                                  t["q_con"], t["delp"], gz, pef, t["w"])
+    wsd = np.full(r["zs"].shape, 0.01)
+    delz, zh, pe, w = (t[k].clone() for k in ("delz", "zh", "pe", "w"))
+    ppe, pk3, pk, peln = (utils.zeros(gi.max_shape) for _ in range(4))
+    RiemannSolver3(factory, RiemannConfig(p_fac=0.05, a_imp=1.0, use_logp=False, beta=0.0))(
+        True, r["dt"], t["cappa"], r["ptop"], t["zs"], to_storage(wsd), delz, t["q_con"],
+        t["delp"], t["pt"], zh, pe, ppe, pk3, pk, peln, w)
+    torch.cuda.synchronize()
+    sl = (slice(gi.isc - 1, gi.iec + 2), slice(gi.jsc - 1, gi.jec + 2))
+    rgz, rpef = ori.riem_solver_c(r["dt"] / 2, r["cappa"][sl], r["ptop"], r["hs"][sl],
+                                  r["ws"][sl], r["pt"][sl], r["q_con"][sl], r["delp"][sl],
+                                  r["gz"][sl], r["w"][sl], 0.05)
+    assert_close(to_np(gz)[sl], rgz, 1e-12, what="gz")
+    assert_close(to_np(pef)[sl], rpef, 1e-12, what="pef")
+    sl = (slice(gi.isc, gi.iec + 1), slice(gi.jsc, gi.jec + 1))
+    z = np.zeros(r["pe"].shape)
+
+    def oracle():
+        return ori.riem_solver3(True, r["dt"], r["cappa"][sl], r["ptop"], r["zs"][sl], wsd[sl],
+                                r["delz"][sl], r["q_con"][sl], r["delp"][sl], r["pt"][sl],
+                                r["zh"][sl], r["pe"][sl], z[sl], z[sl], z[sl], z[sl],
+                                r["w"][sl], 0.05)
+
+    ref = oracle()
+    monkeypatch.setattr(ori, "np", _OneUlp(nz))
+    moved = oracle()
+    for name, g, rr, mm in zip(["zh", "pe", "ppe", "pk3", "pk", "peln", "w", "delz"],
+                               [zh, pe, ppe, pk3, pk, peln, w, delz], ref, moved):
+        # ppe and w come out of cancelling terms: they are measured against
+        # the field's scale, within four times what a last-bit difference in
+        # exp and log does there (log enters pm as the difference of
+        # neighbouring levels' logs)
+        tol, floor = 1e-12, 0.0
+        if name in ("ppe", "w"):
+            floor = 0.5
+            tol = max(tol, 4.0 * np.abs(mm - rr).max() / (0.5 * np.abs(rr).max()))
+        assert_close(to_np(g)[sl], rr, tol, near_zero=1e-12, what=name, scale_floor=floor)
+    # outside its box a solver writes nothing
+    for got, was in ((zh, r["zh"]), (delz, r["delz"]), (w, r["w"])):
+        a = to_np(got)
+        a[sl] = was[sl]
+        assert np.array_equal(a, was)
+
+
+def test_riem_solver_c_wide_offsets():
+    """Storages whose levels lie more than 4 GiB apart: 64-bit offsets, the
+    same results as on dense storages."""
+    n, nz = 5, 3
+    ni, nk = n + 7, nz + 1
+    factory, gi = _factory(n, nz)
+    rng = np.random.default_rng(5)
+    dp = rng.uniform(2.0e4, 3.0e4, size=(ni, ni, nk))
+    ins = dict(cappa=np.full(dp.shape, 0.2857), pt=rng.uniform(5.0, 12.0, size=dp.shape),
+               q_con=np.zeros(dp.shape), delp=dp, w=rng.normal(size=dp.shape),
+               gz=np.cumsum(rng.uniform(2e3, 3e3, size=dp.shape)[..., ::-1], axis=2)[..., ::-1])
+    zero = to_storage(np.zeros((ni, ni)))
+    out = []
+    for wide in (False, True):
+        rows = -(-(1 << 27) // ni) + 1 if wide else ni  # (nk - 1) sk 8 B is past 4 GiB
+
+        def store(a):
+            t = torch.empty((nk, rows, ni), dtype=torch.float64, device="cuda")[:, :ni]
+            t = t.permute(2, 1, 0)
+            t.copy_(torch.as_tensor(np.ascontiguousarray(a)))
+            return t
+
+        f = {k: store(a) for k, a in ins.items()}
+        pef = store(np.zeros(dp.shape))
+        RiemannSolverC(factory, 0.05)(18.75, f["cappa"], 300.0, zero, zero, f["pt"], f["q_con"],
+                                      f["delp"], f["gz"], pef, f["w"])
+        out.append((to_np(f["gz"].clone()), to_np(pef.clone())))
+        del f, pef
+        torch.cuda.empty_cache()
+    assert np.isfinite(out[0][0]).all()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
