@@ -15,8 +15,8 @@ namespace fv3 {
 // Wave-strip march.  One wave (64 lanes) owns a strip of 64 columns of one
 // level of one tile: 58 output interfaces in i plus a 3-cell halo on each
 // side, lane L <-> column i0 - 3 + L.  It marches up the rows of a segment of
-// SEG output rows (MTJ or MTJ_TALL, chosen per launch; SEG + 6 march steps,
-// a multiple of the unroll factor 3).  Stencils across i read the neighbouring lanes' values
+// output rows (their number chosen per launch), 6 halo rows with them, in
+// groups of three steps.  Stencils across i read the neighbouring lanes' values
 // with DPP lane shifts; stencils along j keep a sliding window of rows in
 // registers.  Each PPM face value al and each cell's edge perturbations
 // (bl, br and the smoothness flag, or the monotone slope dm for hord 8) are
@@ -25,8 +25,6 @@ namespace fv3 {
 // last bit.  No LDS and no barriers: waves run independently.
 constexpr int MW = 64;        // lanes = strip columns
 constexpr int MTI = MW - 6;   // output interfaces per strip in i
-constexpr int MTJ = 33;       // output rows per segment in j (default)
-constexpr int MTJ_TALL = 51;  // the taller segment of large batches of narrow tiles
 
 // Whole-wave shifts by one lane with DPP: wave_shr:1 (lane L reads lane
 // L - 1) and wave_shl:1 (lane L reads lane L + 1); the lane without a source
@@ -65,25 +63,28 @@ __device__ __forceinline__ T lane_up(T v, int d) {  // value of lane - d
 
 
 // Face value al at face f (hord < 8, compute_al, xppm.py:147-181) from the
-// cells f-2, f-1, f, f+1 (qa..qd) and their widths (da..dd, read only at the
-// tile-edge faces).  With EDGES every candidate is evaluated and the match is
-// selected without branches (the reference's regions are applied in its
-// order, so the last selection below is its first test); lanes or steps that
-// need none of them keep the interior value.
+// cells f-2, f-1, f, f+1 (qa..qd).  With EDGES every candidate is evaluated
+// and the match is selected without branches (the reference's regions are
+// applied in its order, so the last selection below is its first test); ediv
+// is the value of the faces on the tile edge.
 template <typename T, bool EDGES>
-__device__ __forceinline__ T al_face(T qa, T qb, T qc, T qd, int f, int is, int ie, T da, T db,
-                                     T dc, T dd) {
+__device__ __forceinline__ T al_face(T qa, T qb, T qc, T qd, int f, int is, int ie, T ediv) {
   T al = T(FV3_PPM_P1) * (qb + qc) + T(FV3_PPM_P2) * (qa + qd);
   if constexpr (EDGES) {
     const T c123 = T(FV3_PPM_C1) * qa + T(FV3_PPM_C2) * qb + T(FV3_PPM_C3) * qc;
-    const T ediv = T(0.5) * (((T(2) * db + da) * qb - db * qa) / (da + db) +
-                             ((T(2) * dc + dd) * qc - dc * qd) / (dc + dd));
     const T c321 = T(FV3_PPM_C3) * qb + T(FV3_PPM_C2) * qc + T(FV3_PPM_C1) * qd;
     al = (f == is - 1 || f == ie) ? c123 : al;
     al = (f == is || f == ie + 1) ? ediv : al;
     al = (f == is + 1 || f == ie + 2) ? c321 : al;
   }
   return al;
+}
+
+// One side's term of the edge face value: the cell next to the face (q, width
+// d) extrapolated with the one beyond it (qn, dn).
+template <typename T>
+__device__ __forceinline__ T edge_term(T q, T d, T qn, T dn) {
+  return ((T(2) * d + dn) * q - d * qn) / (dn + d);
 }
 
 // Edge perturbations of a cell from its two face values (hord < 8) and the
@@ -135,21 +136,34 @@ __device__ __forceinline__ T face8(T c, T qm, T blm, T brm, T q0, T bl0, T br0) 
   return qu + (pos ? fpos : fneg);
 }
 
+// The value of every face from the two cells beside it by the edge formula
+// (used on the tile-edge faces), cell i with q, width d and neighbours qm, qp
+// in lane i.  The two terms of an edge face are formed by the two cells: with
+// one division a lane (the cell left of a face with its left neighbour, every
+// other lane with its right one), or with two where the tile is one cell wide
+// and that cell serves both edges (EX = 2).
+template <typename T, int EX>
+__device__ __forceinline__ T edge_face(T q, T qm, T qp, T d, int i, int is, int ie) {
+  const T dm = lane_up(d, 1), dp = lane_dn(d, 1);
+  if constexpr (EX == 2) {
+    return T(0.5) * (lane_up(edge_term(q, d, qm, dm), 1) + edge_term(q, d, qp, dp));
+  } else {
+    const bool left = i == is - 1 || i == ie;
+    const T term = edge_term(q, d, left ? qm : qp, left ? dm : dp);
+    return T(0.5) * (lane_up(term, 1) + term);
+  }
+}
+
 // PPM along i on one row held across the wave: lane L has cell i (= face i
-// on its left) with q, the Courant number c of face i and (tile-edge waves)
-// the width dxv of cell i; dxrow points at dx of column 0 of the row.
-template <typename T, int ORD, bool EDGES, typename S>
-__device__ __forceinline__ T ppm_row(T q, T c, int i, int is, int ie, T dxv,
-                                     const S* __restrict__ dxrow) {
+// on its left) with q, the Courant number c of face i and (EX != 0, strips
+// that meet a tile edge) the width dxv of cell i.
+template <typename T, int ORD, int EX>
+__device__ __forceinline__ T ppm_row(T q, T c, int i, int is, int ie, T dxv) {
   const T qm1 = lane_up(q, 1), qm2 = lane_up(q, 2), qp1 = lane_dn(q, 1);
   if constexpr (ORD < 8) {
-    T dm2 = T(0), dm1 = T(0), dp1 = T(0);
-    if constexpr (EDGES) {
-      dm2 = lane_up(dxv, 2);
-      dm1 = lane_up(dxv, 1);
-      dp1 = lane_dn(dxv, 1);
-    }
-    const T al = al_face<T, EDGES>(qm2, qm1, q, qp1, i, is, ie, dm2, dm1, dxv, dp1);
+    T ediv = T(0);
+    if constexpr (EX != 0) ediv = edge_face<T, EX>(q, qm1, qp1, dxv, i, is, ie);
+    const T al = al_face<T, EX != 0>(qm2, qm1, q, qp1, i, is, ie, ediv);
     const T alp = lane_dn(al, 1);
     T bl, br;
     bool sm;
@@ -158,15 +172,41 @@ __device__ __forceinline__ T ppm_row(T q, T c, int i, int is, int ie, T dxv,
     const bool smm = lane_up((int)sm, 1) != 0;
     return face_lo(c, qm1, blm, brm, smm, q, bl, br, sm);
   } else {
-    const T qp2 = lane_dn(q, 2);
+    const T dm = ppm_dm(qm1, q, qp1);
+    const T dmm = lane_up(dm, 1), dmp = lane_dn(dm, 1);
     T bl, br;
-    if constexpr (EDGES) {
-      const T w[5] = {qm2, qm1, q, qp1, qp2};
-      DxRow<T, S> dw{dxrow + (i - 2), 1, 5};
-      ppm_blbr8_w(w, i, is, ie, dw, bl, br);
-    } else {
-      const T dm = ppm_dm(qm1, q, qp1);
-      cell8(qm1, q, qp1, lane_up(dm, 1), dm, lane_dn(dm, 1), bl, br);
+    cell8(qm1, q, qp1, dmm, dm, dmp, bl, br);
+    if constexpr (EX != 0) {
+      // compute_blbr_ord8plus's edge cells (xppm.py:92-144, 184-266).  The
+      // lanes of a wave hold the cells of both edges, so every form is
+      // evaluated and selected (in the reference's order of precedence, last
+      // match wins), with the clamped value of the edge face.
+      T fv = edge_face<T, EX>(q, qm1, qp1, dxv, i, is, ie);
+      const T minq = fmin(fmin(fmin(qm2, qm1), q), qp1);
+      const T maxq = fmax(fmax(fmax(qm2, qm1), q), qp1);
+      fv = fmin(fmax(fv, minq), maxq);
+      const T fvr = lane_dn(fv, 1);
+      const T s11 = T(FV3_PPM_S11), s14 = T(FV3_PPM_S14), s15 = T(FV3_PPM_S15);
+      const T third = T(1.0 / 3.0);
+      T xl = s14 * dmm + s11 * (qm1 - q) + q, xr = fvr;  // is - 1
+      xr = i == is ? s15 * q + s11 * qp1 - s14 * dmp : xr;
+      xl = i == is + 1 ? s15 * qm1 + s11 * q - s14 * dm : xl;
+      xr = i == is + 1 ? T(0.5) * (q + qp1) + third * (dm - dmp) : xr;
+      xl = i == ie - 1 ? T(0.5) * (qm1 + q) + third * (dmm - dm) : xl;
+      xr = i == ie - 1 ? s15 * qp1 + s11 * q + s14 * dm : xr;
+      xl = i == ie ? s15 * q + s11 * qm1 + s14 * dmm : xl;
+      xr = i == ie ? fvr : xr;
+      xl = (i == is && i != ie - 1 && i != ie) || i == ie + 1 ? fv : xl;
+      xr = i == ie + 1 ? s11 * (qp1 - q) - s14 * dmp + q : xr;
+      T el = xl - q, er = xr - q;
+      // pert_ppm_standard_constraint_fcn (ppm.py:21-34)
+      const T da1 = el - er, da2 = da1 * da1, a6da = T(3) * (el + er) * da1;
+      const bool inside = el * er < T(0);
+      const T cr = a6da < -da2 ? T(-2) * el : er;
+      const T cl = !(a6da < -da2) && a6da > da2 ? T(-2) * er : el;
+      const bool edge = (i >= is - 1 && i <= is + 1) || (i >= ie - 1 && i <= ie + 1);
+      bl = edge ? (inside ? cl : T(0)) : bl;
+      br = edge ? (inside ? cr : T(0)) : br;
     }
     return face8(c, qm1, lane_up(bl, 1), lane_up(br, 1), q, bl, br);
   }
@@ -174,17 +214,18 @@ __device__ __forceinline__ T ppm_row(T q, T c, int i, int is, int ie, T dxv,
 
 // PPM along j in one column: cells are pushed bottom to top; after cell c is
 // pushed, face c - 2 (between cells c - 3 and c - 2) can be evaluated.
-template <typename T, int ORD, bool EDGES>
+// The tile-edge formulas read the widths where they need them (dycol points at
+// the column's width in row 0; rows are clamped into the storage of nj rows).
+template <typename T, int ORD>
 struct ColumnPPM {
   T q[5] = {};    // cells c-4 .. c
-  T dw[5] = {};   // their widths (tile-edge waves, hord < 8)
   T al1 = 0, al2 = 0;            // faces c-2, c-1 (hord < 8)
   T dm0 = 0, dm1 = 0, dm2 = 0;   // slopes of cells c-3, c-2, c-1 (hord 8)
   T bl0 = 0, br0 = 0, bl1 = 0, br1 = 0;  // cells c-3, c-2
   bool sm0 = false, sm1 = false;
 
-  template <typename S>
-  __device__ __forceinline__ void push(T qc, T dc, int c, int is, int ie,
+  template <bool EDGES, typename S>
+  __device__ __forceinline__ void push(T qc, int c, int is, int ie, int nj,
                                        const S* __restrict__ dycol, int64_t sj2) {
 #pragma unroll
     for (int n = 0; n < 4; ++n) q[n] = q[n + 1];
@@ -193,13 +234,14 @@ struct ColumnPPM {
     br0 = br1;
     sm0 = sm1;
     if constexpr (ORD < 8) {
+      T ediv = T(0);
       if constexpr (EDGES) {
-#pragma unroll
-        for (int n = 0; n < 4; ++n) dw[n] = dw[n + 1];
-        dw[4] = dc;
+        auto w = [&](int row) { return T(dycol[(int64_t)min(max(row, 0), nj - 1) * sj2]); };
+        ediv = T(0.5) * (edge_term(q[2], w(c - 2), q[1], w(c - 3)) +
+                         edge_term(q[3], w(c - 1), q[4], w(c)));
       }
       al1 = al2;
-      al2 = al_face<T, EDGES>(q[1], q[2], q[3], q[4], c - 1, is, ie, dw[1], dw[2], dw[3], dw[4]);
+      al2 = al_face<T, EDGES>(q[1], q[2], q[3], q[4], c - 1, is, ie, ediv);
       cell_lo<T, ORD>(al1, al2, q[2], bl1, br1, sm1);
     } else {
       dm0 = dm1;
@@ -267,9 +309,9 @@ __device__ __forceinline__ P pick_slot(const P (&a)[kMaxScalarBatch], int b) {
 
 // S is the storage type of every field, T the type the march computes in
 // (the same, or float for FP64 storage in the mixed-precision form).
-template <typename S, typename T, int ORD, bool EX, bool EY, int SEG>
+template <typename S, typename T, int ORD, int EX>
 __device__ __forceinline__ void fvtp2d_strip(
-    const Dom& d, const YFill& yf, int i0, int j0, const S* __restrict__ qx,
+    const Dom& d, const YFill& yf, int i0, int j0, int rows, const S* __restrict__ qx,
     const S* __restrict__ qy,
     const S* __restrict__ cx, const S* __restrict__ cy, const S* __restrict__ ax,
     const S* __restrict__ ay, const S* __restrict__ ux, const S* __restrict__ uy,
@@ -317,25 +359,23 @@ __device__ __forceinline__ void fvtp2d_strip(
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sv), rs, off, rowb, 0);
     }
   };
-  ColumnPPM<T, ORD, EY> yin, yout;
+  ColumnPPM<T, ORD> yin, yout;
   T sxm[4] = {};     // x-inner means of rows r-3 .. r at face i
   T sym_prev = T(0); // y-inner mean of face r-3
-  // tile-edge width rows are clamped into the storage the same way
-  auto jrow = [&](int j) { return (int64_t)min(max(j, 0), nj - 1) * sj2; };
   const S* dycol = dy + ic;
   // every value a march step uses is loaded by the step before it, so the
   // loads of one step are in flight while the previous step computes
   struct StepIn {
-    T qx, qy, cx, ax, ar, dx, dy;  // row r
+    T qx, qy, cx, ax, ar, dx;  // row r
     T cyf, ayf;                    // row f = r - 2
     T ag, cxg, dxg;                // row g = r - 3
     T uxg, uyf;                    // the mass fluxes at the outputs
   };
-  auto load_step = [&](int r, StepIn& v) {
+  auto load_step = [&](auto ey, int r, StepIn& v) {
     const int f = r - 2, g = r - 3;
     v.qx = ld(qx, r, sj);
     v.qy = ld(qy, r, sj);
-    if constexpr (EX && EY) {
+    if constexpr (EX != 0 && decltype(ey)::value) {
       // corner strips only: the y corner fill of q_y (the row test is
       // wave-uniform, the column test per lane)
       const bool south = r >= d.js - 3 && r < d.js, north = r > d.je && r <= d.je + 3;
@@ -356,30 +396,28 @@ __device__ __forceinline__ void fvtp2d_strip(
     v.cx = ld(cx, r, sj);
     v.ax = ld(ax, r, sj);
     v.ar = ld(ar, r, sj2);
-    v.dx = EX ? ld(dx, r, sj2) : T(0);
-    v.dy = EY ? ld(dy, r, sj2) : T(0);
+    v.dx = EX != 0 ? ld(dx, r, sj2) : T(0);
     v.cyf = ld(cy, f, sj);
     v.ayf = ld(ay, f, sj);
     v.ag = ld(ar, g, sj2);
     v.cxg = ld(cx, g, sj);
-    v.dxg = EX ? ld(dx, g, sj2) : T(0);
+    v.dxg = EX != 0 ? ld(dx, g, sj2) : T(0);
     v.uxg = ld(ux, g, sj);
     v.uyf = ld(uy, f, sj);
   };
   StepIn nx;
-  load_step(j0 - 3, nx);
+  load_step(std::true_type{}, j0 - 3, nx);
   T ay_g = T(0);  // ay of row g = r - 3 (row f of the previous step)
-#pragma unroll 3
-  for (int s = 0; s < SEG + 6; ++s) {
-    const int r = j0 - 3 + s;
+  auto step = [&](auto ey, int r) {
+    constexpr bool EY = decltype(ey)::value;
     const StepIn cu = nx;
-    load_step(r + 1, nx);
+    load_step(ey, r + 1, nx);
     const int f = r - 2, g = r - 3;
-    const bool wfx = out_lane && g >= j0 && g < j0 + SEG && i <= d.iec + 1 && g <= d.jec;
-    const bool wfy = out_lane && f >= j0 && f < j0 + SEG && i <= d.iec && f <= d.jec + 1;
+    const bool wfx = out_lane && g >= j0 && g < j0 + rows && i <= d.iec + 1 && g <= d.jec;
+    const bool wfy = out_lane && f >= j0 && f < j0 + rows && i <= d.iec && f <= d.jec + 1;
     // x-inner PPM of q_x on row r (faces i), then q_j of row r
     // (fvtp2d.py:50-60)
-    const T xm = ppm_row<T, ORD, EX>(cu.qx, cu.cx, i, d.is, d.ie, cu.dx, dx + jrow(r));
+    const T xm = ppm_row<T, ORD, EX>(cu.qx, cu.cx, i, d.is, d.ie, cu.dx);
     const T sxr = xm;
     const T f1 = lane_dn(cu.ax, 1);
     const T fx1_0 = cu.ax * sxr;
@@ -389,7 +427,7 @@ __device__ __forceinline__ void fvtp2d_strip(
     for (int n = 0; n < 3; ++n) sxm[n] = sxm[n + 1];
     sxm[3] = sxr;
     // y-inner PPM of q_y: face f = r - 2
-    yin.push(cu.qy, cu.dy, r, d.js, d.je, dycol, sj2);
+    yin.template push<EY>(cu.qy, r, d.js, d.je, nj, dycol, sj2);
     const T symf = yin.face(cu.cyf);
     // q_i of row g = r - 3 (fvtp2d.py:33-47)
     const T qig = (yin.q[1] * cu.ag + ay_g * sym_prev - cu.ayf * symf) /
@@ -397,23 +435,39 @@ __device__ __forceinline__ void fvtp2d_strip(
     sym_prev = symf;
     ay_g = cu.ayf;
     // x-outer on q_i of row g: q_x_flux (fvtp2d.py:63-92)
-    const T outx = ppm_row<T, ORD, EX>(qig, cu.cxg, i, d.is, d.ie, cu.dxg, dx + jrow(g));
+    const T outx = ppm_row<T, ORD, EX>(qig, cu.cxg, i, d.is, d.ie, cu.dxg);
     st(rfx, g, wfx, T(0.5) * (outx + sxm[0]) * cu.uxg);
     // y-outer PPM of q_j: face f, q_y_flux
-    yout.push(qjr, cu.dy, r, d.js, d.je, dycol, sj2);
+    yout.template push<EY>(qjr, r, d.js, d.je, nj, dycol, sj2);
     const T outy = yout.face(cu.cyf);
     st(rfy, f, wfy, T(0.5) * (outy + symf) * cu.uyf);
+  };
+  // Groups of three steps; only those whose rows meet a y edge take the edge
+  // formulas and the corner fill (a push of cell c forms face c - 1 and, for
+  // hord 8, cell c - 2; the fill is for the row loaded ahead, r + 1).
+  auto near = [](int r, int a) { return r + 3 >= a - 3 && r <= a + 3; };
+  const int rend = j0 + rows + 3;
+  int r = j0 - 3;
+  while (r < rend) {
+    for (; r < rend && (near(r, d.js) || near(r, d.je)); r += 3) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) step(std::true_type{}, r + m);
+    }
+    for (; r < rend && !(near(r, d.js) || near(r, d.je)); r += 3) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) step(std::false_type{}, r + m);
+    }
   }
 }
 
-template <typename S, typename T, int ORD, int SEG>
-__global__ void __launch_bounds__(MW)
+template <typename S, typename T, int ORD>
+__global__ void __launch_bounds__(MW) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 3 : 4)))
     fvtp2d_kernel(Dom d, ScalarBatch<S> sb, const S* __restrict__ crx,
                   const S* __restrict__ cry, const S* __restrict__ xfx,
                   const S* __restrict__ yfx, const S* __restrict__ xmf,
                   const S* __restrict__ ymf, const S* __restrict__ area,
                   const S* __restrict__ dxa, const S* __restrict__ dya, int nbi, int nbj,
-                  YFill yf) {
+                  int seg, YFill yf) {
   const int per_plane = nbi * nbj;
   const int total = per_plane * d.nk * d.ntiles * sb.n;
   const int lb = xcd_logical_block(blockIdx.x, total);
@@ -428,32 +482,60 @@ __global__ void __launch_bounds__(MW)
   S* __restrict__ fx = pick_slot(sb.fx, b);
   S* __restrict__ fy = pick_slot(sb.fy, b);
   const int i0 = d.isc + bi * MTI;
-  const int j0 = d.jsc + bj * SEG;
+  const int j0 = d.jsc + bj * seg;
+  const int rows = min(seg, d.jec + 2 - j0);
   const int64_t off3 = (int64_t)t * d.st + (int64_t)k * d.sk;
   const int64_t off2 = (int64_t)t * d.st2;
   const S* ux = (xmf ? xmf : xfx) + off3;
   const S* uy = (ymf ? ymf : yfx) + off3;
-  // the tile-edge formulas of a direction are needed when the strip's
-  // stencil reach (cells i0-4 .. i0+MTI+4, rows j0-4 .. j0+SEG+4) touches
-  // an edge region of that direction
+  // the x edge formulas are needed when the strip's stencil reach (cells
+  // i0-4 .. i0+MTI+4) touches an edge region
   auto near = [](int lo, int hi, int a) { return hi >= a - 2 && lo <= a + 3; };
   const bool ex = near(i0 - 4, i0 + MTI + 4, d.is) || near(i0 - 4, i0 + MTI + 4, d.ie);
-  const bool ey = near(j0 - 4, j0 + SEG + 4, d.js) || near(j0 - 4, j0 + SEG + 4, d.je);
-#define FV3_TP_STRIP(EX_, EY_)                                                                  \
-  fvtp2d_strip<S, T, ORD, EX_, EY_, SEG>(d, yf, i0, j0, q_x + off3, q_y + off3, crx + off3, \
-                                 cry + off3,                                                  \
-                                 xfx + off3, yfx + off3, ux, uy, area + off2, dxa + off2,     \
-                                 dya + off2, fx + off3, fy + off3)
-  if (ex && ey) {
-    FV3_TP_STRIP(true, true);
+#define FV3_TP_STRIP(EX_)                                                                        \
+  fvtp2d_strip<S, T, ORD, EX_>(d, yf, i0, j0, rows, q_x + off3, q_y + off3, crx + off3,      \
+                               cry + off3, xfx + off3, yfx + off3, ux, uy, area + off2,      \
+                               dxa + off2, dya + off2, fx + off3, fy + off3)
+  if (ex && d.is == d.ie) {
+    FV3_TP_STRIP(2);
   } else if (ex) {
-    FV3_TP_STRIP(true, false);
-  } else if (ey) {
-    FV3_TP_STRIP(false, true);
+    FV3_TP_STRIP(1);
   } else {
-    FV3_TP_STRIP(false, false);
+    FV3_TP_STRIP(0);
   }
 #undef FV3_TP_STRIP
+}
+
+// Output rows per segment of a launch of `planes` strips (strips along i x
+// levels x tiles x scalars) of nfj output rows.  A segment marches its rows
+// plus 6 halo rows in groups of three steps, so taller segments take fewer
+// steps per output row and shorter ones more waves.  Measured inside the
+// acoustic call (hord 6, cube tiles), a step takes 1.15 us plus 0.62 us per
+// wave on a SIMD while the waves' latencies overlap, and the SIMDs work off at
+// most a step in 0.97 us (FP32: 0.95, 0.3 and 0.59 us); a launch adds about
+// four steps.  The segment count with the least time by these figures is
+// taken.  Against the fixed 33 (for large batches 51) rows, with the edge
+// forms then in every step of a strip that met a y edge, per launch in the
+// acoustic call: six C12 tiles 60 -> 35 us, six C24 61 -> 38 us, six C48 84 ->
+// 49 us, six C96 127 -> 120 us (33 rows as before; 51 rows 135 us), six C128
+// 228 -> 201 us, 96 C48 tiles in FP32 304 -> 255 us; hord 8 alone on six C128
+// tiles 336 -> 235 us.
+static int segment_rows(int nfj, int64_t planes, bool fp32) {
+  const double lone = fp32 ? 0.95 : 1.15, per = fp32 ? 0.3 : 0.62, busy = fp32 ? 0.59 : 0.97;
+  int best = 0;
+  double least = 0.0;
+  for (int nb = 1; nb <= nfj; ++nb) {
+    const int seg = ((nfj + nb - 1) / nb + 2) / 3 * 3;  // seg + 6 halo rows fill whole groups
+    const double w = (double)planes * ((nfj + seg - 1) / seg) / kSimdsPerGpu;
+    const double step = lone + per * w > busy * w ? lone + per * w : busy * w;
+    const double t = step * (seg + 6 + 4);
+    if (best == 0 || t < least) {
+      best = seg;
+      least = t;
+    }
+    if (seg == 3) break;
+  }
+  return best;
 }
 
 // T: storage type; C: arithmetic type of the kernel.  sb: the scalars
@@ -482,21 +564,9 @@ static int fvtp2d_batch_launch(const fv3_domain* dom, int hord, const ScalarBatc
   Dom d = to_dom(dom);
   const int nfi = d.iec + 2 - d.isc, nfj = d.jec + 2 - d.jsc;
   const int nbi = (nfi + MTI - 1) / MTI;
-  // Segment height: each segment marches its rows plus 6 halo rows, so
-  // taller segments take fewer steps per output row, but fewer waves.  The
-  // taller segment is taken when it needs fewer march steps and the launch
-  // still has four waves per SIMD (large batches of narrow tiles, such as
-  // 192 C48 tiles); otherwise 33 rows (six C96 tiles: 97 rows in three
-  // segments, the fastest height of a sweep over 13-49 rows).
   const int64_t planes = (int64_t)nbi * d.nk * d.ntiles * sb.n;
-  int mtj = MTJ;
-  {
-    const int nb_s = (nfj + MTJ - 1) / MTJ, nb_t = (nfj + MTJ_TALL - 1) / MTJ_TALL;
-    if ((int64_t)nb_t * (MTJ_TALL + 6) < (int64_t)nb_s * (MTJ + 6) &&
-        planes * nb_t >= 4 * kSimdsPerGpu)
-      mtj = MTJ_TALL;
-  }
-  const int nbj = (nfj + mtj - 1) / mtj;
+  const int seg = segment_rows(nfj, planes, sizeof(C) == 4);
+  const int nbj = (nfj + seg - 1) / seg;
   const int64_t total = (int64_t)nbi * nbj * d.nk * d.ntiles * sb.n;
   FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);
   const int64_t launched = (total + kNumXcd - 1) / kNumXcd * kNumXcd;
@@ -514,31 +584,16 @@ static int fvtp2d_batch_launch(const fv3_domain* dom, int hord, const ScalarBatc
   TimedLaunch timed("fvtp2d_kernel", s,
                     nfld * sizeof(T) * (double)(d.iec - d.isc + 1) * (d.jec - d.jsc + 1) *
                         d.nk * d.ntiles);
-  auto go = [&](auto seg) {
-    constexpr int SEG = decltype(seg)::value;
-    switch (hord) {
-      case 5:
-        hipLaunchKernelGGL((fvtp2d_kernel<T, C, 5, SEG>), grid, block, 0, s, d, sb, crx, cry, xfx,
-                           yfx, xmf, ymf, area, dxa, dya, nbi, nbj, yf);
-        break;
-      case 6:
-        hipLaunchKernelGGL((fvtp2d_kernel<T, C, 6, SEG>), grid, block, 0, s, d, sb, crx, cry, xfx,
-                           yfx, xmf, ymf, area, dxa, dya, nbi, nbj, yf);
-        break;
-      case 7:
-        hipLaunchKernelGGL((fvtp2d_kernel<T, C, 7, SEG>), grid, block, 0, s, d, sb, crx, cry, xfx,
-                           yfx, xmf, ymf, area, dxa, dya, nbi, nbj, yf);
-        break;
-      default:
-        hipLaunchKernelGGL((fvtp2d_kernel<T, C, 8, SEG>), grid, block, 0, s, d, sb, crx, cry, xfx,
-                           yfx, xmf, ymf, area, dxa, dya, nbi, nbj, yf);
-        break;
-    }
+  auto go = [&](auto ord) {
+    hipLaunchKernelGGL((fvtp2d_kernel<T, C, decltype(ord)::value>), grid, block, 0, s, d, sb, crx,
+                       cry, xfx, yfx, xmf, ymf, area, dxa, dya, nbi, nbj, seg, yf);
   };
-  if (mtj == MTJ_TALL)
-    go(std::integral_constant<int, MTJ_TALL>{});
-  else
-    go(std::integral_constant<int, MTJ>{});
+  switch (hord) {
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    default: go(std::integral_constant<int, 8>{}); break;
+  }
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }
