@@ -42,7 +42,7 @@ REPO = HERE.parent
 # kernel -> (source, timing name, macro names, candidate (rows, waves) pairs)
 KERNELS: Dict[str, Tuple[str, str, Tuple[str, str], List[Tuple[int, int]]]] = {
     "delnflux": ("delnflux.hip", "delnflux_kernel", ("FV3_DN_TJ", "FV3_DN_NY"),
-                 [(4, 4), (8, 2), (8, 4), (8, 8), (12, 4), (16, 4), (16, 8), (24, 4)]),
+                 [(17, 4), (25, 4), (33, 1), (33, 2), (33, 4), (33, 8), (49, 4)]),
     "a2b": ("a2b.hip", "a2b_interp_kernel", ("FV3_AB_TJ", "FV3_AB_NY"),
             [(8, 4), (12, 4), (16, 4), (16, 8), (24, 8), (32, 8), (32, 16)]),
 }

@@ -3,10 +3,13 @@
 //
 // Reference: fv3core/stencils/fxadv.py:1-520, d_sw.py:1-1131, xtp_u.py,
 // ytp_v.py, divergence_damping.py:1-490.  fv3_d_sw runs the reference's
-// sequence from one host call; the transports reuse fv3_fvtp2d,
-// fv3_delnflux and fv3_copy_corners_xy of this library, the B-grid
-// interpolation launch_a2b_ord4.  Pointwise stencils that read only their
-// own point of the fields another stencil writes are fused into one pass.
+// sequence from one host call; the transports reuse fv3_fvtp2d and
+// fv3_copy_corners_xy of this library, the B-grid interpolation
+// launch_a2b_ord4.  Pointwise stencils that read only their own point of the
+// fields another stencil writes are fused into one pass, and those that read
+// the del-n fluxes of one cell are epilogues of the del-n march: the pair of
+// full-size flux arrays between them is gone.
+#include "delnflux.hpp"
 #include "kernels.hpp"
 #include "ppm.hpp"
 
@@ -219,40 +222,51 @@ __global__ void __launch_bounds__(64)
   for (int n = 0; n < nv; ++n) vcc[vo[n]] = vval[n];
 }
 
-// fxadv_fluxes_stencil (fxadv.py:386-421)
+// fxadv_fluxes_stencil (fxadv.py:386-421) and the Courant-number part of
+// flux_capacitor (d_sw.py:67-93), which adds crx and cry on the full domain
+// (where the fluxes leave them as they were, too).
 template <typename T>
 void launch_fxadv_fluxes(hipStream_t s, const Dom& d, const Met<T>& m, T dt, const T* ucc,
-                         const T* vcc, T* crx, T* cry, T* xfx, T* yfx) {
+                         const T* vcc, T* crx, T* cry, T* xfx, T* yfx, T* cx, T* cy) {
   const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
   launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
     const int64_t o = at3(d, i, j, k, t);
     const int64_t o2 = at2(d, i, j, t);
+    T cxv, cyv;
     if (i >= d.isc && i <= d.iec + 1) {
       const T prod = dt * ucc[o];
       if (prod > T(0)) {
-        crx[o] = prod * m.rdxa[o2 - 1];
+        cxv = prod * m.rdxa[o2 - 1];
         xfx[o] = m.dy[o2] * prod * m.sin_sg3[o2 - 1];
       } else {
-        crx[o] = prod * m.rdxa[o2];
+        cxv = prod * m.rdxa[o2];
         xfx[o] = m.dy[o2] * prod * m.sin_sg1[o2];
       }
+      crx[o] = cxv;
+    } else {
+      cxv = crx[o];
     }
     if (j >= d.jsc && j <= d.jec + 1) {
       const T prod = dt * vcc[o];
       if (prod > T(0)) {
-        cry[o] = prod * m.rdya[o2 - d.sj2];
+        cyv = prod * m.rdya[o2 - d.sj2];
         yfx[o] = m.dx[o2] * prod * m.sin_sg4[o2 - d.sj2];
       } else {
-        cry[o] = prod * m.rdya[o2];
+        cyv = prod * m.rdya[o2];
         yfx[o] = m.dx[o2] * prod * m.sin_sg2[o2];
       }
+      cry[o] = cyv;
+    } else {
+      cyv = cry[o];
     }
+    cx[o] = cx[o] + cxv;
+    cy[o] = cy[o] + cyv;
   });
 }
 
 template <typename T>
 int run_fxadv(hipStream_t s, const Dom& d, const Met<T>& m, T dt, const T* uc, const T* vc,
-              T* crx, T* cry, T* xfx, T* yfx, T* ucc, T* vcc, const char* who) {
+              T* crx, T* cry, T* xfx, T* yfx, T* cx, T* cy, T* ucc, T* vcc, const char* who) {
   launch_fxadv_main(s, d, m, uc, vc, ucc, vcc);
   FV3_HIP_CHECK_LAUNCH(who);
   launch_fxadv_vc_edges(s, d, m, vc, ucc, vcc);
@@ -264,7 +278,7 @@ int run_fxadv(hipStream_t s, const Dom& d, const Met<T>& m, T dt, const T* uc, c
     hipLaunchKernelGGL((fxadv_corner_kernel<T>), grid, dim3(64), 0, s, d, m, uc, vc, ucc, vcc);
     FV3_HIP_CHECK_LAUNCH(who);
   }
-  launch_fxadv_fluxes(s, d, m, dt, ucc, vcc, crx, cry, xfx, yfx);
+  launch_fxadv_fluxes(s, d, m, dt, ucc, vcc, crx, cry, xfx, yfx, cx, cy);
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }
@@ -435,73 +449,299 @@ void launch_ke(hipStream_t s, const Dom& d, const Met<T>& m, T dt, const T* uc, 
 }
 
 // ---------------------------------------------------------- pointwise d_sw
-// flux_capacitor (full domain; the mass-flux temporaries are zero outside
-// where the transport writes them) + heat_diss (compute domain).
+// The stencils that read a transport's or a field's del-n fluxes run as
+// epilogues of the pass that forms them (delnflux.hpp): f0, f1 are the del-n x
+// fluxes at i and i + 1, g0, g1 the y fluxes at j and j + 1.  Fields whose
+// neighbours other lanes still read go to scratch slabs.  Bytes per cell-level
+// against separate launches, in field passes: mass fluxes 7 instead of 12,
+// w 5 instead of 10, q_con 5 instead of 11, pt 8 instead of 14, vorticity 12
+// instead of 22.
+
+// delp: the transport's mass fluxes with their damping, and flux_capacitor's
+// sums of them (d_sw.py:67-93).
 template <typename T>
-void launch_capacitor_heat(hipStream_t s, const Dom& d, const Met<T>& m, T dt, int nonhydro,
-                           const DswCols<T>& cols, const DswState<T>& st, const T* fx,
-                           const T* fy, const T* fx2, const T* fy2, T* dw, T* heat_s) {
-  const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
-  T* cx = st.cx;
-  T* cy = st.cy;
-  T* mfx = st.mfx;
-  T* mfy = st.mfy;
-  const T* crx = st.crx;
-  const T* cry = st.cry;
-  const T* w = st.w;
-  T* diss = st.diss_est;
-  const T* damp_w = cols.damp_w;
-  const T* ke_bg = cols.ke_bg;
-  launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    cx[o] = cx[o] + crx[o];
-    cy[o] = cy[o] + cry[o];
-    if (i >= d.isc && i <= d.iec + 1 && j >= d.jsc && j <= d.jec) mfx[o] = mfx[o] + fx[o];
-    if (i >= d.isc && i <= d.iec && j >= d.jsc && j <= d.jec + 1) mfy[o] = mfy[o] + fy[o];
-    if (!nonhydro || i < d.isc || i > d.iec || j < d.jsc || j > d.jec) return;
-    if (damp_w[k] > T(1e-5)) {
-      const T dd8 = ke_bg[k] * fabs(dt);
-      const T dwv = (fx2[o] - fx2[o + 1] + fy2[o] - fy2[o + d.sj]) * m.rarea[at2(d, i, j, t)];
-      const T hs = dd8 - dwv * (w[o] + T(0.5) * dwv);
-      dw[o] = dwv;
-      heat_s[o] = hs;
-      diss[o] = diss[o] + hs;
+struct MassFluxEpilogue {
+  T *fx, *fy, *mfx, *mfy;
+  int64_t sj;
+
+  struct In {
+    T fx, fy, mx, my;
+  };
+  __device__ __forceinline__ void plane(const Dom& d, int, T, int64_t off3, int64_t) {
+    fx += off3;
+    fy += off3;
+    mfx += off3;
+    mfy += off3;
+    sj = d.sj;
+  }
+  template <typename C>
+  __device__ __forceinline__ In load(const C& c, int j) const {
+    return {c.f(fx, j), c.f(fy, j), c.f(mfx, j), c.f(mfy, j)};
+  }
+  __device__ __forceinline__ void apply(const In& n, int i, int j, T f0, T, T g0, T, bool fxo,
+                                        bool fyo, bool) const {
+    const int64_t row = (int64_t)j * sj;
+    if (fxo) {
+      const T v = n.fx + f0;
+      (fx + row)[i] = v;
+      (mfx + row)[i] = n.mx + v;
     }
-  });
-}
+    if (fyo) {
+      const T v = n.fy + g0;
+      (fy + row)[i] = v;
+      (mfy + row)[i] = n.my + v;
+    }
+  }
+};
 
-// flux_adjust (d_sw.py:50-64): q = q * delp + flux_increment(gx, gy) on the compute domain.
+// w: heat_diss (d_sw.py:96-109) from w's del-n fluxes.
 template <typename T>
-void launch_flux_adjust(hipStream_t s, const Dom& d, const Met<T>& m, T* q, const T* delp,
-                        const T* gx, const T* gy) {
-  const Box comp{d.isc, d.iec, d.jsc, d.jec};
-  launch_box(s, d, comp, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    q[o] = q[o] * delp[o] + (gx[o] - gx[o + 1] + gy[o] - gy[o + d.sj]) * m.rarea[at2(d, i, j, t)];
-  });
-}
+struct HeatDissEpilogue {
+  const T *w, *rarea, *damp_w, *ke_bg;
+  T *dw, *heat_s, *diss;
+  T adt, dd8;
+  bool on;
+  int64_t sj;
 
-// apply_pt_delp_fluxes (d_sw.py:149-180) on the compute domain.
-template <typename T>
-void launch_pt_delp(hipStream_t s, const Dom& d, const Met<T>& m, T* pt, T* delp, const T* gx,
-                    const T* gy, const T* fx, const T* fy) {
-  const Box comp{d.isc, d.iec, d.jsc, d.jec};
-  launch_box(s, d, comp, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const T ra = m.rarea[at2(d, i, j, t)];
-    const T dp = delp[o];
-    const T ptn = pt[o] * dp + (gx[o] - gx[o + 1] + gy[o] - gy[o + d.sj]) * ra;
-    const T dpn = dp + (fx[o] - fx[o + 1] + fy[o] - fy[o + d.sj]) * ra;
-    pt[o] = ptn / dpn;
-    delp[o] = dpn;
-  });
-}
+  struct In {
+    T w, diss, ra;
+  };
+  __device__ __forceinline__ void plane(const Dom& d, int k, T, int64_t off3, int64_t off2) {
+    on = damp_w[k] > T(1e-5);
+    dd8 = ke_bg[k] * adt;
+    w += off3;
+    dw += off3;
+    heat_s += off3;
+    diss += off3;
+    rarea += off2;
+    sj = d.sj;
+  }
+  template <typename C>
+  __device__ __forceinline__ In load(const C& c, int j) const {
+    return {c.f(w, j), c.f(diss, j), c.m(rarea, j)};
+  }
+  __device__ __forceinline__ void apply(const In& n, int i, int j, T f0, T f1, T g0, T g1, bool,
+                                        bool, bool cell) const {
+    if (!cell || !on) return;
+    const int64_t row = (int64_t)j * sj;
+    const T dwv = (f0 - f1 + g0 - g1) * n.ra;
+    const T hs = dd8 - dwv * (n.w + T(0.5) * dwv);
+    (dw + row)[i] = dwv;
+    (heat_s + row)[i] = hs;
+    (diss + row)[i] = n.diss + hs;
+  }
+};
 
-// compute_vorticity (full domain) + adjust_w_and_qcon (compute domain).
+// The transport's fluxes around a cell with the mass-weighted damping
+// (delnflux.py:903-905).
 template <typename T>
-void launch_vorticity_adjust(hipStream_t s, const Dom& d, const Met<T>& m, const T* u,
-                             const T* v, T* wk, T* w, const T* delp, const T* dw, T* q_con,
-                             const T* damp_w) {
+struct DampedFluxes {
+  T x0, x1, y0, y1, m, mw, me, ms, mn;
+  template <typename C>
+  __device__ __forceinline__ void load(const C& c, int j, const T* gx, const T* gy,
+                                       const T* mass) {
+    x0 = c.f(gx, j);
+    x1 = c.f(gx, j, 1);
+    y0 = c.f(gy, j);
+    y1 = c.f(gy, j + 1);
+    m = c.f(mass, j);
+    mw = c.f(mass, j, -1);
+    me = c.f(mass, j, 1);
+    ms = c.f(mass, j - 1);
+    mn = c.f(mass, j + 1);
+  }
+  // flux_increment (d_sw.py:43-47) of the damped fluxes
+  __device__ __forceinline__ T increment(T dk, T f0, T f1, T g0, T g1, T ra) const {
+    const T a0 = x0 + T(0.5) * dk * (mw + m) * f0, a1 = x1 + T(0.5) * dk * (m + me) * f1;
+    const T b0 = y0 + T(0.5) * dk * (ms + m) * g0, b1 = y1 + T(0.5) * dk * (m + mn) * g1;
+    return (a0 - a1 + b0 - b1) * ra;
+  }
+};
+
+// q_con: flux_adjust (d_sw.py:50-64) with the damped fluxes, into out.
+template <typename T>
+struct FluxAdjustEpilogue {
+  const T *q, *delp, *gx, *gy, *rarea;
+  T* out;
+  T dk;
+  int64_t sj;
+
+  struct In {
+    DampedFluxes<T> g;
+    T q, ra;
+  };
+  __device__ __forceinline__ void plane(const Dom& d, int, T dk_, int64_t off3, int64_t off2) {
+    dk = dk_;
+    q += off3;
+    delp += off3;
+    gx += off3;
+    gy += off3;
+    out += off3;
+    rarea += off2;
+    sj = d.sj;
+  }
+  template <typename C>
+  __device__ __forceinline__ In load(const C& c, int j) const {
+    In n;
+    n.g.load(c, j, gx, gy, delp);
+    n.q = c.f(q, j);
+    n.ra = c.m(rarea, j);
+    return n;
+  }
+  __device__ __forceinline__ void apply(const In& n, int i, int j, T f0, T f1, T g0, T g1, bool,
+                                        bool, bool cell) const {
+    if (cell)
+      (out + (int64_t)j * sj)[i] = n.q * n.g.m + n.g.increment(dk, f0, f1, g0, g1, n.ra);
+  }
+};
+
+// pt and delp: apply_pt_delp_fluxes (d_sw.py:149-180) with the damped fluxes
+// of pt and the mass fluxes, into pt_out and delp_out.
+template <typename T>
+struct PtDelpEpilogue {
+  const T *pt, *delp, *gx, *gy, *fx, *fy, *rarea;
+  T *pt_out, *delp_out;
+  T dk;
+  int64_t sj;
+
+  struct In {
+    DampedFluxes<T> g;
+    T pt, ra, fx0, fx1, fy0, fy1;
+  };
+  __device__ __forceinline__ void plane(const Dom& d, int, T dk_, int64_t off3, int64_t off2) {
+    dk = dk_;
+    pt += off3;
+    delp += off3;
+    gx += off3;
+    gy += off3;
+    fx += off3;
+    fy += off3;
+    pt_out += off3;
+    delp_out += off3;
+    rarea += off2;
+    sj = d.sj;
+  }
+  template <typename C>
+  __device__ __forceinline__ In load(const C& c, int j) const {
+    In n;
+    n.g.load(c, j, gx, gy, delp);
+    n.pt = c.f(pt, j);
+    n.ra = c.m(rarea, j);
+    n.fx0 = c.f(fx, j);
+    n.fx1 = c.f(fx, j, 1);
+    n.fy0 = c.f(fy, j);
+    n.fy1 = c.f(fy, j + 1);
+    return n;
+  }
+  __device__ __forceinline__ void apply(const In& n, int i, int j, T f0, T f1, T g0, T g1, bool,
+                                        bool, bool cell) const {
+    if (!cell) return;
+    const int64_t row = (int64_t)j * sj;
+    const T dp = n.g.m;
+    const T ptn = n.pt * dp + n.g.increment(dk, f0, f1, g0, g1, n.ra);
+    const T dpn = dp + (n.fx0 - n.fx1 + n.fy0 - n.fy1) * n.ra;
+    (pt_out + row)[i] = ptn / dpn;
+    (delp_out + row)[i] = dpn;
+  }
+};
+
+// Vorticity: vort_differencing (d_sw.py:183-193), heat_source_from_vorticity_
+// damping on the compute domain (the part of it that reaches the output;
+// d_sw.py:353-434) and update_u_and_v (437-460) from the winds in us, vs.
+template <typename T>
+struct VortDampEpilogue {
+  const T *us, *vs, *vort, *delp, *heat_s;
+  const T *rdx, *rdy, *rsin2, *cosa_s;
+  const T *kef, *damp_vt;
+  T *u, *v, *heat_total;
+  int d_con_on;
+  T kefk;
+  bool heat, damp;
+  int64_t sj;
+
+  struct In {
+    T u0, u1, v0, v1, w00, w10, w01, w11, dp, hs, ht, rdx0, rdx1, rdy0, rdy1, rs, cs;
+  };
+  __device__ __forceinline__ void plane(const Dom& d, int k, T, int64_t off3, int64_t off2) {
+    kefk = kef[k];
+    heat = kefk > T(kDconThreshold);
+    damp = damp_vt[k] > T(1e-5);
+    us += off3;
+    vs += off3;
+    vort += off3;
+    delp += off3;
+    heat_s += off3;
+    u += off3;
+    v += off3;
+    heat_total += off3;
+    rdx += off2;
+    rdy += off2;
+    rsin2 += off2;
+    cosa_s += off2;
+    sj = d.sj;
+  }
+  template <typename C>
+  __device__ __forceinline__ In load(const C& c, int j) const {
+    In n{};
+    n.u0 = c.f(us, j);
+    n.v0 = c.f(vs, j);
+    if (d_con_on) {
+      n.hs = c.f(heat_s, j);
+      n.ht = c.f(heat_total, j);
+      if (heat) {
+        n.u1 = c.f(us, j + 1);
+        n.v1 = c.f(vs, j, 1);
+        n.w00 = c.f(vort, j);
+        n.w10 = c.f(vort, j, 1);
+        n.w01 = c.f(vort, j + 1);
+        n.w11 = c.f(vort, j + 1, 1);
+        n.dp = c.f(delp, j);
+        n.rdx0 = c.m(rdx, j);
+        n.rdx1 = c.m(rdx, j + 1);
+        n.rdy0 = c.m(rdy, j);
+        n.rdy1 = c.m(rdy, j, 1);
+        n.rs = c.m(rsin2, j);
+        n.cs = c.m(cosa_s, j);
+      }
+    }
+    return n;
+  }
+  __device__ __forceinline__ void apply(const In& n, int i, int j, T ut0, T ut1, T vt0, T vt1,
+                                        bool fxo, bool fyo, bool cell) const {
+    const int64_t row = (int64_t)j * sj;
+    if (cell && d_con_on) {
+      T hs = n.hs;
+      if (heat) {
+        // ubt, gy at j and j+1; vbt, gx at i and i+1
+        const T ubt0 = ((n.w00 - n.w10) + vt0) * n.rdx0, ubt1 = ((n.w01 - n.w11) + vt1) * n.rdx1;
+        const T fy0 = n.u0 * n.rdx0, fy1 = n.u1 * n.rdx1;
+        const T gy0 = fy0 * ubt0, gy1 = fy1 * ubt1;
+        const T vbt0 = ((n.w00 - n.w01) - ut0) * n.rdy0, vbt1 = ((n.w10 - n.w11) - ut1) * n.rdy1;
+        const T fx0 = n.v0 * n.rdy0, fx1 = n.v1 * n.rdy1;
+        const T gx0 = fx0 * vbt0, gx1 = fx1 * vbt1;
+        const T u2 = fy0 + fy1, du2 = ubt0 + ubt1;
+        const T v2 = fx0 + fx1, dv2 = vbt0 + vbt1;
+        const T dampterm = n.rs * ((ubt0 * ubt0 + ubt1 * ubt1 + vbt0 * vbt0 + vbt1 * vbt1) +
+                                   T(2) * (gy0 + gy1 + gx0 + gx1) -
+                                   n.cs * (u2 * dv2 + v2 * du2 + du2 * dv2));
+        hs = n.dp * (hs - T(0.25) * kefk * dampterm);
+      }
+      (heat_total + row)[i] = n.ht + hs;
+    }
+    if (fyo) (u + row)[i] = damp ? n.u0 + vt0 : n.u0;
+    if (fxo) (v + row)[i] = damp ? n.v0 - ut0 : n.v0;
+  }
+};
+
+// compute_vorticity (full domain); on the compute domain flux_adjust of w from
+// its transport fluxes wgx, wgy (nonhydrostatic), adjust_w_and_qcon
+// (d_sw.py:463-481), and the write-back of delp, pt from their scratch slabs
+// (delpn, ptn, and q_con's in qcn, mass-weighted).
+template <typename T>
+void launch_vorticity_adjust(hipStream_t s, const Dom& d, const Met<T>& m, int nonhydro,
+                             const T* u, const T* v, T* wk, T* w, const T* wgx, const T* wgy,
+                             T* delp, const T* delpn, T* pt, const T* ptn, const T* dw, T* q_con,
+                             const T* qcn, const T* damp_w) {
   const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
   launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
     const int64_t o = at3(d, i, j, k, t);
@@ -510,87 +750,38 @@ void launch_vorticity_adjust(hipStream_t s, const Dom& d, const Met<T>& m, const
     wk[o] = (u[o] - u[o + d.sj] * m.dx[o2 + d.sj2] / dx) * (ra * dx) +
             (v[o + 1] * m.dy[o2 + 1] / dy - v[o]) * (ra * dy);
     if (i < d.isc || i > d.iec || j < d.jsc || j > d.jec) return;
-    T wn = w[o] / delp[o];
+    const T dpn = delpn[o];
+    T wn = w[o];
+    if (nonhydro) wn = wn * delp[o] + (wgx[o] - wgx[o + 1] + wgy[o] - wgy[o + d.sj]) * ra;
+    wn = wn / dpn;
     if (damp_w[k] > T(1e-5)) wn = wn + dw[o];
     w[o] = wn;
-    q_con[o] = q_con[o] / delp[o];
+    q_con[o] = qcn[o] / dpn;
+    delp[o] = dpn;
+    pt[o] = ptn[o];
   });
 }
 
-// vort_differencing (corners; levels with d_con > threshold) + compute_vort
-// into a separate slab (full domain), so both read the old vorticity.
+// compute_vort (d_sw.py:240-241): the absolute vorticity the transport moves.
 template <typename T>
-void launch_vort_diff(hipStream_t s, const Dom& d, const Met<T>& m, const T* vort, const T* wk,
-                      T* vxd, T* vyd, T* vort2, const T* dcon) {
+void launch_absolute_vort(hipStream_t s, const Dom& d, const Met<T>& m, const T* wk, T* vort2) {
   const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
   launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
     const int64_t o = at3(d, i, j, k, t);
-    if (dcon[k] > T(kDconThreshold)) {
-      if (i >= d.isc && i <= d.iec && j >= d.jsc && j <= d.jec + 1) vxd[o] = vort[o] - vort[o + 1];
-      if (i >= d.isc && i <= d.iec + 1 && j >= d.jsc && j <= d.jec) vyd[o] = vort[o] - vort[o + d.sj];
-    }
     vort2[o] = wk[o] + m.f0[at2(d, i, j, t)];
   });
 }
 
-// u_and_v_from_ke (d_sw.py:244-266)
+// u_and_v_from_ke (d_sw.py:244-266), into us and vs
 template <typename T>
 void launch_uv_from_ke(hipStream_t s, const Dom& d, const Met<T>& m, const T* ke, const T* fx,
-                       const T* fy, T* u, T* v) {
+                       const T* fy, const T* u, const T* v, T* us, T* vs) {
   const Box bx{d.isc, d.iec + 1, d.jsc, d.jec + 1};
   launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
     const int64_t o = at3(d, i, j, k, t);
     const int64_t o2 = at2(d, i, j, t);
-    if (i <= d.iec) u[o] = u[o] * m.dx[o2] + ke[o] - ke[o + 1] + fy[o];
-    if (j <= d.jec) v[o] = v[o] * m.dy[o2] + ke[o] - ke[o + d.sj] - fx[o];
-  });
-}
-
-// heat_source_from_vorticity_damping on the compute domain (the only part
-// of the heat source that reaches the output; d_sw.py:353-434).
-template <typename T>
-void launch_heat_source(hipStream_t s, const Dom& d, const Met<T>& m, const T* vxd, const T* vyd,
-                        const T* ut, const T* vt, const T* u, const T* v, const T* delp,
-                        const T* heat_s, T* heat_total, const T* kef, int d_con_on) {
-  if (!d_con_on) return;
-  const Box comp{d.isc, d.iec, d.jsc, d.jec};
-  launch_box(s, d, comp, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const int64_t o2 = at2(d, i, j, t);
-    const int64_t sj = d.sj, sj2 = d.sj2;
-    T hs = heat_s[o];
-    if (kef[k] > T(kDconThreshold)) {
-      // ubt, gy at j and j+1; vbt, gx at i and i+1
-      const T rdx0 = m.rdx[o2], rdx1 = m.rdx[o2 + sj2];
-      const T rdy0 = m.rdy[o2], rdy1 = m.rdy[o2 + 1];
-      const T ubt0 = (vxd[o] + vt[o]) * rdx0, ubt1 = (vxd[o + sj] + vt[o + sj]) * rdx1;
-      const T fy0 = u[o] * rdx0, fy1 = u[o + sj] * rdx1;
-      const T gy0 = fy0 * ubt0, gy1 = fy1 * ubt1;
-      const T vbt0 = (vyd[o] - ut[o]) * rdy0, vbt1 = (vyd[o + 1] - ut[o + 1]) * rdy1;
-      const T fx0 = v[o] * rdy0, fx1 = v[o + 1] * rdy1;
-      const T gx0 = fx0 * vbt0, gx1 = fx1 * vbt1;
-      const T u2 = fy0 + fy1, du2 = ubt0 + ubt1;
-      const T v2 = fx0 + fx1, dv2 = vbt0 + vbt1;
-      const T dampterm =
-          m.rsin2[o2] * ((ubt0 * ubt0 + ubt1 * ubt1 + vbt0 * vbt0 + vbt1 * vbt1) +
-                         T(2) * (gy0 + gy1 + gx0 + gx1) -
-                         m.cosa_s[o2] * (u2 * dv2 + v2 * du2 + du2 * dv2));
-      hs = delp[o] * (hs - T(0.25) * kef[k] * dampterm);
-    }
-    heat_total[o] = heat_total[o] + hs;
-  });
-}
-
-// update_u_and_v (d_sw.py:437-460)
-template <typename T>
-void launch_update_uv(hipStream_t s, const Dom& d, const T* ut, const T* vt, T* u, T* v,
-                      const T* damp_vt) {
-  const Box bx{d.isc, d.iec + 1, d.jsc, d.jec + 1};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    if (!(damp_vt[k] > T(1e-5))) return;
-    const int64_t o = at3(d, i, j, k, t);
-    if (i <= d.iec) u[o] = u[o] + vt[o];
-    if (j <= d.jec) v[o] = v[o] - ut[o];
+    if (i <= d.iec) us[o] = u[o] * m.dx[o2] + ke[o] - ke[o + 1] + fy[o];
+    if (j <= d.jec) vs[o] = v[o] * m.dy[o2] + ke[o] - ke[o + d.sj] - fx[o];
   });
 }
 
@@ -893,7 +1084,7 @@ void launch_ke_ord(hipStream_t s, const Dom& d, const Met<T>& m, T dt, const T* 
 }
 
 // The transports of d_sw for each storage type: fv_tp_2d with its corner
-// fills, and the del-n damping of the fluxes.
+// fills.
 inline int dsw_transport(const fv3_domain* d, int hord, double* q, double* qy, const double* crx,
                          const double* cry, const double* xfx, const double* yfx,
                          const double* xmf, const double* ymf, const double* area,
@@ -909,20 +1100,6 @@ inline int dsw_transport(const fv3_domain* d, int hord, float* q, float* qy, con
                          float* fx, float* fy, bool, void* stream) {
   return fvtp2d_corner_fill_f32(d, hord, q, qy, crx, cry, xfx, yfx, xmf, ymf, area, dxa, dya, fx,
                                 fy, stream);
-}
-
-inline int dsw_delnflux(const fv3_domain* d, int mode, const int* nord4, const double* q,
-                        const double* mass, const double* damp, const double* del6_u,
-                        const double* del6_v, const double* rarea, double* fx, double* fy,
-                        void* stream) {
-  return fv3_delnflux_f64(d, mode, nord4, q, mass, damp, del6_u, del6_v, rarea, fx, fy, stream);
-}
-
-inline int dsw_delnflux(const fv3_domain* d, int mode, const int* nord4, const float* q,
-                        const float* mass, const float* damp, const float* del6_u,
-                        const float* del6_v, const float* rarea, float* fx, float* fy,
-                        void* stream) {
-  return fv3_delnflux_f32(d, mode, nord4, q, mass, damp, del6_u, del6_v, rarea, fx, fy, stream);
 }
 
 int check_dsw_metrics(const fv3_metrics* g, const char* who) {
@@ -974,58 +1151,69 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
   T* W[22];
   for (int n = 0; n < 22; ++n) W[n] = work + (int64_t)n * work_slab;
   T *ucc = W[0], *vcc = W[1], *fx = W[2], *fy = W[3], *gx = W[4], *gy = W[5];
-  T *fx2 = W[6], *fy2 = W[7], *dw = W[8], *heat_s = W[9], *wk = W[10], *vort = W[11];
-  T *ke = W[12], *vxd = W[13], *vyd = W[14], *ut = W[15], *vt = W[16], *qy = W[17];
+  T *wgx = W[6], *wgy = W[7], *dw = W[8], *heat_s = W[9], *wk = W[10], *vort = W[11];
+  T *ke = W[12], *delpn = W[13], *ptn = W[14], *qcn = W[15], *qy = W[17];
+  T *us = W[4], *vs = W[5];  // the winds before their damping (gx, gy are free by then)
   T *a2x = W[18], *a2e = W[20], *vort2 = W[21];  // W[19]: the last divergence pass
   const T* area = m.area;
   const T* dxa = m.dxa;
   const T* dya = m.dya;
-  const T* del6_u = m.del6_u;
-  const T* del6_v = m.del6_v;
   const T* rarea = m.rarea;
 
-  // transport of q: corner copies (x in place, y applied as the transport
-  // reads q), fv_tp_2d on nk + 1 levels, then del-n damping of the fluxes on
-  // nk levels
-  auto transport = [&](T* q, int hord, const T* mfx_, const T* mfy_, const int* nord4,
-                       const T* damp, const T* mass, T* ox, T* oy) -> int {
-    int r = dsw_transport(&d1, hord, q, qy, st.crx, st.cry, st.xfx, st.yfx, mfx_, mfy_, area, dxa,
-                          dya, ox, oy, p->transport_fp32 != 0, stream);
-    if (r) return r;
-    if (nord4) {
-      r = dsw_delnflux(dom, mass ? FV3_DELN_MASS : FV3_DELN_ADD, nord4, q, mass, damp, del6_u,
-                       del6_v, rarea, ox, oy, stream);
-    }
-    return r;
+  // transport of q on nk + 1 levels: corner copies (x in place, y applied as
+  // the transport reads q), then fv_tp_2d
+  auto transport = [&](T* q, int hord, const T* mfx_, const T* mfy_, T* ox, T* oy) -> int {
+    return dsw_transport(&d1, hord, q, qy, st.crx, st.cry, st.xfx, st.yfx, mfx_, mfy_, area, dxa,
+                         dya, ox, oy, p->transport_fp32 != 0, stream);
+  };
+  const double cells = (double)(d.iec - d.isc + 1) * (d.jec - d.jsc + 1) * d.nk * d.ntiles;
+  // the del-n pass of q on nk levels with its epilogue (`fields` read or written)
+  auto deln = [&](const int* nord4, bool use_damp, const T* q, const T* damp, const auto& epi,
+                  double fields) -> int {
+    return deln_launch<T>(dom, nord4, use_damp ? 1 : 0, q, damp, m.del6_u, m.del6_v, rarea, epi,
+                          fields * sizeof(T) * cells, stream, who);
   };
 
-  rc = run_fxadv<T>(s, d, m, dt, st.uc, st.vc, st.crx, st.cry, st.xfx, st.yfx, ucc, vcc, who);
+  rc = run_fxadv<T>(s, d, m, dt, st.uc, st.vc, st.crx, st.cry, st.xfx, st.yfx, st.cx, st.cy, ucc,
+                    vcc, who);
   if (rc) return rc;
-  rc = transport(st.delp, p->hord_dp, nullptr, nullptr, p->nord_v4, cols.damp_vt_deln, nullptr,
-                 fx, fy);
+  rc = transport(st.delp, p->hord_dp, nullptr, nullptr, fx, fy);
   if (rc) return rc;
+  {
+    const MassFluxEpilogue<T> epi{fx, fy, st.mfx, st.mfy, 0};
+    rc = deln(p->nord_v4, true, st.delp, cols.damp_vt_deln, epi, 9.0);
+    if (rc) return rc;
+  }
   const int nonhydro = !p->hydrostatic;
   if (nonhydro) {
-    rc = dsw_delnflux(dom, FV3_DELN_STORE, p->nord_w4, st.w, nullptr, cols.damp_w_nosg, del6_u,
-                      del6_v, rarea, fx2, fy2, stream);
+    HeatDissEpilogue<T> epi{};
+    epi.w = st.w;
+    epi.rarea = rarea;
+    epi.damp_w = cols.damp_w;
+    epi.ke_bg = cols.ke_bg;
+    epi.dw = dw;
+    epi.heat_s = heat_s;
+    epi.diss = st.diss_est;
+    epi.adt = fabs(dt);
+    rc = deln(p->nord_w4, true, st.w, cols.damp_w_nosg, epi, 5.0);
+    if (rc) return rc;
+    rc = transport(st.w, p->hord_vt, fx, fy, wgx, wgy);
     if (rc) return rc;
   }
-  launch_capacitor_heat<T>(s, d, m, dt, nonhydro, cols, st, fx, fy, fx2, fy2, dw, heat_s);
-  FV3_HIP_CHECK_LAUNCH(who);
-  if (nonhydro) {
-    rc = transport(st.w, p->hord_vt, fx, fy, nullptr, nullptr, nullptr, gx, gy);
+  rc = transport(st.q_con, p->hord_dp, fx, fy, gx, gy);
+  if (rc) return rc;
+  {
+    const FluxAdjustEpilogue<T> epi{st.q_con, st.delp, gx, gy, rarea, qcn, T(0), 0};
+    rc = deln(p->nord_t4, false, st.q_con, cols.damp_t_deln, epi, 5.0);
     if (rc) return rc;
-    launch_flux_adjust<T>(s, d, m, st.w, st.delp, gx, gy);
-    FV3_HIP_CHECK_LAUNCH(who);
   }
-  rc = transport(st.q_con, p->hord_dp, fx, fy, p->nord_t4, cols.damp_t_deln, st.delp, gx, gy);
+  rc = transport(st.pt, p->hord_tm, fx, fy, gx, gy);
   if (rc) return rc;
-  launch_flux_adjust<T>(s, d, m, st.q_con, st.delp, gx, gy);
-  FV3_HIP_CHECK_LAUNCH(who);
-  rc = transport(st.pt, p->hord_tm, fx, fy, p->nord_v4, cols.damp_vt_deln, st.delp, gx, gy);
-  if (rc) return rc;
-  launch_pt_delp<T>(s, d, m, st.pt, st.delp, gx, gy, fx, fy);
-  FV3_HIP_CHECK_LAUNCH(who);
+  {
+    const PtDelpEpilogue<T> epi{st.pt, st.delp, gx, gy, fx, fy, rarea, ptn, delpn, T(0), 0};
+    rc = deln(p->nord_v4, false, st.pt, cols.damp_vt_deln, epi, 8.0);
+    if (rc) return rc;
+  }
   switch (p->hord_mt) {
     case 5: launch_ke_ord<T, 5>(s, d, m, dt, st.uc, st.vc, st.u, st.v, ucc, vcc, ke); break;
     case 6: launch_ke_ord<T, 6>(s, d, m, dt, st.uc, st.vc, st.u, st.v, ucc, vcc, ke); break;
@@ -1033,7 +1221,8 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
     default: launch_ke_ord<T, 8>(s, d, m, dt, st.uc, st.vc, st.u, st.v, ucc, vcc, ke); break;
   }
   FV3_HIP_CHECK_LAUNCH(who);
-  launch_vorticity_adjust<T>(s, d, m, st.u, st.v, wk, st.w, st.delp, dw, st.q_con, cols.damp_w);
+  launch_vorticity_adjust<T>(s, d, m, nonhydro, st.u, st.v, wk, st.w, wgx, wgy, st.delp, delpn,
+                             st.pt, ptn, dw, st.q_con, qcn, cols.damp_w);
   FV3_HIP_CHECK_LAUNCH(who);
   // divergence damping
   const int k_lo = p->div_k0 < dom->nk ? p->div_k0 : dom->nk;
@@ -1045,20 +1234,32 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
   rc = run_div_high<T>(s, dom, m, p, cols, dt, wk, st.divgd, st.vc, st.uc, st.delpc, vort, ke,
                        a2x, a2e, W[19], who);
   if (rc) return rc;
-  launch_vort_diff<T>(s, d, m, vort, wk, vxd, vyd, vort2, cols.d_con_col);
+  launch_absolute_vort<T>(s, d, m, wk, vort2);
   FV3_HIP_CHECK_LAUNCH(who);
-  rc = transport(vort2, p->hord_vt, nullptr, nullptr, nullptr, nullptr, nullptr, fx, fy);
+  rc = transport(vort2, p->hord_vt, nullptr, nullptr, fx, fy);
   if (rc) return rc;
-  launch_uv_from_ke<T>(s, d, m, ke, fx, fy, st.u, st.v);
+  launch_uv_from_ke<T>(s, d, m, ke, fx, fy, st.u, st.v, us, vs);
   FV3_HIP_CHECK_LAUNCH(who);
-  rc = dsw_delnflux(dom, FV3_DELN_STORE, p->nord_v4, wk, nullptr, cols.damp_v_nosg, del6_u,
-                    del6_v, rarea, ut, vt, stream);
-  if (rc) return rc;
-  launch_heat_source<T>(s, d, m, vxd, vyd, ut, vt, st.u, st.v, st.delp, heat_s, st.heat_source,
-                        cols.d_con_col, p->d_con > kDconThreshold);
-  FV3_HIP_CHECK_LAUNCH(who);
-  launch_update_uv<T>(s, d, ut, vt, st.u, st.v, cols.damp_vt);
-  FV3_HIP_CHECK_LAUNCH(who);
+  {
+    VortDampEpilogue<T> epi{};
+    epi.us = us;
+    epi.vs = vs;
+    epi.vort = vort;
+    epi.delp = st.delp;
+    epi.heat_s = heat_s;
+    epi.rdx = m.rdx;
+    epi.rdy = m.rdy;
+    epi.rsin2 = m.rsin2;
+    epi.cosa_s = m.cosa_s;
+    epi.kef = cols.d_con_col;
+    epi.damp_vt = cols.damp_vt;
+    epi.u = st.u;
+    epi.v = st.v;
+    epi.heat_total = st.heat_source;
+    epi.d_con_on = p->d_con > kDconThreshold;
+    rc = deln(p->nord_v4, true, wk, cols.damp_v_nosg, epi, 10.0);
+    if (rc) return rc;
+  }
   return FV3_OK;
 }
 

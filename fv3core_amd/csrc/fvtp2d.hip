@@ -9,6 +9,7 @@
 #include "common.hpp"
 #include "timing.hpp"
 #include "ppm.hpp"
+#include "strip.hpp"
 
 namespace fv3 {
 
@@ -25,42 +26,6 @@ namespace fv3 {
 // last bit.  No LDS and no barriers: waves run independently.
 constexpr int MW = 64;        // lanes = strip columns
 constexpr int MTI = MW - 6;   // output interfaces per strip in i
-
-// Whole-wave shifts by one lane with DPP: wave_shr:1 (lane L reads lane
-// L - 1) and wave_shl:1 (lane L reads lane L + 1); the lane without a source
-// receives 0.  They are register moves on the VALU, without the LDS round
-// trip of a general lane permute.
-constexpr int kWaveShr1 = 0x138;
-constexpr int kWaveShl1 = 0x130;
-
-template <int CTRL>
-__device__ __forceinline__ int dpp32(int v) {
-  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL, typename T>
-__device__ __forceinline__ T dpp_shift(T v) {
-  if constexpr (sizeof(T) == 8) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)dpp32<CTRL>((int)(unsigned)u);
-    const unsigned hi = (unsigned)dpp32<CTRL>((int)(unsigned)(u >> 32));
-    return __builtin_bit_cast(T, ((unsigned long long)hi << 32) | lo);
-  } else if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(T, dpp32<CTRL>(__builtin_bit_cast(int, v)));
-  } else {
-    return (T)dpp32<CTRL>((int)v);
-  }
-}
-template <typename T>
-__device__ __forceinline__ T lane_dn(T v, int d) {  // value of lane + d
-  for (int n = 0; n < d; ++n) v = dpp_shift<kWaveShl1>(v);
-  return v;
-}
-template <typename T>
-__device__ __forceinline__ T lane_up(T v, int d) {  // value of lane - d
-  for (int n = 0; n < d; ++n) v = dpp_shift<kWaveShr1>(v);
-  return v;
-}
-
 
 // Face value al at face f (hord < 8, compute_al, xppm.py:147-181) from the
 // cells f-2, f-1, f, f+1 (qa..qd).  With EDGES every candidate is evaluated

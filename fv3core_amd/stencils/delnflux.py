@@ -1,7 +1,7 @@
 """DelnFlux and DelnFluxNoSG (fv3core/stencils/delnflux.py:901-1207) on the GPU.
 
 Both call the fused kernel ``fv3_delnflux``: d2 preamble, corner copies,
-the del-2 flux and the ``nmax`` higher-order passes run in LDS per block.
+the del-2 flux and the ``nmax`` higher-order passes in one march up the rows.
 """
 from __future__ import annotations
 

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from fv3core_amd.stencils.delnflux import DelnFluxNoSG
+from fv3core_amd.stencils.delnflux import DelnFlux, DelnFluxNoSG
 from fv3core_amd.stencils.fvtp2d import (
     CopiedCorners,
     FiniteVolumeTransport,
@@ -351,3 +351,73 @@ def test_fvtp2d_strips_and_segments(n, nz, tiles, hord, dtype):
     a = to_np(fx[0]).copy()
     a[sx] = 0.0
     assert not a.any()
+
+
+# Tiles narrower than the corner windows (one to three cells, where one window
+# spans the tile) and as narrow as two windows, one and two strips along i, few
+# and many planes (short segments along j and one whole one), bands that mix
+# the del-2 flux with one or two extra passes, all corners, one corner and none.
+@pytest.mark.parametrize("edges", [(True, True, True, True), (True, False, True, False),
+                                   (False, False, False, False)])
+@pytest.mark.parametrize("n,nz,tiles,bands", [
+    (1, 4, 1, [2, 2, 2, 2]), (2, 4, 1, [1, 1, 1, 1]), (3, 5, 1, [0, 0, 2, 2]),
+    (4, 4, 1, [2, 2, 2, 2]), (5, 4, 1, [0, 0, 0, 0]), (13, 4, 1, [0, 1, 0, 2]),
+    (57, 4, 1, [2, 2, 2, 2]), (58, 4, 1, [1, 0, 1, 1]), (13, 79, 60, [0, 0, 2, 2]),
+    (59, 40, 48, [2, 2, 2, 2])])
+@pytest.mark.parametrize("with_mass", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_delnflux_strips_windows_and_bands(n, nz, tiles, bands, edges, with_mass, dtype):
+    d = transport_inputs(n, nz, workload=33)
+    rng = np.random.default_rng(n)
+    shape = d["q"].shape
+    for name in ("del6_u", "del6_v"):
+        d[name] = rng.uniform(0.8, 1.2, d[name].shape)
+    d["rarea"] = rng.uniform(0.1, 0.2, d["rarea"].shape)
+    d["q"] = rng.normal(0.0, 1.0, shape)
+    d["mass"] = rng.uniform(0.5, 1.5, shape)
+    d["fx0"], d["fy0"] = rng.normal(0.0, 1.0, (2,) + shape)
+    if dtype == torch.float32:
+        d = {k: (v.astype(np.float32).astype(np.float64) if isinstance(v, np.ndarray) else v)
+             for k, v in d.items()}
+    grid, damp = grid_from_numpy(d, dtype=dtype)
+    damp = damp.__class__(damp.del6_u, damp.del6_v, 1.0, 1.0)
+    factory, gi = _factory(n, nz, edges)
+    nord = np.array(bands + [bands[3]] * (nz - 3), dtype=float)
+    damp_c = np.linspace(0.5, 0.9, nz + 1)
+
+    def batch(a):
+        t = utils.zeros((tiles,) + gi.max_shape, dtype=dtype)
+        t.copy_(torch.as_tensor(a, dtype=dtype))
+        return t
+
+    fx, fy = batch(d["fx0"]), batch(d["fy0"])
+    mass = batch(d["mass"]) if with_mass else None
+    DelnFlux(factory, damp, grid.rarea, nord, damp_c)(batch(d["q"]), fx, fy, mass=mass)
+    sx2, sy2 = batch(d["fx0"]), batch(d["fy0"])
+    column = np.linspace(0.5, 1.5, nz)
+    DelnFluxNoSG(factory, damp, grid.rarea, nord)(batch(d["q"]), sx2, sy2, column, mass=mass)
+    torch.cuda.synchronize()
+
+    t = _tile(n, edges)
+    mass_np = d["mass"][:, :, :nz] if with_mass else None
+    args = (d["del6_u"], d["del6_v"], d["rarea"])
+    rfx, rfy = ofv.delnflux(d["q"][:, :, :nz], d["fx0"][:, :, :nz], d["fy0"][:, :, :nz], *args,
+                            nord, damp_c, 1.0, t, mass=mass_np)
+    rsx, rsy = ofv.delnflux_nosg(d["q"][:, :, :nz], *args, bands, column, t, mass=mass_np)
+    sx = (slice(3, n + 4), slice(3, n + 3), slice(0, nz))
+    sy = (slice(3, n + 3), slice(3, n + 4), slice(0, nz))
+    # Every pass takes differences of values of one size: at most two roundings
+    # of a pass's terms enter each of its five sums, four neighbours times the
+    # metric factors (below 1) deep, so 64 roundings of the largest term of the
+    # passes, which is no more than 2 * 1.2 times the largest input.
+    eps = 2.0 ** (-53 if dtype == torch.float64 else -24)
+    for tile in {0, tiles - 1}:
+        for got, ref, sl, start in ((fx, rfx, sx, "fx0"), (fy, rfy, sy, "fy0"),
+                                    (sx2, rsx, sx, "fx0"), (sy2, rsy, sy, "fy0")):
+            scale = 2.4 * max(np.abs(d["q"]).max(), np.abs(ref[sl]).max())
+            err = np.abs(to_np(got[tile])[sl] - ref[sl]).max()
+            assert err <= 64 * eps * scale, (err, scale)
+            # nothing is written outside the fluxes
+            rest = to_np(got[tile]).copy() - d[start]
+            rest[sl] = 0.0
+            assert not rest.any()
