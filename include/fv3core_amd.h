@@ -211,7 +211,8 @@ int32_t fv3_delnflux_f32(const fv3_domain* d, int32_t mode, const int32_t nord4[
  * kord <= 10 (its magnitude selects the limiter), mode = iv in {-2,...,2};
  * qs (IJ, bottom value for iv = -2) may be NULL (then 0); qmin is the
  * kord-9 floor.  work: 7 slabs, each of work_slab elements laid out like the
- * fields (work_slab >= (ntiles-1)*st + (km+1)*sk).
+ * fields (work_slab >= (ntiles-1)*st + (km+1)*sk); left alone for km <= 128,
+ * where a column's intermediates stay on chip.
  */
 int32_t fv3_map_single_f64(const fv3_domain* d, int32_t kord, int32_t mode, int32_t i1,
                            int32_t i2, int32_t j1, int32_t j2, double* q1, const double* pe1,

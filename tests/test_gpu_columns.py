@@ -230,3 +230,60 @@ def test_riem_solver_c_wide_offsets():
         torch.cuda.empty_cache()
     assert np.isfinite(out[0][0]).all()
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+# Column heights at the edges of a set, a wave and a workgroup of each set size
+# and past the kernel that spreads layers; a box that does not fill a workgroup.
+@pytest.mark.parametrize("nz", [6, 7, 20, 21, 80, 81, 128, 129])
+@pytest.mark.parametrize("kord,mode", [(9, 1), (10, 0), (10, -2), (8, -1), (9, 2)])
+def test_map_single_layer_sets(nz, kord, mode):
+    n = 5
+    factory, gi = _factory(n, nz)
+    box = (gi.isc, gi.iec, gi.jsc, gi.jec - 1)
+    rng = np.random.default_rng(nz)
+    shape = gi.max_shape[:2] + (nz + 1,)
+    pe1 = 100.0 + np.cumsum(rng.uniform(500.0, 1500.0, shape), axis=2)
+    pe2 = pe1.copy()
+    # target interfaces up to two layers away, in order, ends in common
+    pe2[..., 1:-1] = np.sort(pe1[..., 1:-1] + rng.uniform(-1500.0, 1500.0, shape)[..., 1:-1])
+    pe2 = np.clip(pe2, pe1[..., :1] + np.arange(nz + 1), pe1[..., -1:] - np.arange(nz, -1, -1))
+    src = rng.normal(0.0, 1.0, shape) + np.sin(0.4 * np.arange(nz + 1))
+    if mode == 0:
+        src = np.abs(src)
+    qs = rng.normal(0.0, 1.0, shape[:2]) if mode == -2 else None
+    q1 = to_storage(src)
+    MapSingle(factory, kord, mode, *box)(q1, to_storage(pe1), to_storage(pe2),
+                                         qs=None if qs is None else to_storage(qs))
+    torch.cuda.synchronize()
+    ref = orm.map_single(src, pe1, pe2, kord, mode, *box, qs=qs)
+    # a target layer's integral is a difference of parabola terms of the
+    # field's size over at least a thousandth of a layer, so values near zero
+    # are compared on the field's scale
+    err = np.abs(to_np(q1)[..., :nz] - ref[..., :nz]).max()
+    assert err <= 1e-12 * np.abs(src).max(), err
+
+
+def test_map_single_unordered_and_special_columns():
+    """Columns whose target interfaces are out of order, and columns with an
+    infinity, a NaN or zeros in the field: as the oracle's walk from the top."""
+    n = 4
+    d = remap_inputs(n, NZ, workload=53)
+    factory, gi = _factory(n)
+    src, pe1, pe2 = d["pt"].copy(), d["pe1"].copy(), d["pe2"].copy()
+    c = gi.isc
+    pe2[c, c, 30], pe2[c, c, 33] = pe2[c, c, 33], pe2[c, c, 30]
+    pe2[c + 1, c, 5] = 0.5 * (pe1[c + 1, c, 40] + pe1[c + 1, c, 41])
+    src[c + 2, c, 20] = np.inf
+    src[c + 3, c, 50] = np.nan
+    src[c, c + 1, :] = 0.0
+    q1 = to_storage(src)
+    box = (gi.isc, gi.iec, gi.jsc, gi.jec)
+    MapSingle(factory, 9, 1, *box)(q1, to_storage(pe1), to_storage(pe2))
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        ref = orm.map_single(src, pe1, pe2, 9, 1, *box)
+    got = to_np(q1)[..., :NZ]
+    finite = np.isfinite(ref[..., :NZ])
+    assert (np.isfinite(got) == finite).all()
+    assert_close(np.where(finite, got, 0.0), np.where(finite, ref[..., :NZ], 0.0), 1e-12,
+                 what="q1")
