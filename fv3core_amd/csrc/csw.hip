@@ -2,23 +2,27 @@
 // CGridShallowWaterDynamics (c_sw).
 //
 // Reference: fv3core/stencils/d2a2c_vect.py:1-651, fv3core/stencils/c_sw.py:
-// 1-659.  Each launch is one pointwise pass over an index box; statements of
-// the reference that only feed a neighbour's value (GT4Py temporaries read
-// at an offset) are recomputed at that neighbour instead of being stored.
-// Region statements become index tests against the tile-edge anchors, with
-// the reference's statement order deciding which formula a point gets.
+// 1-659.  Three marches up the rows of each level, 64 columns to a wave, the
+// neighbours across i by lane shifts and those across j in registers, so that
+// only what a later march needs goes through memory.  Region statements become
+// index tests against the tile-edge anchors, with the reference's statement
+// order deciding which formula a point gets.
 //
 // Launch sequence of fv3_c_sw (workspace slabs in brackets):
-//   1 d2a:    utmp, vtmp on the full domain [W0, W1]; ua, va
-//   2 fill:   x corner fills of utmp (3 cells) and ua (2 cells)
-//   3 uc:     uc, ut (ut_main + east_west_edges, then geoadjust_ut)
-//   4 fill:   y corner fills of vtmp and va; x fills of delp, pt, w
-//   5 vc:     vc, vt (north_south_edges + vt_main, then geoadjust_vt)
-//   6 fluxx:  fx, fx1, fx2 [W2..W4]; divergence_corner -> divgd (nord > 0)
-//   7 fill:   y corner fills of delp, pt, w
-//   8 trans:  delpc, ptc, omga, ke [W5]
-//   9 vort:   circulation_cgrid + absolute_vorticity [W6]
-//  10 update: update_y_velocity (vc) and update_x_velocity (uc)
+//   1 fill:      x, then y corner fills of delp, pt, w
+//   2 d2a2c:     ua, va, ut, vt; uc, vc before the update [W0, W1]
+//   3 transport: delpc, ptc, omga, ke [W2]; divergence_corner -> divgd (nord > 0)
+//   4 update:    vorticity; update_y_velocity (vc), update_x_velocity (uc)
+//
+// What bounds it: memory, at about half the rate of a large copy (a wave streams
+// up to 16 fields in pieces of 512 bytes; rows per segment from 9 to 35, 1 to 16
+// waves a workgroup, tiles spread over the XCDs or kept on one and non-temporal
+// stores all measure within 10 %).  31 passes over full-size fields against 54
+// of one pointwise pass per stencil.  Measured, FP64, 79 levels: six C97 tiles
+// 593 -> 420 us (d2a2c 169 -> 126, transport with the divergence 301 -> 195,
+// update with the vorticity 112 -> 97); 96 C48 tiles in FP32 1510 -> 975 us;
+// six C12 tiles, where a launch is its latency, 52 us as before.
+#include "strip.hpp"
 #include "stencil.hpp"
 
 namespace fv3 {
@@ -73,334 +77,445 @@ __device__ __forceinline__ T contravariant(T v1, T v2, T cosa, T rsin2) {
 }
 
 // ---------------------------------------------------------------- d2a2c_vect
-// set_tmps, lagrange_interpolation_y_p1/x_p1, avg_box, contravariant_components
+// set_tmps, lagrange_interpolation_y_p1/x_p1, avg_box, contravariant_components,
+// ut_main + east_west_edges, north_south_edges + vt_main and, when geo != 0,
+// geoadjust_ut / geoadjust_vt, as one march: at row r the strip forms the A-grid
+// winds of row r, uc of row r and vc of row r - 1.
+//
+// The corner fills turn the interpolated covariant winds (and the A-grid winds)
+// by a quarter: a cell (is - 1 - a, js - 1) takes -+ the other component of
+// (is - 1, js + a) before uc is formed, a cell (is - 1, js - 1 - a) that of
+// (is + a, js - 1) before vc is formed, and so at the other corners.  The few
+// lanes and rows they reach form the other component from u and v again.
 template <typename T>
-void launch_d2a(hipStream_t s, const Dom& d, const D2A2CBounds& b, const Met<T>& m,
-                const T* u, const T* v, T* utmp, T* vtmp, T* ua, T* va) {
-  const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
-  launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
+struct D2A2C {
+  D2A2CBounds b;
+  Met<T> m;
+  int geo;
+  T dt2;
+  const T *u, *v;
+  T *ua, *va, *uc, *vc, *utc, *vtc;
+
+  // utmp / vtmp of any cell from u rows j - 1 .. j + 2 / v columns i - 1 .. i + 2
+  __device__ __forceinline__ T ut_of(bool band, int i, int j, T um, T u0, T u1, T u2) const {
+    if (band) return T(0.5) * (u0 + u1);
+    return i >= b.is1 && i <= b.ie1 && j >= b.js1 && j <= b.je1
+               ? T(kA2) * (um + u2) + T(kA1) * (u0 + u1)
+               : T(kBigNumber);
+  }
+  __device__ __forceinline__ T vt_of(bool band, int i, int j, T vm, T v0, T v1, T v2) const {
+    if (band) return T(0.5) * (v0 + v1);
+    return i >= b.is2 && i <= b.ie2 && j >= b.js2 && j <= b.je2
+               ? T(kA2) * (vm + v2) + T(kA1) * (v0 + v1)
+               : T(kBigNumber);
+  }
+  __device__ __forceinline__ bool band(const Dom& d, int i, int j) const {
     const int off = b.avg_offset;
-    const bool band = j < d.js + off || j > d.je - off || i < d.is + off || i > d.ie - off;
-    T ut, vt;
-    if (band) {
-      ut = T(0.5) * (u[o] + u[o + d.sj]);
-      vt = T(0.5) * (v[o] + v[o + 1]);
-    } else {
-      ut = (i >= b.is1 && i <= b.ie1 && j >= b.js1 && j <= b.je1)
-               ? T(kA2) * (u[o - d.sj] + u[o + 2 * d.sj]) + T(kA1) * (u[o] + u[o + d.sj])
-               : T(kBigNumber);
-      vt = (i >= b.is2 && i <= b.ie2 && j >= b.js2 && j <= b.je2)
-               ? T(kA2) * (v[o - 1] + v[o + 2]) + T(kA1) * (v[o] + v[o + 1])
-               : T(kBigNumber);
-    }
-    utmp[o] = ut;
-    vtmp[o] = vt;
-    if (i >= d.isc - 2 && i <= d.iec + 2 && j >= d.jsc - 2 && j <= d.jec + 2) {
-      const int64_t o2 = at2(d, i, j, t);
-      const T cs = m.cosa_s[o2], r2 = m.rsin2[o2];
-      ua[o] = contravariant(ut, vt, cs, r2);
-      va[o] = contravariant(vt, ut, cs, r2);
-    }
-  });
-}
+    return j < d.js + off || j > d.je - off || i < d.is + off || i > d.ie - off;
+  }
 
-// ut_main + east_west_edges (+ geoadjust_ut when geo != 0), on
-// [isc-1, iec+2] x [jsc-1, jec+1].
-template <typename T>
-void launch_uc(hipStream_t s, const Dom& d, const D2A2CBounds& b, const Met<T>& m, int geo,
-               T dt2, const T* utmp, const T* ua, const T* v, T* uc, T* utc) {
-  const Box bx{d.isc - 1, d.iec + 2, d.jsc - 1, d.jec + 1};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const int64_t o2 = at2(d, i, j, t);
-    T ucv, utv;
-    if (i == d.is - 1 || i == d.ie) {
-      ucv = T(kC1) * utmp[o - 2] + T(kC2) * utmp[o - 1] + T(kC3) * utmp[o];
-      utv = contravariant(ucv, v[o], m.cosa_u[o2], m.rsin_u[o2]);
-    } else if (i == d.is || i == d.ie + 1) {
-      // edge_interpolate4_x (d2a2c_vect.py:254-260; n2 uses t1 as there)
-      const T dm2 = m.dxa[o2 - 2], dm1 = m.dxa[o2 - 1], d0 = m.dxa[o2], dp1 = m.dxa[o2 + 1];
-      const T t1 = dm2 + dm1, t2 = d0 + dp1;
-      const T n1 = (t1 + dm1) * ua[o - 1] - dm1 * ua[o - 2];
-      const T n2 = (t1 + d0) * ua[o] - d0 * ua[o + 1];
-      utv = T(0.5) * (n1 / t1 + n2 / t2);
-      ucv = utv > T(0) ? utv * m.sin_sg3[o2 - 1] : utv * m.sin_sg1[o2];
-    } else if (i == d.is + 1 || i == d.ie + 2) {
-      ucv = T(kC1) * utmp[o + 1] + T(kC2) * utmp[o] + T(kC3) * utmp[o - 1];
-      utv = contravariant(ucv, v[o], m.cosa_u[o2], m.rsin_u[o2]);
-    } else if (i >= b.ifirst && i <= b.ilast) {
-      ucv = T(kA2) * (utmp[o - 2] + utmp[o + 1]) + T(kA1) * (utmp[o - 1] + utmp[o]);
-      utv = contravariant(ucv, v[o], m.cosa_u[o2], m.rsin_u[o2]);
-    } else {
-      return;
-    }
-    uc[o] = ucv;
-    if (geo) {
-      utv = utv > T(0) ? dt2 * utv * m.dy[o2] * m.sin_sg3[o2 - 1]
-                       : dt2 * utv * m.dy[o2] * m.sin_sg1[o2];
-    }
-    utc[o] = utv;
-  });
-}
+  // what a corner fill reads: both components at cell (i, j), which lies in the
+  // band beside the tile edges
+  __device__ __forceinline__ void cell(const Dom& d, int64_t o3, int64_t o2, int i, int j, T& ut,
+                                       T& vt, T& uaa, T& vaa) const {
+    const T *pu = u + o3 + (int64_t)j * d.sj + i, *pv = v + o3 + (int64_t)j * d.sj + i;
+    const int64_t om = o2 + (int64_t)j * d.sj2 + i;
+    ut = T(0.5) * (pu[0] + pu[d.sj]);
+    vt = T(0.5) * (pv[0] + pv[1]);
+    uaa = contravariant(ut, vt, m.cosa_s[om], m.rsin2[om]);
+    vaa = contravariant(vt, ut, m.cosa_s[om], m.rsin2[om]);
+  }
 
-// north_south_edges + vt_main (+ geoadjust_vt), on [isc-1, iec+1] x [jsc-1, jec+2].
-template <typename T>
-void launch_vc(hipStream_t s, const Dom& d, const D2A2CBounds& b, const Met<T>& m, int geo,
-               T dt2, const T* vtmp, const T* va, const T* u, T* vc, T* vtc) {
-  const Box bx{d.isc - 1, d.iec + 1, d.jsc - 1, d.jec + 2};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const int64_t o2 = at2(d, i, j, t);
-    const int64_t sj = d.sj, sj2 = d.sj2;
-    T vcv, vtv;
-    if (j >= b.jfirst && j <= b.jlast) {
-      vcv = T(kA2) * (vtmp[o - 2 * sj] + vtmp[o + sj]) + T(kA1) * (vtmp[o - sj] + vtmp[o]);
-      vtv = contravariant(vcv, u[o], m.cosa_v[o2], m.rsin_v[o2]);
-    } else if (j == d.js - 1 || j == d.je) {
-      vcv = T(kC1) * vtmp[o - 2 * sj] + T(kC2) * vtmp[o - sj] + T(kC3) * vtmp[o];
-      vtv = contravariant(vcv, u[o], m.cosa_v[o2], m.rsin_v[o2]);
-    } else if (j == d.js || j == d.je + 1) {
-      const T dm2 = m.dya[o2 - 2 * sj2], dm1 = m.dya[o2 - sj2], d0 = m.dya[o2],
-              dp1 = m.dya[o2 + sj2];
-      const T t1 = dm2 + dm1, t2 = d0 + dp1;
-      const T n1 = (t1 + dm1) * va[o - sj] - dm1 * va[o - 2 * sj];
-      const T n2 = (t1 + d0) * va[o] - d0 * va[o + sj];
-      vtv = T(0.5) * (n1 / t1 + n2 / t2);
-      vcv = vtv > T(0) ? vtv * m.sin_sg4[o2 - sj2] : vtv * m.sin_sg2[o2];
-    } else if (j == d.js + 1 || j == d.je + 2) {
-      vcv = T(kC1) * vtmp[o + sj] + T(kC2) * vtmp[o] + T(kC3) * vtmp[o - sj];
-      vtv = contravariant(vcv, u[o], m.cosa_v[o2], m.rsin_v[o2]);
-    } else {
-      vcv = T(kA2) * (vtmp[o - 2 * sj] + vtmp[o + sj]) + T(kA1) * (vtmp[o - sj] + vtmp[o]);
-      vtv = contravariant(vcv, u[o], m.cosa_v[o2], m.rsin_v[o2]);
-    }
-    vc[o] = vcv;
-    if (geo) {
-      vtv = vtv > T(0) ? dt2 * vtv * m.dx[o2] * m.sin_sg4[o2 - sj2]
-                       : dt2 * vtv * m.dx[o2] * m.sin_sg2[o2];
-    }
-    vtc[o] = vtv;
-  });
-}
+  __device__ __forceinline__ void operator()(const Dom& d, int i0, int r0, int rows, int k,
+                                             int t) const {
+    const int lane = threadIdx.x, i = i0 - 2 + lane;
+    const StripColumn<T> col(d, i);
+    const int64_t o3 = (int64_t)t * d.st + (int64_t)k * d.sk, o2 = (int64_t)t * d.st2;
+    const bool out = lane >= 2 && lane < 62;
+    const bool a_i = out && i <= d.iec + 2, uc_i = a_i && i >= d.isc - 1,
+               vc_i = uc_i && i <= d.iec + 1;
+    const bool cl = i < d.is || i > d.ie;  // a corner's columns
+    // x's edge formulas (east_west_edges)
+    const bool xe = i == d.is || i == d.ie + 1, xl = i == d.is - 1 || i == d.ie,
+               xr = !xl && (i == d.is + 1 || i == d.ie + 2);
+    struct Row {
+      T v, u3, cs, r2, cu, ru, dy, s3, s1, dxa, cv, rv, dx, s4, s2;
+    };
+    auto load = [&](int r) {
+      Row w;
+      w.v = col.f(v + o3, r);
+      w.u3 = col.f(u + o3, r + 2);
+      w.cs = col.m(m.cosa_s + o2, r);
+      w.r2 = col.m(m.rsin2 + o2, r);
+      w.cu = col.m(m.cosa_u + o2, r);
+      w.ru = col.m(m.rsin_u + o2, r);
+      w.s3 = col.m(m.sin_sg3 + o2, r, -1);
+      w.s1 = col.m(m.sin_sg1 + o2, r);
+      w.dxa = col.m(m.dxa + o2, r);
+      w.cv = col.m(m.cosa_v + o2, r - 1);
+      w.rv = col.m(m.rsin_v + o2, r - 1);
+      w.s4 = col.m(m.sin_sg4 + o2, r - 2);
+      w.s2 = col.m(m.sin_sg2 + o2, r - 1);
+      w.dy = geo ? col.m(m.dy + o2, r) : T(0);
+      w.dx = geo ? col.m(m.dx + o2, r - 1) : T(0);
+      return w;
+    };
+    const int ra = r0 - 3;
+    T um = 0, u0 = col.f(u + o3, ra - 1), u1 = col.f(u + o3, ra), u2 = col.f(u + o3, ra + 1);
+    T vt1 = 0, vt2 = 0, vt3 = 0, va1 = 0, va2 = 0, va3 = 0;  // rows r - 1 .. r - 3
+    strip_march(ra, r0 + rows - 1, load(ra), [&](int r, const Row& w, Row& nx) {
+      nx = load(r + 1);
+      um = u0;
+      u0 = u1;
+      u1 = u2;
+      u2 = w.u3;
+      const bool bd = band(d, i, r);
+      const T v1 = lane_dn(w.v, 1);
+      const T ut = ut_of(bd, i, r, um, u0, u1, u2);
+      const T vt = vt_of(bd, i, r, lane_up(w.v, 1), w.v, v1, lane_dn(v1, 1));
+      T utx = ut, vty = vt;
+      T uax = contravariant(ut, vt, w.cs, w.r2), vay = contravariant(vt, ut, w.cs, w.r2);
+      if (r < d.js || r > d.je) {
+        if (cl) {
+          const bool south = r < d.js, west = i < d.is;
+          const int ax = west ? d.is - 1 - i : i - d.ie - 1, ay = south ? d.js - 1 - r : r - d.je - 1;
+          const T mult = west == south ? T(-1) : T(1);
+          T cut, cvt, cua, cva;
+          if (ay == 0 && ax < 3) {
+            cell(d, o3, o2, west ? d.is - 1 : d.ie + 1, south ? d.js + ax : d.je - ax, cut, cvt,
+                 cua, cva);
+            utx = mult * cvt;
+            if (ax < 2) uax = mult * cva;
+          }
+          if (ax == 0 && ay < 3) {
+            cell(d, o3, o2, west ? d.is + ay : d.ie - ay, south ? d.js - 1 : d.je + 1, cut, cvt,
+                 cua, cva);
+            vty = mult * cut;
+            if (ay < 2) vay = mult * cua;
+          }
+        }
+      }
+      // uc of row r
+      T ucv, utv;
+      {
+        const T tm2 = lane_up(utx, 2), tm1 = lane_up(utx, 1), tp1 = lane_dn(utx, 1);
+        const T am2 = lane_up(uax, 2), am1 = lane_up(uax, 1), ap1 = lane_dn(uax, 1);
+        const T dm2 = lane_up(w.dxa, 2), dm1 = lane_up(w.dxa, 1), dp1 = lane_dn(w.dxa, 1);
+        if (xl || xr)
+          ucv = T(kC1) * (xl ? tm2 : tp1) + T(kC2) * (xl ? tm1 : utx) + T(kC3) * (xl ? utx : tm1);
+        else
+          ucv = T(kA2) * (tm2 + tp1) + T(kA1) * (tm1 + utx);
+        utv = contravariant(ucv, w.v, w.cu, w.ru);
+        if (xe) {
+          // edge_interpolate4_x (d2a2c_vect.py:254-260; n2 uses t1 as there)
+          const T t1 = dm2 + dm1, t2 = w.dxa + dp1;
+          const T n1 = (t1 + dm1) * am1 - dm1 * am2;
+          const T n2 = (t1 + w.dxa) * uax - w.dxa * ap1;
+          utv = T(0.5) * (n1 / t1 + n2 / t2);
+          ucv = utv > T(0) ? utv * w.s3 : utv * w.s1;
+        }
+        if (geo) utv = utv > T(0) ? dt2 * utv * w.dy * w.s3 : dt2 * utv * w.dy * w.s1;
+      }
+      // vc of row j = r - 1
+      const int j = r - 1;
+      T vcv, vtv;
+      const bool jm = j >= b.jfirst && j <= b.jlast;
+      if (!jm && (j == d.js || j == d.je + 1) && j != d.js - 1 && j != d.je) {
+        const T dm2 = col.m(m.dya + o2, j - 2), dm1 = col.m(m.dya + o2, j - 1),
+                d0 = col.m(m.dya + o2, j), dp1 = col.m(m.dya + o2, j + 1);
+        const T t1 = dm2 + dm1, t2 = d0 + dp1;
+        const T n1 = (t1 + dm1) * va2 - dm1 * va3;
+        const T n2 = (t1 + d0) * va1 - d0 * vay;
+        vtv = T(0.5) * (n1 / t1 + n2 / t2);
+        vcv = vtv > T(0) ? vtv * w.s4 : vtv * w.s2;
+      } else {
+        if (!jm && (j == d.js - 1 || j == d.je))
+          vcv = T(kC1) * vt3 + T(kC2) * vt2 + T(kC3) * vt1;
+        else if (!jm && (j == d.js + 1 || j == d.je + 2))
+          vcv = T(kC1) * vty + T(kC2) * vt1 + T(kC3) * vt2;
+        else
+          vcv = T(kA2) * (vt3 + vty) + T(kA1) * (vt2 + vt1);
+        vtv = contravariant(vcv, um, w.cv, w.rv);
+      }
+      if (geo) vtv = vtv > T(0) ? dt2 * vtv * w.dx * w.s4 : dt2 * vtv * w.dx * w.s2;
+      const bool sa = a_i && r >= r0 && r <= d.jec + 2;
+      const bool su = uc_i && r >= r0 && r >= d.jsc - 1 && r <= d.jec + 1;
+      const bool sv = vc_i && r >= r0 && j >= d.jsc - 1;
+      col.store(ua + o3, r, uax, sa);
+      col.store(va + o3, r, vay, sa);
+      col.store(uc + o3, r, ucv, su);
+      col.store(utc + o3, r, utv, su);
+      col.store(vc + o3, j, vcv, sv);
+      col.store(vtc + o3, j, vtv, sv);
+      vt3 = vt2;
+      vt2 = vt1;
+      vt1 = vty;
+      va3 = va2;
+      va2 = va1;
+      va1 = vay;
+    });
+  }
+};
 
-const int kCornerMult[4] = {-1, 1, 1, -1};  // sw, se, nw, ne (d2a2c_vect.py:24-38)
-const int kUnitMult[4] = {1, 1, 1, 1};
-
-// The d2a2c part shared by fv3_d2a2c_vect and fv3_c_sw.  When extra_x is
-// set, the x corner fills of delp, pt, w (fields 4, 5, 6 of ff) ride along
-// with the y fills of vtmp and va.
+// The d2a2c part shared by fv3_d2a2c_vect and fv3_c_sw.
 template <typename T>
 int run_d2a2c(hipStream_t s, const fv3_domain* dom, const Met<T>& m, int geo, T dt2, T* uc,
-              T* vc, const T* u, const T* v, T* ua, T* va, T* utc, T* vtc, T* utmp, T* vtmp,
-              T* delp, T* pt, T* w, const char* who) {
-  Dom d = to_dom(dom);
-  const D2A2CBounds b = d2a2c_bounds(dom);
-  const Box edges{dom->isc - 3, dom->iec + 3, dom->jsc - 3, dom->jec + 3};
-  FillFields<T> ff{};
-  ff.f[0] = utmp;
-  ff.f[1] = vtmp;
-  ff.f[2] = ua;
-  ff.f[3] = va;
-  ff.f[4] = delp;
-  ff.f[5] = pt;
-  ff.f[6] = w;
-  launch_d2a(s, d, b, m, u, v, utmp, vtmp, ua, va);
-  FV3_HIP_CHECK_LAUNCH(who);
-  FillTable fx;
-  fx.n = 0;
-  append_fill(&fx, dom, kFill3X, 0, 1, kCornerMult, edges);
-  append_fill(&fx, dom, kFill2X, 2, 3, kCornerMult, edges);
-  launch_fill(s, d, fx, ff);
-  FV3_HIP_CHECK_LAUNCH(who);
-  launch_uc(s, d, b, m, geo, dt2, utmp, ua, v, uc, utc);
-  FV3_HIP_CHECK_LAUNCH(who);
-  FillTable fy;
-  fy.n = 0;
-  append_fill(&fy, dom, kFill3Y, 1, 0, kCornerMult, edges);
-  append_fill(&fy, dom, kFill2Y, 3, 2, kCornerMult, edges);
-  if (delp) {
-    for (int f = 4; f <= 6; ++f) append_fill(&fy, dom, kFill2X, f, f, kUnitMult, edges);
-  }
-  launch_fill(s, d, fy, ff);
-  FV3_HIP_CHECK_LAUNCH(who);
-  launch_vc(s, d, b, m, geo, dt2, vtmp, va, u, vc, vtc);
-  FV3_HIP_CHECK_LAUNCH(who);
-  return FV3_OK;
+              T* vc, const T* u, const T* v, T* ua, T* va, T* utc, T* vtc, const char* who) {
+  const Dom d = to_dom(dom);
+  const D2A2C<T> f{d2a2c_bounds(dom), m, geo, dt2, u, v, ua, va, uc, vc, utc, vtc};
+  return launch_strips(s, d, d.isc - 2, d.iec + 2, d.jsc - 2, d.jec + 3, 60, 3, f, who);
 }
 
 // ----------------------------------------------------------------------- c_sw
-// compute_nonhydro_fluxes_x on [isc-1, iec+2] x [jsc-1, jec+1] and, when
-// divgd is given, divergence_corner on [isc, iec+1] x [jsc, jec+1].
+// compute_nonhydro_fluxes_x, transportdelp_update_vorticity_and_kineticenergy
+// on [isc-1, iec+1]^2 with initialize_delpc_ptc (zero) on the rest of the full
+// domain and, when divg is given, divergence_corner on [isc, iec+1] x
+// [jsc, jec+1]: at row r the strip forms the x fluxes and the divergence of row
+// r and finishes the cells of row r - 1.
+//
+// delp, pt and w hold the x corner fills with the y fills over them; only the
+// cell next to a corner, (is - 1, js - 1), differs between the two, and the x
+// fluxes take it from (is - 1, js), where the x fill reads.
 template <typename T>
-void launch_fluxx_div(hipStream_t s, const Dom& d, const Met<T>& m, const T* delp, const T* pt,
-                      const T* w, const T* utc, T* fx, T* fx1, T* fx2, const T* u, const T* v,
-                      const T* ua, const T* va, T* divg) {
-  const Box bx{d.isc - 1, d.iec + 2, d.jsc - 1, d.jec + 1};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    {
-      const T c = utc[o];
-      const int64_t up = c > T(0) ? o - 1 : o;
-      const T f1 = c * delp[up];
-      fx1[o] = f1;
-      fx[o] = f1 * pt[up];
-      fx2[o] = f1 * w[up];
-    }
-    if (divg == nullptr || i < d.isc || i > d.iec + 1 || j < d.jsc) return;
-    // divergence_corner (c_sw.py:172-289)
-    const int64_t o2 = at2(d, i, j, t);
-    const int64_t sj = d.sj, sj2 = d.sj2;
-    const T half = T(0.5), quarter = T(0.25);
-    const T dxc = m.dxc[o2], dyc = m.dyc[o2];
-    const T s1 = m.sin_sg1[o2], s2 = m.sin_sg2[o2];
-    const T s3m = m.sin_sg3[o2 - 1], s4m = m.sin_sg4[o2 - sj2];
-    const T ra = m.rarea_c[o2];
-    const bool west = i == d.is || i == d.ie + 1;
-    const bool south = j == d.js || j == d.je + 1;
-    // uf, vf at the point; uf1 (i-1), vf1 (j-1) in the variants the regions use
-    const T uf = (u[o] - quarter * (va[o - sj] + va[o]) * (m.cos_sg4[o2 - sj2] + m.cos_sg2[o2])) *
-                 dyc * half * (s4m + s2);
-    const T vf = (v[o] - quarter * (ua[o - 1] + ua[o]) * (m.cos_sg3[o2 - 1] + m.cos_sg1[o2])) *
-                 dxc * half * (s3m + s1);
-    T out;
-    if (west && south) {
-      const T uf1 = u[o - 1] * m.dyc[o2 - 1] * half * (m.sin_sg4[o2 - 1 - sj2] + m.sin_sg2[o2 - 1]);
-      const T uf0 = u[o] * dyc * half * (s4m + s2);
-      const T vf0 = v[o] * dxc * half * (s3m + s1);
-      if (j == d.js) {
-        out = (-vf0 + uf1 - uf0) * ra;
-      } else {
-        const T vf1 =
-            v[o - sj] * m.dxc[o2 - sj2] * half * (m.sin_sg3[o2 - 1 - sj2] + m.sin_sg1[o2 - sj2]);
-        out = (vf1 + uf1 - uf0) * ra;
+struct CswTransport {
+  Met<T> m;
+  T dt2;
+  const T *delp, *pt, *w, *utc, *vtc, *ua, *va, *uc, *vc, *u, *v;
+  T *delpc, *ptc, *wc, *ke, *divg;
+
+  __device__ __forceinline__ void operator()(const Dom& d, int i0, int j0, int rows, int k,
+                                             int t) const {
+    const int lane = threadIdx.x, i = i0 - 1 + lane;
+    const StripColumn<T> col(d, i);
+    const int64_t o3 = (int64_t)t * d.st + (int64_t)k * d.sk, o2 = (int64_t)t * d.st2;
+    const bool out = lane >= 1 && lane < 63 && i <= d.iec + 3;
+    const bool cell_i = out && i >= d.isc - 1 && i <= d.iec + 1;
+    const bool div_i = out && i >= d.isc && i <= d.iec + 1;
+    const bool west = i == d.is || i == d.ie + 1;  // beside a tile edge
+    const bool kl = i == d.ie || i == d.is - 1, kr = !kl && west;
+    const bool corner = i == d.is - 1 || i == d.ie + 1;
+    // rows that only hold zeros
+    for (int j = j0; j < j0 + rows; ++j) {
+      if (j >= d.jsc - 1 && j <= d.jec + 1) continue;
+      if (out) {
+        (delpc + o3 + (int64_t)j * d.sj)[i] = T(0);
+        (ptc + o3 + (int64_t)j * d.sj)[i] = T(0);
       }
-    } else if (south) {
-      const T uf0 = u[o] * dyc * half * (s4m + s2);
-      const T uf1 = u[o - 1] * m.dyc[o2 - 1] * half * (m.sin_sg4[o2 - 1 - sj2] + m.sin_sg2[o2 - 1]);
-      const T vf1 = (v[o - sj] - quarter * (ua[o - 1 - sj] + ua[o - sj]) *
-                                     (m.cos_sg3[o2 - 1 - sj2] + m.cos_sg1[o2 - sj2])) *
-                    m.dxc[o2 - sj2] * half * (m.sin_sg3[o2 - 1 - sj2] + m.sin_sg1[o2 - sj2]);
-      out = (vf1 - vf + uf1 - uf0) * ra;
-    } else if (west) {
-      const T vf0 = v[o] * dxc * half * (s3m + s1);
-      const T vf1 =
-          v[o - sj] * m.dxc[o2 - sj2] * half * (m.sin_sg3[o2 - 1 - sj2] + m.sin_sg1[o2 - sj2]);
-      const T uf1 = (u[o - 1] - quarter * (va[o - 1 - sj] + va[o - 1]) *
-                                    (m.cos_sg4[o2 - 1 - sj2] + m.cos_sg2[o2 - 1])) *
-                    m.dyc[o2 - 1] * half * (m.sin_sg4[o2 - 1 - sj2] + m.sin_sg2[o2 - 1]);
-      out = (vf1 - vf0 + uf1 - uf) * ra;
-    } else {
-      const T vfm = (v[o - sj] - quarter * (ua[o - 1 - sj] + ua[o - sj]) *
-                                     (m.cos_sg3[o2 - 1 - sj2] + m.cos_sg1[o2 - sj2])) *
-                    m.dxc[o2 - sj2] * half * (m.sin_sg3[o2 - 1 - sj2] + m.sin_sg1[o2 - sj2]);
-      const T ufm = (u[o - 1] - quarter * (va[o - 1 - sj] + va[o - 1]) *
-                                    (m.cos_sg4[o2 - 1 - sj2] + m.cos_sg2[o2 - 1])) *
-                    m.dyc[o2 - 1] * half * (m.sin_sg4[o2 - 1 - sj2] + m.sin_sg2[o2 - 1]);
-      out = (vfm - vf + ufm - uf) * ra;
     }
-    divg[o] = out;
-  });
-}
+    const int jb = max(j0, d.jsc - 1), je = min(j0 + rows - 1, d.jec + 1);
+    if (jb > je) return;
+    struct Row {
+      T dp, pt, w, ut, vt, ua, va, uc, vc, u, v, ra;
+    };
+    struct Div {
+      T s1, s2, s3, s4, c1, c2, c3, c4, dxc, dyc, rac;
+    };
+    auto load = [&](int r) {
+      Row x;
+      x.dp = col.f(delp + o3, r);
+      x.pt = col.f(pt + o3, r);
+      x.w = col.f(w + o3, r);
+      x.ut = col.f(utc + o3, r);
+      x.vt = col.f(vtc + o3, r);
+      x.ua = col.f(ua + o3, r);
+      x.va = col.f(va + o3, r);
+      x.uc = col.f(uc + o3, r);
+      x.vc = col.f(vc + o3, r);
+      x.u = col.f(u + o3, r);
+      x.v = col.f(v + o3, r);
+      x.ra = col.m(m.rarea + o2, r);
+      return x;
+    };
+    auto load_div = [&](int r) {
+      Div y{};
+      y.s1 = col.m(m.sin_sg1 + o2, r);
+      y.c1 = col.m(m.cos_sg1 + o2, r);
+      y.s3 = col.m(m.sin_sg3 + o2, r);
+      y.c3 = col.m(m.cos_sg3 + o2, r);
+      if (divg) {
+        y.s2 = col.m(m.sin_sg2 + o2, r);
+        y.c2 = col.m(m.cos_sg2 + o2, r);
+        y.s4 = col.m(m.sin_sg4 + o2, r - 1);
+        y.c4 = col.m(m.cos_sg4 + o2, r - 1);
+        y.dxc = col.m(m.dxc + o2, r);
+        y.dyc = col.m(m.dyc + o2, r);
+        y.rac = col.m(m.rarea_c + o2, r);
+      }
+      return y;
+    };
+    const T half = T(0.5), quarter = T(0.25);
+    T dp1 = 0, pt1 = 0, w1 = 0, va1 = 0, vc1 = 0, ra1 = 0, u1 = 0;  // row r - 1
+    T gx = 0, gx1 = 0, gx2 = 0;                                     // its x flux differences
+    T fy = 0, fy1 = 0, fy2 = 0, kx = 0, vf1 = 0;  // its lower y fluxes, ua kev, vf
+    struct Both {
+      Row x;
+      Div y;
+    };
+    const Both first{load(jb - 1), load_div(jb - 1)};
+    strip_march(jb - 1, je + 1, first, [&](int r, const Both& cur, Both& nx) {
+      nx.x = load(r + 1);
+      nx.y = load_div(r + 1);
+      const Row& x = cur.x;
+      const Div& y = cur.y;
+      // y fluxes at interface r
+      const bool dn = x.vt > T(0);
+      const T hy1 = x.vt * (dn ? dp1 : x.dp);
+      const T hy = hy1 * (dn ? pt1 : x.pt), hy2 = hy1 * (dn ? w1 : x.w);
+      // the cells of row j = r - 1
+      const int j = r - 1;
+      const T dpc = dp1 + (gx1 + fy1 - hy1) * ra1;
+      const T ptv = (pt1 * dp1 + (gx + fy - hy) * ra1) / dpc;
+      const T wv = (w1 * dp1 + (gx2 + fy2 - hy2) * ra1) / dpc;
+      T vort = va1 > T(0) ? vc1 : x.vc;
+      if (j == d.js - 1 || j == d.je) {
+        if (va1 <= T(0)) vort = vort * col.m(m.sin_sg4 + o2, j) + x.u * col.m(m.cos_sg4 + o2, j);
+      } else if (j == d.js || j == d.je + 1) {
+        if (va1 > T(0)) vort = vort * col.m(m.sin_sg2 + o2, j) + u1 * col.m(m.cos_sg2 + o2, j);
+      }
+      col.store(delpc + o3, j, cell_i ? dpc : T(0), out && j >= jb);
+      col.store(ptc + o3, j, cell_i ? ptv : T(0), out && j >= jb);
+      col.store(wc + o3, j, wv, cell_i && j >= jb);
+      col.store(ke + o3, j, half * dt2 * (kx + va1 * vort), cell_i && j >= jb);
+      // x fluxes of row r
+      {
+        T xd = x.dp, xp = x.pt, xw = x.w;
+        if ((r == d.js - 1 || r == d.je + 1) && corner) {
+          const int rs = r < d.js ? r + 1 : r - 1;
+          xd = col.f(delp + o3, rs);
+          xp = col.f(pt + o3, rs);
+          xw = col.f(w + o3, rs);
+        }
+        const T ld = lane_up(xd, 1), lp = lane_up(xp, 1), lw = lane_up(xw, 1);
+        const bool rt = x.ut > T(0);
+        const T f1 = x.ut * (rt ? ld : xd);
+        const T f = f1 * (rt ? lp : xp), f2 = f1 * (rt ? lw : xw);
+        gx1 = f1 - lane_dn(f1, 1);
+        gx = f - lane_dn(f, 1);
+        gx2 = f2 - lane_dn(f2, 1);
+      }
+      // the x part of the kinetic energy of row r
+      {
+        const T ucp = lane_dn(x.uc, 1), vp = lane_dn(x.v, 1);
+        T kev = x.ua > T(0) ? x.uc : ucp;
+        if (kl) {
+          if (x.ua <= T(0)) kev = kev * y.s3 + vp * y.c3;
+        } else if (kr) {
+          if (x.ua > T(0)) kev = kev * y.s1 + x.v * y.c1;
+        }
+        kx = x.ua * kev;
+      }
+      if (divg) {
+        // divergence_corner (c_sw.py:172-289): next to a tile edge the flux
+        // along it leaves the other wind out, and at a tile corner one of the
+        // two vf is missing
+        const bool south = r == d.js || r == d.je + 1;
+        const T s3m = lane_up(y.s3, 1), c3m = lane_up(y.c3, 1), uam = lane_up(x.ua, 1);
+        const T uw = south ? x.u : x.u - quarter * (va1 + x.va) * (y.c4 + y.c2);
+        const T uf = uw * y.dyc * half * (y.s4 + y.s2);
+        const T vw = west ? x.v : x.v - quarter * (uam + x.ua) * (c3m + y.c1);
+        const T vf = vw * y.dxc * half * (s3m + y.s1);
+        const T uf1 = lane_up(uf, 1);
+        T sum = vf1 - vf;
+        if (south && west) sum = r == d.js ? -vf : vf1;
+        col.store(divg + o3, r, (sum + uf1 - uf) * y.rac,
+                  div_i && r >= jb && r >= d.jsc && r <= je);
+        vf1 = vf;
+      }
+      dp1 = x.dp;
+      pt1 = x.pt;
+      w1 = x.w;
+      va1 = x.va;
+      vc1 = x.vc;
+      ra1 = x.ra;
+      u1 = x.u;
+      fy = hy;
+      fy1 = hy1;
+      fy2 = hy2;
+    });
+  }
+};
 
-// transportdelp_update_vorticity_and_kineticenergy on [isc-1, iec+1]^2, with
-// initialize_delpc_ptc (zero) on the rest of the full domain.
+// circulation_cgrid + absolute_vorticity on [isc, iec+1]^2, update_y_velocity
+// (vc on [isc, iec] x [jsc, jec+1]) and update_x_velocity (uc on [isc, iec+1] x
+// [jsc, jec]); c and e are the winds of D2A2C, copied to uc and vc around those
+// boxes.  At row r the strip forms the vorticity and vc of row r and uc of row
+// r - 1.
 template <typename T>
-void launch_transport(hipStream_t s, const Dom& d, const Met<T>& m, T dt2, const T* delp,
-                      const T* pt, const T* w, const T* utc, const T* vtc, const T* fx,
-                      const T* fx1, const T* fx2, const T* ua, const T* va, const T* uc,
-                      const T* vc, const T* u, const T* v, T* delpc, T* ptc, T* wc, T* ke) {
-  const Box full{d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3};
-  launch_box(s, d, full, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    if (i < d.isc - 1 || i > d.iec + 1 || j < d.jsc - 1 || j > d.jec + 1) {
-      delpc[o] = T(0);
-      ptc[o] = T(0);
-      return;
-    }
-    const int64_t o2 = at2(d, i, j, t);
-    const int64_t sj = d.sj;
-    // y fluxes at j and j + 1
-    const T c0 = vtc[o], c1 = vtc[o + sj];
-    const int64_t up0 = c0 > T(0) ? o - sj : o;
-    const int64_t up1 = c1 > T(0) ? o : o + sj;
-    const T fy1_0 = c0 * delp[up0], fy1_1 = c1 * delp[up1];
-    const T fy_0 = fy1_0 * pt[up0], fy_1 = fy1_1 * pt[up1];
-    const T fy2_0 = fy1_0 * w[up0], fy2_1 = fy1_1 * w[up1];
-    const T ra = m.rarea[o2];
-    const T dp = delp[o];
-    const T dpc = dp + (fx1[o] - fx1[o + 1] + fy1_0 - fy1_1) * ra;
-    delpc[o] = dpc;
-    ptc[o] = (pt[o] * dp + (fx[o] - fx[o + 1] + fy_0 - fy_1) * ra) / dpc;
-    wc[o] = (w[o] * dp + (fx2[o] - fx2[o + 1] + fy2_0 - fy2_1) * ra) / dpc;
-    // kinetic energy and vorticity on the A grid
-    const T uav = ua[o], vav = va[o];
-    T kev = uav > T(0) ? uc[o] : uc[o + 1];
-    T vort = vav > T(0) ? vc[o] : vc[o + sj];
-    if (j == d.js - 1 || j == d.je) {
-      if (vav <= T(0)) vort = vort * m.sin_sg4[o2] + u[o + sj] * m.cos_sg4[o2];
-    } else if (j == d.js || j == d.je + 1) {
-      if (vav > T(0)) vort = vort * m.sin_sg2[o2] + u[o] * m.cos_sg2[o2];
-    }
-    if (i == d.ie || i == d.is - 1) {
-      if (uav <= T(0)) kev = kev * m.sin_sg3[o2] + v[o + 1] * m.cos_sg3[o2];
-    } else if (i == d.ie + 1 || i == d.is) {
-      if (uav > T(0)) kev = kev * m.sin_sg1[o2] + v[o] * m.cos_sg1[o2];
-    }
-    ke[o] = T(0.5) * dt2 * (uav * kev + vav * vort);
-  });
-}
+struct CswUpdate {
+  Met<T> m;
+  T dt2;
+  const T *c, *e, *ke, *u, *v;
+  T *uc, *vc;
 
-// circulation_cgrid + absolute_vorticity on [isc, iec+1]^2.
-template <typename T>
-void launch_vort(hipStream_t s, const Dom& d, const Met<T>& m, const T* uc, const T* vc,
-                 T* vort) {
-  const Box bx{d.isc, d.iec + 1, d.jsc, d.jec + 1};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const int64_t o2 = at2(d, i, j, t);
-    const T fx = m.dxc[o2] * uc[o];
-    const T fy = m.dyc[o2] * vc[o];
-    const T fx1 = m.dxc[o2 - d.sj2] * uc[o - d.sj];
-    const T fy1 = m.dyc[o2 - 1] * vc[o - 1];
-    const bool ej = j == d.js || j == d.je + 1;
-    T vc_;
-    if (i == d.is && ej) {
-      vc_ = fx1 - fx + fy;
-    } else if (i == d.ie + 1 && ej) {
-      vc_ = fx1 - fx - fy1;
-    } else {
-      vc_ = fx1 - fx - fy1 + fy;
-    }
-    vort[o] = m.fC[o2] + m.rarea_c[o2] * vc_;
-  });
-}
+  __device__ __forceinline__ void operator()(const Dom& d, int i0, int j0, int rows, int k,
+                                             int t) const {
+    const int lane = threadIdx.x, i = i0 - 1 + lane;
+    const StripColumn<T> col(d, i);
+    const int64_t o3 = (int64_t)t * d.st + (int64_t)k * d.sk, o2 = (int64_t)t * d.st2;
+    const bool uc_i = lane >= 1 && lane < 63 && i <= d.iec + 2, vc_i = uc_i && i <= d.iec + 1;
+    const bool uu = i >= d.isc && i <= d.iec + 1, vu = i >= d.isc && i <= d.iec;
+    const bool west = i == d.is || i == d.ie + 1;
+    struct Row {
+      T c, e, ke, u, v, dxc, dyc, f, rac, cv, sv, cu, su, rdx, rdy;
+    };
+    auto load = [&](int r) {
+      Row x;
+      x.c = col.f(c + o3, r);
+      x.e = col.f(e + o3, r);
+      x.ke = col.f(ke + o3, r);
+      x.u = col.f(u + o3, r);
+      x.v = col.f(v + o3, r);
+      x.dxc = col.m(m.dxc + o2, r);
+      x.dyc = col.m(m.dyc + o2, r);
+      x.f = col.m(m.fC + o2, r);
+      x.rac = col.m(m.rarea_c + o2, r);
+      x.cv = col.m(m.cosa_v + o2, r);
+      x.sv = col.m(m.sina_v + o2, r);
+      x.cu = col.m(m.cosa_u + o2, r);
+      x.su = col.m(m.sina_u + o2, r);
+      x.rdx = col.m(m.rdxc + o2, r);
+      x.rdy = col.m(m.rdyc + o2, r);
+      return x;
+    };
+    T fx1 = 0, ke1 = 0;                     // row r - 1
+    T c1 = 0, tmp1 = 0, vort1 = 0, g1 = 0;  // its uc and what updates it
+    strip_march(j0 - 1, j0 + rows, load(j0 - 1), [&](int r, const Row& x, Row& nx) {
+      nx = load(r + 1);
+      const T fx = x.dxc * x.c, fy = x.dyc * x.e;
+      const T fy1 = lane_up(fy, 1);
+      T cir = fx1 - fx - fy1 + fy;
+      if (r == d.js || r == d.je + 1) {
+        if (i == d.is)
+          cir = fx1 - fx + fy;
+        else if (i == d.ie + 1)
+          cir = fx1 - fx - fy1;
+      }
+      const T vort = x.f + x.rac * cir;
+      const T vortp = lane_dn(vort, 1), kem = lane_up(x.ke, 1);
+      const int j = r - 1;
+      const T uflux = tmp1 > T(0) ? vort1 : vort;
+      col.store(uc + o3, j, uu && j >= d.jsc && j <= d.jec ? c1 + tmp1 * uflux + g1 : c1,
+                uc_i && j >= j0 && j <= d.jec + 1);
+      T vcv = x.e;
+      if (r >= d.jsc && r <= d.jec + 1) {
+        const T tmp =
+            (r == d.js || r == d.je + 1) ? dt2 * x.u : dt2 * (x.u - vcv * x.cv) / x.sv;
+        const T flux = tmp > T(0) ? vort : vortp;
+        const T up = vcv - tmp * flux + x.rdy * (ke1 - x.ke);
+        vcv = vu ? up : vcv;
+      }
+      col.store(vc + o3, r, vcv, vc_i && r >= j0 && r < j0 + rows);
+      c1 = x.c;
+      tmp1 = west ? dt2 * x.v : dt2 * (x.v - x.c * x.cu) / x.su;
+      g1 = x.rdx * (kem - x.ke);
+      vort1 = vort;
+      fx1 = fx;
+      ke1 = x.ke;
+    });
+  }
+};
 
-// update_y_velocity (vc on [isc, iec] x [jsc, jec+1]) and update_x_velocity
-// (uc on [isc, iec+1] x [jsc, jec]) in one pass over [isc, iec+1] x [jsc, jec+1].
-template <typename T>
-void launch_update(hipStream_t s, const Dom& d, const Met<T>& m, T dt2, const T* vort,
-                   const T* ke, const T* u, const T* v, T* uc, T* vc) {
-  const Box bx{d.isc, d.iec + 1, d.jsc, d.jec + 1};
-  launch_box(s, d, bx, 0, d.nk, [=] __device__(int i, int j, int k, int t) {
-    const int64_t o = at3(d, i, j, k, t);
-    const int64_t o2 = at2(d, i, j, t);
-    if (i <= d.iec) {
-      const T vcv = vc[o];
-      T tmp = (j == d.js || j == d.je + 1) ? dt2 * u[o]
-                                            : dt2 * (u[o] - vcv * m.cosa_v[o2]) / m.sina_v[o2];
-      const T flux = tmp > T(0) ? vort[o] : vort[o + 1];
-      vc[o] = vcv - tmp * flux + m.rdyc[o2] * (ke[o - d.sj] - ke[o]);
-    }
-    if (j <= d.jec) {
-      const T ucv = uc[o];
-      T tmp = (i == d.is || i == d.ie + 1) ? dt2 * v[o]
-                                            : dt2 * (v[o] - ucv * m.cosa_u[o2]) / m.sina_u[o2];
-      const T flux = tmp > T(0) ? vort[o] : vort[o + d.sj];
-      uc[o] = ucv + tmp * flux + m.rdxc[o2] * (ke[o - 1] - ke[o]);
-    }
-  });
-}
+const int kUnitMult[4] = {1, 1, 1, 1};
 
 int check_csw_domain(const fv3_domain* dom, const char* who) {
   int rc = check_domain(dom, who);
@@ -471,38 +586,30 @@ int run_c_sw(const fv3_domain* dom, const fv3_metrics* g, int32_t nord, T dt2, T
               FV3_E_ARG, "%s: work_slab too small", who);
   const Met<T> m = to_met<T>(g);
   hipStream_t s = as_stream(stream);
-  T* utmp = work;
-  T* vtmp = work + work_slab;
-  T* fx = work + 2 * work_slab;
-  T* fx1 = work + 3 * work_slab;
-  T* fx2 = work + 4 * work_slab;
-  T* ke = work + 5 * work_slab;
-  T* vort = work + 6 * work_slab;
-  rc = run_d2a2c<T>(s, dom, m, 1, dt2, uc, vc, u, v, ua, va, ut, vt, utmp, vtmp, delp, pt, w,
-                    who);
-  if (rc) return rc;
-  Dom d = to_dom(dom);
-  launch_fluxx_div<T>(s, d, m, delp, pt, w, ut, fx, fx1, fx2, u, v, ua, va,
-                      nord > 0 ? divgd : nullptr);
-  FV3_HIP_CHECK_LAUNCH(who);
+  T* uc0 = work;
+  T* vc0 = work + work_slab;
+  T* ke = work + 2 * work_slab;
+  const Dom d = to_dom(dom);
   const Box edges{dom->isc - 3, dom->iec + 3, dom->jsc - 3, dom->jec + 3};
-  FillTable fy;
-  fy.n = 0;
+  FillTable fill;
+  fill.n = 0;
   FillFields<T> ff{};
   ff.f[0] = delp;
   ff.f[1] = pt;
   ff.f[2] = w;
-  for (int f = 0; f < 3; ++f) append_fill(&fy, dom, kFill2Y, f, f, kUnitMult, edges);
-  launch_fill(s, d, fy, ff);
+  for (int f = 0; f < 3; ++f) append_fill(&fill, dom, kFill2X, f, f, kUnitMult, edges);
+  for (int f = 0; f < 3; ++f) append_fill(&fill, dom, kFill2Y, f, f, kUnitMult, edges);
+  launch_fill(s, d, fill, ff);
   FV3_HIP_CHECK_LAUNCH(who);
-  launch_transport<T>(s, d, m, dt2, delp, pt, w, ut, vt, fx, fx1, fx2, ua, va, uc, vc, u, v,
-                      delpc, ptc, omga, ke);
-  FV3_HIP_CHECK_LAUNCH(who);
-  launch_vort<T>(s, d, m, uc, vc, vort);
-  FV3_HIP_CHECK_LAUNCH(who);
-  launch_update<T>(s, d, m, dt2, vort, ke, u, v, uc, vc);
-  FV3_HIP_CHECK_LAUNCH(who);
-  return FV3_OK;
+  rc = run_d2a2c<T>(s, dom, m, 1, dt2, uc0, vc0, u, v, ua, va, ut, vt, who);
+  if (rc) return rc;
+  const CswTransport<T> transport{m,  dt2, delp, pt, w,     ut,  vt, ua, va,
+                                  uc0, vc0, u,   v,  delpc, ptc, omga, ke,
+                                  nord > 0 ? divgd : nullptr};
+  rc = launch_strips(s, d, d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3, 62, 2, transport, who);
+  if (rc) return rc;
+  const CswUpdate<T> update{m, dt2, uc0, vc0, ke, u, v, uc, vc};
+  return launch_strips(s, d, d.isc - 1, d.iec + 2, d.jsc - 1, d.jec + 2, 62, 2, update, who);
 }
 
 }  // namespace
@@ -528,7 +635,7 @@ int32_t fv3_d2a2c_vect_f64(const fv3_domain* dom, const fv3_metrics* g, double* 
               FV3_E_ARG, "%s: work_slab too small", who);
   const Met<double> m = to_met<double>(g);
   return run_d2a2c<double>(as_stream(stream), dom, m, 0, 0.0, uc, vc, u, v, ua, va, utc, vtc,
-                           work, work + work_slab, nullptr, nullptr, nullptr, who);
+                           who);
 }
 
 int32_t fv3_c_sw_f64(const fv3_domain* dom, const fv3_metrics* g, int32_t nord, double dt2,

@@ -4,21 +4,21 @@
 
 namespace fv3 {
 
-// A segment marches its rows plus 6 halo rows.  Measured in the acoustic call
-// (FP64, two extra passes): a step takes 0.65 us plus 0.28 us per wave on a
+// Measured on the del-n march in the acoustic call (FP64, two extra passes, 6
+// rows beside a segment's own): a step takes 0.65 us plus 0.28 us per wave on a
 // SIMD up to three waves, about 0.75 us plus 0.37 us per wave above that, and a
 // launch adds about four steps; the segment count with the least time by these
 // figures is taken, of heights up to DN_TJ rows where there are more than
 // three waves (96 C48 tiles in FP32: one 49-row segment 266 us, two of 25 rows
 // 230 us).
-int deln_segment_rows(int nfj, int64_t planes) {
+int strip_segment_rows(int rows, int extra, int64_t planes) {
   int best = 0;
   double least = 0.0;
-  for (int nb = 1; nb <= nfj; ++nb) {
-    const int seg = (nfj + nb - 1) / nb;
-    const double w = (double)planes * ((nfj + seg - 1) / seg) / kSimdsPerGpu;
+  for (int nb = 1; nb <= rows; ++nb) {
+    const int seg = (rows + nb - 1) / nb;
+    const double w = (double)planes * ((rows + seg - 1) / seg) / kSimdsPerGpu;
     if (w > 3.0 && seg > FV3_DN_TJ) continue;
-    const double t = (w <= 3.0 ? 0.65 + 0.28 * w : 0.75 + 0.37 * w) * (seg + 6 + 4);
+    const double t = (w <= 3.0 ? 0.65 + 0.28 * w : 0.75 + 0.37 * w) * (seg + extra + 4);
     if (best == 0 || t < least) {
       best = seg;
       least = t;

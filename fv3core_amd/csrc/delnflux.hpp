@@ -304,9 +304,6 @@ __global__ void __launch_bounds__(DN_W * DN_NY)
     deln_strip<T, 0>(d, a, epi, dk, i0, j0, rows, q, u6, v6, ra);
 }
 
-// Rows per segment of a launch of `planes` strips of nfj interface rows.
-int deln_segment_rows(int nfj, int64_t planes);
-
 // Runs the passes on every level of the domain with epilogue epi; `bytes` is
 // the call's algorithmic traffic.
 template <typename T, typename EPI>
@@ -346,7 +343,7 @@ int deln_launch(const fv3_domain* dom, const int32_t* nord4, int use_damp, const
     a.wi = d.ie - d.is + 1 < 4 ? 1 : 2;
     a.wj = d.je - d.js + 1 < 4 ? 1 : 2;
   }
-  a.seg = deln_segment_rows(nfj, (int64_t)a.nbi * d.nk * d.ntiles);
+  a.seg = strip_segment_rows(nfj, 6, (int64_t)a.nbi * d.nk * d.ntiles);
   a.nbj = (nfj + a.seg - 1) / a.seg;
   const int64_t total = (int64_t)(a.nbi * a.nbj + a.wi * a.wj) * d.nk * d.ntiles;
   FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);

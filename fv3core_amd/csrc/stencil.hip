@@ -11,18 +11,14 @@ struct FillRow {
   int corner, di, dj, sdi, sdj;
 };
 
-// fill_corners_2cells_mult_x / 3cells_mult_x, statement order (corners.py:127-204)
+// fill_corners_2cells_mult_x, statement order (corners.py:127-163)
 const FillRow k2X[] = {{0, -1, -1, 0, 1},  {0, -2, -1, 1, 2},  {1, 1, -1, 0, 1},
                        {1, 2, -1, -1, 2},  {2, -1, 1, 0, -1},  {2, -2, 1, 1, -2},
                        {3, 1, 1, 0, -1},   {3, 2, 1, -1, -2}};
-const FillRow k3X[] = {{0, -3, -1, 2, 3}, {1, 3, -1, -2, 3}, {2, -3, 1, 2, -3},
-                       {3, 3, 1, -2, -3}};
-// fill_corners_2cells_mult_y / 3cells_mult_y (corners.py:207-300)
+// fill_corners_2cells_mult_y (corners.py:207-255)
 const FillRow k2Y[] = {{0, -1, -1, 1, 0},  {0, -1, -2, 2, 1},  {1, 1, -1, -1, 0},
                        {1, 1, -2, -2, 1},  {2, -1, 1, 1, 0},   {2, -1, 2, 2, -1},
                        {3, 1, 1, -1, 0},   {3, 1, 2, -2, -1}};
-const FillRow k3Y[] = {{0, -1, -3, 3, 2}, {1, 1, -3, -3, 2}, {2, -1, 3, 3, -2},
-                       {3, 1, 3, -3, -2}};
 
 bool add_rows(FillTable* tab, const fv3_domain* d, const FillRow* rows, int nrows, int dst_f,
               int src_f, const int mult[4], Box lim) {
@@ -54,12 +50,7 @@ bool add_rows(FillTable* tab, const fv3_domain* d, const FillRow* rows, int nrow
 
 bool append_fill(FillTable* tab, const fv3_domain* d, FillKind kind, int dst_f, int src_f,
                  const int mult[4], Box lim) {
-  const bool x = kind == kFill2X || kind == kFill3X;
-  const bool three = kind == kFill3X || kind == kFill3Y;
-  // the 3-cell variants run the 2-cell statements first (corners.py:166-204)
-  if (!add_rows(tab, d, x ? k2X : k2Y, 8, dst_f, src_f, mult, lim)) return false;
-  if (three && !add_rows(tab, d, x ? k3X : k3Y, 4, dst_f, src_f, mult, lim)) return false;
-  return true;
+  return add_rows(tab, d, kind == kFill2X ? k2X : k2Y, 8, dst_f, src_f, mult, lim);
 }
 
 }  // namespace fv3

@@ -81,9 +81,9 @@ struct FillTable {
   signed char mult[kMaxFill];
 };
 
-enum FillKind { kFill2X = 0, kFill3X = 1, kFill2Y = 2, kFill3Y = 3 };
+enum FillKind { kFill2X, kFill2Y };
 
-// Appends fill_corners_{2,3}cells_mult_{x,y}(q = field dst_f, q_corner =
+// Appends fill_corners_2cells_mult_{x,y}(q = field dst_f, q_corner =
 // field src_f) with multipliers (sw, se, nw, ne), limited to the box lim.
 // Returns false when the table is full.
 bool append_fill(FillTable* tab, const fv3_domain* d, FillKind kind, int dst_f, int src_f,

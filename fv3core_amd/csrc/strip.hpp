@@ -49,11 +49,11 @@ __device__ __forceinline__ T lane_up(T v, int d) {  // value of lane - d
 // 64-bit per-lane pointers.
 template <typename T>
 struct StripColumn {
-  int i, nj;
+  int i, ni, nj;
   uint32_t off0, offm, offp;  // byte offsets of columns i, i - 1, i + 1
   int64_t sj, sj2;
   __device__ __forceinline__ StripColumn(const Dom& d, int i_)
-      : i(i_), nj(d.nj), sj(d.sj), sj2(d.sj2) {
+      : i(i_), ni(d.ni), nj(d.nj), sj(d.sj), sj2(d.sj2) {
     auto at = [&](int c) { return (uint32_t)min(max(c, 0), d.ni - 1) * (uint32_t)sizeof(T); };
     off0 = at(i);
     offm = at(i - 1);
@@ -73,6 +73,82 @@ struct StripColumn {
   __device__ __forceinline__ T m(const T* __restrict__ p, int j, int di = 0) const {
     return get(p, row(j, sj2), di == 0 ? off0 : di < 0 ? offm : offp);
   }
+  // Stores v to row j of field p where keep holds (in a row and column of the
+  // storage), without a branch: a buffer store whose range is the row drops the
+  // offsets past it.  Loads and stores are counted by one counter in order, so
+  // behind a branch the next wait for loads would also wait for every store
+  // that might have been issued.
+  __device__ __forceinline__ void store(T* p, int j, T v, bool keep) const {
+    const uint64_t a = (uint64_t)(p + row(j, sj));
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a),
+                   hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((uint64_t)hi << 32 | lo), 0, ni * (int)sizeof(T), 0x00027000);
+    const uint32_t off = keep ? (uint32_t)i * (uint32_t)sizeof(T) : 0x80000000u;
+    if constexpr (sizeof(T) == 8) {
+      typedef uint32_t Pair __attribute__((ext_vector_type(2)));
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(Pair, v), rsrc, off, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, off, 0, 0);
+    }
+  }
 };
+
+// Runs step(row, cur, next) for rows r0 .. r1, where cur holds the row's loads
+// and step starts those of row + 1 into next.  Two rows per pass, with the
+// buffers in turn: copying next to cur would wait for the loads just started.
+template <typename ROW, typename F>
+__device__ __forceinline__ void strip_march(int r0, int r1, ROW a, F step) {
+  ROW b;
+  for (int r = r0;;) {
+    step(r, a, b);
+    if (++r > r1) return;
+    step(r, b, a);
+    if (++r > r1) return;
+  }
+}
+
+// How a launch is cut: columns from i0 in strips of `width` (the lanes left of
+// a wave's 64 once its neighbours are taken off), rows j0 .. j1 in segments.
+struct StripPlan {
+  int i0, j0, j1, width, nbi, nbj, seg;
+};
+
+constexpr int kStripWaves = 4;  // waves (strips) per workgroup
+
+// Runs body(d, i, j, rows, k, t) for every strip (first column i), segment
+// (first row j), level and tile, one wave each.
+template <typename F>
+__global__ void __launch_bounds__(64 * kStripWaves) strip_kernel(Dom d, StripPlan p, F body) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int per_plane = p.nbi * p.nbj, total = per_plane * d.nk * d.ntiles;
+  const int unit =
+      xcd_logical_block(blockIdx.x, (total + kStripWaves - 1) / kStripWaves) * kStripWaves + wave;
+  if (unit >= total) return;
+  const int plane = unit / per_plane, within = unit % per_plane;
+  const int j = p.j0 + within / p.nbi * p.seg;
+  body(d, p.i0 + within % p.nbi * p.width, j, min(p.seg, p.j1 + 1 - j), plane % d.nk, plane / d.nk);
+}
+
+// Rows per segment of a march of `extra` rows beside its own, over `rows` rows
+// of `planes` strips.
+int strip_segment_rows(int rows, int extra, int64_t planes);
+
+// Strips over columns [i0, i1] and rows [j0, j1] of every level and tile.
+template <typename F>
+inline int launch_strips(hipStream_t s, const Dom& d, int i0, int i1, int j0, int j1, int width,
+                         int extra, const F& body, const char* who) {
+  StripPlan p{i0, j0, j1, width, (i1 - i0 + width) / width, 1, j1 - j0 + 1};
+  p.seg = strip_segment_rows(p.seg, extra, (int64_t)p.nbi * d.nk * d.ntiles);
+  p.nbj = (j1 - j0 + p.seg) / p.seg;
+  const int64_t total = (int64_t)p.nbi * p.nbj * d.nk * d.ntiles;
+  FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);
+  const int64_t blocks = (total + kStripWaves - 1) / kStripWaves;
+  const int64_t launched = (blocks + kNumXcd - 1) / kNumXcd * kNumXcd;
+  hipLaunchKernelGGL((strip_kernel<F>), dim3((unsigned)launched), dim3(64, kStripWaves), 0, s, d,
+                     p, body);
+  FV3_HIP_CHECK_LAUNCH(who);
+  return FV3_OK;
+}
 
 }  // namespace fv3

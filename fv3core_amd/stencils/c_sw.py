@@ -2,7 +2,7 @@
 
 One call of ``fv3_c_sw`` runs the reference's sequence (d2a2c_vect,
 divergence_corner, geoadjust, corner fills, C-grid fluxes of delp/pt/w,
-kinetic energy, vorticity, C-grid momentum update) as ten launches.  The
+kinetic energy, vorticity, C-grid momentum update) as four launches.  The
 component owns ``delpc`` and ``ptc`` and returns them, as the reference
 does (c_sw.py:405-410, 659).  The Coriolis parameter ``fC`` comes from
 ``grid_data`` (the reference reads it from its global grid object).

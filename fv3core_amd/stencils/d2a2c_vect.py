@@ -1,7 +1,7 @@
 """DGrid2AGrid2CGridVectors (fv3core/stencils/d2a2c_vect.py:374-651) on the GPU.
 
-The reference's eleven stencils run as five launches of ``fv3_d2a2c_vect``
-(temporaries, x corner fills, uc/utc, y corner fills, vc/vtc).
+The reference's eleven stencils run as one launch of ``fv3_d2a2c_vect``, a
+march up the rows with the temporaries in registers.
 """
 from __future__ import annotations
 

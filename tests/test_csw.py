@@ -236,3 +236,35 @@ def test_gpu_c_sw_matches_oracle(cube_tiles, nord):
         outside[:, case.n + 6:] = False
         assert np.all(got["delpc"][outside] == 0) and np.all(got["ptc"][outside] == 0)
         assert got["delpc"][comp].min() > 0
+
+
+# The smallest domain, strips of the three marches that end with the domain and
+# one column past it (60 and 62 columns of n + 4 and n + 6), and batches whose
+# levels take segments of several heights.
+@pytest.mark.gpu
+@pytest.mark.parametrize("cube_tiles", [False, True])
+@pytest.mark.parametrize("n,nz,nord", [(5, 4, 0), (6, 4, 2), (56, 3, 2), (57, 4, 2), (58, 3, 0),
+                                       (59, 3, 2), (20, 90, 2)])
+def test_gpu_c_sw_strips_and_segments(n, nz, nord, cube_tiles):
+    from fv3core_amd.stencils.c_sw import CGridShallowWaterDynamics
+
+    case = Case(n, nz, cube_tiles, seed=31 + n)
+    u, v = _d2a2c_inputs(case)
+    names = ("delp", "pt", "u", "v", "w", "uc", "vc", "ua", "va", "ut", "vt", "divgd", "omga")
+    ins = dict(zip(names, [case.field(1000.0, 80.0), case.field(300.0, 15.0), u, v,
+                           case.field(0.0, 0.8)] + [case.field(0.0, 5.0) for _ in range(8)]))
+    dev = {k: case.dev(a) for k, a in ins.items()}
+    csw = CGridShallowWaterDynamics(case.factory, case.grid_data(), False, 0, nord)
+    delpc, ptc = csw(*(dev[k] for k in names), 37.5)
+    torch.cuda.synchronize()
+    t = case.tile
+    halo1 = (slice(t.isc - 1, t.iec + 2), slice(t.jsc - 1, t.jec + 2))
+    full = (slice(0, n + 6), slice(0, n + 6))
+    for ti in range(case.ntiles):
+        ref = ocs.c_sw(*(ins[k][ti][..., :nz] for k in names), 37.5, case.metric[ti], t, nord)
+        for name, got in list(dev.items()) + [("delpc", delpc), ("ptc", ptc)]:
+            box = halo1 if name in ("delpc", "ptc", "omga") else full
+            g, want = case.host(got)[ti][..., :nz][box], ref[name][box]
+            # differences of neighbouring values: the fields' own scale bounds
+            # what a rounding in any term can move
+            assert np.abs(g - want).max() <= 1e-13 * np.abs(want).max(), (ti, name)
