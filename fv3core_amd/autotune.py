@@ -44,7 +44,7 @@ KERNELS: Dict[str, Tuple[str, str, Tuple[str, str], List[Tuple[int, int]]]] = {
     "delnflux": ("delnflux.hip", "delnflux_kernel", ("FV3_DN_TJ", "FV3_DN_NY"),
                  [(17, 4), (25, 4), (33, 1), (33, 2), (33, 4), (33, 8), (49, 4)]),
     "a2b": ("a2b.hip", "a2b_interp_kernel", ("FV3_AB_TJ", "FV3_AB_NY"),
-            [(8, 4), (12, 4), (16, 4), (16, 8), (24, 8), (32, 8), (32, 16)]),
+            [(11, 4), (19, 4), (33, 1), (33, 2), (33, 4), (49, 4), (97, 4)]),
 }
 
 

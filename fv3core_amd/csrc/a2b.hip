@@ -1,17 +1,18 @@
 // AGrid2BGridFourthOrder (a2b_ord4): cell-centre values to cell corners.
 //
-// Reference: fv3core/stencils/a2b_ord4.py:1-695.  Four launches:
+// Reference: fv3core/stencils/a2b_ord4.py:1-695.  Three launches for up to four
+// fields on one grid:
 //   0 weights: the corner extrapolation weights from great-circle
 //             distances on the A/B-grid longitudes and latitudes (12 per
 //             tile, grid only);
 //   1 edges:  the four corner extrapolations and the tile-edge lines
-//             qout_x_edge / qout_y_edge, into qout and the edge temporary;
-//   2 means + interp: ppm_volume_mean_x on [isc, iec+1] x [jsc-2, jec+2]
-//             and ppm_volume_mean_y on [isc-2, iec+2] x [jsc, jec+1], each
-//             formed in LDS only where a block's corners read it, then
-//             a2b_interpolation on the corners off the tile-edge lines;
-//   3 copy:   the optional copy back into qin.
+//             qout_x_edge / qout_y_edge, into qout;
+//   2 interp: ppm_volume_mean_x and ppm_volume_mean_y, formed in registers as
+//             a strip marches up the rows, and a2b_interpolation on the corners
+//             off the tile-edge lines;
+// and the optional copy back into qin.
 #include "kernels.hpp"
+#include "strip.hpp"
 #include "tile_config.hpp"
 #include "timing.hpp"
 
@@ -170,179 +171,213 @@ __device__ __forceinline__ T volume_mean(const T (&q7)[7], const T (&dx7)[7], in
   return T(kB2) * (q[-2] + q[1]) + T(kB1) * (q[-1] + q[0]);
 }
 
-// Launches 2 and 3 fused: one workgroup owns a TI x TJ block of corners of
-// one level.  It stages q over the block plus a 3-cell halo in LDS, forms
-// the x volume means on the rows j-3 .. j+2 and the y volume means on the
-// columns i-3 .. i+2 of its corners there, then interpolates.  Lane x of
-// every wave owns LDS column x; wave y owns rows y, y+8, ...  (The metric
-// terms are read from global memory: staging them in LDS as well, once per
-// block over several levels, measured slower through the lower occupancy.)
-constexpr int AB_W = 64;           // LDS columns = TI + 6
-constexpr int AB_TI = AB_W - 6;    // corners per block in i
-constexpr int AB_TJ = FV3_AB_TJ;    // corners per block in j
-constexpr int AB_H = AB_TJ + 6;    // q rows: j0-3 .. j0+TJ+2
-constexpr int AB_NY = FV3_AB_NY;    // waves per block
-
-struct A2BArgs {
-  int ci0, cj0, nci, ncj;  // corner box (interpolation off the edge lines)
-  int nbi;                 // blocks along i
-  int k0;
-  int nrow;                // rows of the edge ratios (jsc-2 .. jec+2)
+// A quotient by a divisor that several share: the division's own steps
+// (reciprocal, Newton, residual correction, fix-up of zeros, infinities and
+// NaN), so the bits are those of a / b but where a quotient is near the ends of
+// the exponent range.
+template <typename T>
+struct Divisor {
+  T b;
+  __device__ __forceinline__ explicit Divisor(T v) : b(v) {}
+  __device__ __forceinline__ T quot(T a) const { return a / b; }
+};
+template <>
+struct Divisor<double> {
+  double b, y;
+  __device__ __forceinline__ explicit Divisor(double v) : b(v) {
+    y = __builtin_amdgcn_rcp(v);
+    y = fma(y, fma(-v, y, 1.0), y);
+    y = fma(y, fma(-v, y, 1.0), y);
+  }
+  __device__ __forceinline__ double quot(double a) const {
+    const double q = a * y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), y, q), b, a);
+  }
 };
 
+// The field and level of level kk of a set.
 template <typename T>
-__global__ void __launch_bounds__(AB_W * AB_NY)
-    a2b_interp_kernel(Dom d, Met<T> m, A2BArgs a, const T* __restrict__ qin,
-                      const T* __restrict__ edges, const T* __restrict__ xr,
-                      T* __restrict__ qout) {
-  __shared__ T sq[AB_H][AB_W];
-  __shared__ T sx[AB_H - 1][AB_W];  // x means on rows j0-3 .. j0+TJ+1
-  __shared__ T sy[AB_TJ][AB_W];     // y means on rows j0 .. j0+TJ-1
-  const int li = threadIdx.x, ty = threadIdx.y;
-  const int bi = blockIdx.x % a.nbi, bj = blockIdx.x / a.nbi;
-  const int k = a.k0 + (int)blockIdx.y, t = blockIdx.z;
-  const int i0 = a.ci0 + bi * AB_TI, j0 = a.cj0 + bj * AB_TJ;
-  const int i = i0 - 3 + li;  // absolute column of this lane
-  const int jb = j0 - 3;      // absolute row of LDS row 0
-  const bool col_ok = i >= 0 && i < d.ni;
-  const int64_t off3 = (int64_t)t * d.st + (int64_t)k * d.sk;
-  const int64_t off2 = (int64_t)t * d.st2;
-  for (int r = ty; r < AB_H; r += AB_NY) {
-    const int j = jb + r;
-    sq[r][li] = (col_ok && j >= 0 && j < d.nj) ? qin[off3 + (int64_t)j * d.sj + i] : T(0);
+__device__ __forceinline__ int a2b_field(const A2BFields<T>& f, int& k) {
+  int n = 0;
+  while (n + 1 < f.n && k >= f.nk[n]) {
+    k -= f.nk[n];
+    ++n;
   }
-  __syncthreads();
-  // x means where launch 2 formed them: i in [isc, iec+1], j in [jsc-2, jec+2].
-  // The lanes of one wave span the whole row, so the one-sided forms of the
-  // tile-edge interfaces diverge within it.  They share one instruction
-  // stream here: the outer form at is equals the one at ie+1 (the same two
-  // halves, added in the other order), and the inner form at is+1 or ie is
-  // the outer form of its neighbour combined with interior means, mirrored
-  // about the interface for the east side.  Each value keeps the operations
-  // of volume_mean, so the same bits; a wave runs 6 divisions a row instead
-  // of one set per form present in it.
-  if (li >= 3 && li < AB_W - 3 && i >= d.isc && i <= d.iec + 1) {
-    // form: 0 interior, 1 outer, 2 inner west, 3 inner east, in volume_mean's
-    // order of precedence; sh: the outer form's point, relative to i
-    int form = 0, sh = 0;
-    if (i == d.ie) {
-      form = 3;
-      sh = 1;
-    } else if (i == d.ie + 1) {
-      form = 1;
-    } else if (i == d.is + 1) {
-      form = 2;
-      sh = -1;
-    } else if (i == d.is) {
-      form = 1;
-    }
-    const bool west = form == 2;
-    for (int r = ty; r < AB_H - 1; r += AB_NY) {
-      const int j = jb + r;
-      if (j < d.jsc - 2 || j > d.jec + 2) continue;
-      const T* q = &sq[r][li];
-      T v = T(kB2) * (q[-2] + q[1]) + T(kB1) * (q[-1] + q[0]);
-      if (form != 0) {
-        // the outer form at is or ie+1 (qx_edge_west there) from its ratios
-        const T* gr = xr + ((int64_t)t * a.nrow + (j - (d.jsc - 2))) * 4;
-        const bool wside = i <= d.is + 1;
-        const T g_in = wside ? gr[0] : gr[2], g_ou = wside ? gr[1] : gr[3];
-        const T* qb = q + sh;
-        const T outer = T(0.5) * (((T(2) + g_in) * qb[0] - qb[1]) / (T(1) + g_in) +
-                                  ((T(2) + g_ou) * qb[-1] - qb[-2]) / (T(1) + g_ou));
-        if (form == 1) {
-          v = outer;
-        } else {
-          // qx_edge_west2 at is+1 (its left = outer) or qx_edge_east2 at ie
-          // (its right = outer), with q[k] -> q[-1-k] on the east side; its
-          // ratio dxa(is+1) / dxa(is) or dxa(ie-1) / dxa(ie) is the outer
-          // form's g_in or g_ou
-          auto qm = [&](int k) { return west ? q[k] : q[-1 - k]; };
-          const T g = west ? g_in : g_ou;
-          const T inner = T(kB2) * (qm(-1) + qm(2)) + T(kB1) * (qm(0) + qm(1));
-          v = (T(3) * (g * qm(-1) + qm(0)) - (g * outer + inner)) / (T(2) + T(2) * g);
-        }
-      }
-      sx[r][li] = v;
-    }
-  }
-  // y means where launch 2 formed them: i in [isc-2, iec+2], j in [jsc, jec+1]
-  if (li < AB_W - 1 && i >= d.isc - 2 && i <= d.iec + 2) {
-    for (int r = ty; r < AB_TJ; r += AB_NY) {
-      const int j = j0 + r;
-      if (j >= d.jsc && j <= d.jec + 1) {
-        // the row is uniform across the wave: only the rows on the tile-edge
-        // interfaces read the cell lengths and take the one-sided forms
-        T v = T(kB2) * (sq[r + 1][li] + sq[r + 4][li]) + T(kB1) * (sq[r + 2][li] + sq[r + 3][li]);
-        if (j == d.js || j == d.js + 1 || j == d.je || j == d.je + 1) {
-          const int64_t o2 = off2 + (int64_t)j * d.sj2 + i;
-          T q7[7], dy7[7];
-#pragma unroll
-          for (int n = 0; n < 7; ++n) {
-            q7[n] = sq[r + n][li];
-            dy7[n] = m.dya[o2 + (int64_t)(n - 3) * d.sj2];
-          }
-          v = volume_mean(q7, dy7, j, d.js, d.je);
-        }
-        sy[r][li] = v;
-      }
-    }
-  }
-  __syncthreads();
-  // a2b_interpolation on the block's corners (qx rows and qy columns -3 .. +2)
-  if (li < 3 || li >= 3 + AB_TI || i >= a.ci0 + a.nci) return;
-  const int64_t sj = d.sj;
-  for (int r = ty; r < AB_TJ; r += AB_NY) {
-    const int j = j0 + r;
-    if (j >= a.cj0 + a.ncj) break;
-    const int x = r + 3;  // sx row of j
-    const int64_t o = off3 + (int64_t)j * sj + i;
-    T qxx = T(kA2) * (sx[x - 2][li] + sx[x + 1][li]) + T(kA1) * (sx[x - 1][li] + sx[x][li]);
-    T qyy = T(kA2) * (sy[r][li - 2] + sy[r][li + 1]) + T(kA1) * (sy[r][li - 1] + sy[r][li]);
-    if (j == d.js + 1) {
-      const T up = T(kA2) * (sx[x - 1][li] + sx[x + 2][li]) + T(kA1) * (sx[x][li] + sx[x + 1][li]);
-      qxx = T(kCc1) * (sx[x - 1][li] + sx[x][li]) + T(kCc2) * (edges[o - sj] + up);
-    }
-    if (j == d.je) {
-      const T lo = T(kA2) * (sx[x - 3][li] + sx[x][li]) + T(kA1) * (sx[x - 2][li] + sx[x - 1][li]);
-      qxx = T(kCc1) * (sx[x - 1][li] + sx[x][li]) + T(kCc2) * (edges[o + sj] + lo);
-    }
-    if (i == d.is + 1) {
-      const T rr = T(kA2) * (sy[r][li - 1] + sy[r][li + 2]) + T(kA1) * (sy[r][li] + sy[r][li + 1]);
-      qyy = T(kCc1) * (sy[r][li - 1] + sy[r][li]) + T(kCc2) * (edges[o - 1] + rr);
-    }
-    if (i == d.ie) {
-      const T l = T(kA2) * (sy[r][li - 3] + sy[r][li]) + T(kA1) * (sy[r][li - 2] + sy[r][li - 1]);
-      qyy = T(kCc1) * (sy[r][li - 1] + sy[r][li]) + T(kCc2) * (edges[o + 1] + l);
-    }
-    qout[o] = T(0.5) * (qxx + qyy);
-  }
+  k += f.k0[n];
+  return n;
 }
+
+// Volume means and interpolation on the corners [ci0, ci1] x [cj0, cj1] off the
+// tile-edge lines: at row r of q a strip forms the x means of row r and the
+// corners of row r - 2, whose means and rows lie in windows of registers.
+//
+// What bounds it: memory, one row of q in and one of corners out per step of
+// about 130 instructions.  The LDS blocks of 58 x 16 corners it replaces read
+// six more rows per block and passed both means through LDS behind two
+// barriers.  KR rows are loaded at a time, one block ahead (two measured 2 %
+// faster than three and 15 % faster than four, which leave fewer waves).
+// Measured in the acoustic call with its five fields in two sets instead of
+// five, means, weights and edge lines together: six C96 tiles 374 -> 262 us, 96
+// C48 tiles mixed 1330 -> 960 us, six C128 tiles 650 -> 435 us, six C12 tiles
+// 93 -> 60 us.
+template <typename T>
+struct A2BInterp {
+  Met<T> m;
+  A2BFields<T> f;
+  const T* xr;
+  int nrow;  // rows of the edge ratios (jsc-2 .. jec+2)
+  int ci0, ci1, cj0, cj1;
+
+  static constexpr int KR = 2;  // rows loaded at a time
+  struct Rows {
+    T q[KR], e[KR], gi[KR], go[KR];
+  };
+
+  __device__ __forceinline__ void operator()(const Dom& d, int i0, int j0, int rows, int k,
+                                             int t) const {
+    const int n = a2b_field(f, k);
+    const int64_t o3 = (int64_t)t * d.st + (int64_t)k * d.sk, o2 = (int64_t)t * d.st2;
+    const T* const q = f.qin[n] + o3;
+    T* const qout = f.qout[n] + o3;
+    const int lane = threadIdx.x, i = i0 - 3 + lane;
+    const StripColumn<T> col(d, i);
+    const bool out = lane >= 3 && lane < 61 && i <= ci1;
+    // x means: form 0 interior, 1 outer (at is or ie + 1), 2 inner west, 3 inner
+    // east, in volume_mean's order of precedence.  The outer form at is equals
+    // the one at ie + 1 (the same two halves, added in the other order), and the
+    // inner form at is + 1 or ie is the outer form of its neighbour combined
+    // with interior means, mirrored for the east side; its ratio is the outer
+    // form's g_in or g_ou.
+    int form = 0;
+    if (i == d.ie)
+      form = 3;
+    else if (i == d.ie + 1)
+      form = 1;
+    else if (i == d.is + 1)
+      form = 2;
+    else if (i == d.is)
+      form = 1;
+    const bool west = form == 2;
+    // the corner on the tile-edge line beside i == is + 1 or ie, if any
+    const int ce = i == d.ie ? i + 1 : i == d.is + 1 ? i - 1 : min(max(i, ci0), ci1);
+    const StripColumn<T> edge(d, ce);
+    const T* const gr = xr + (int64_t)t * nrow * 4 + (i <= d.is + 1 ? 0 : 2);
+    auto load = [&](int r) {
+      Rows w;
+#pragma unroll
+      for (int u = 0; u < KR; ++u) {
+        w.q[u] = col.f(q, r + u);
+        w.e[u] = edge.f(qout, r + u - 2);
+        const T* g = gr + min(max(r + u - (d.jsc - 2), 0), nrow - 1) * 4;
+        w.gi[u] = g[0];
+        w.go[u] = g[1];
+      }
+      return w;
+    };
+    T q1 = 0, q2 = 0, q3 = 0, q4 = 0, q5 = 0;  // rows r - 1 .. r - 5
+    T s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0;  // their x means
+    const int last = j0 + rows - 1;
+    auto row = [&](int r, T q0, T ev, T g_in, T g_ou) {
+      const T qm1 = lane_up(q0, 1), qm2 = lane_up(qm1, 1), qm3 = lane_up(qm2, 1);
+      const T qp1 = lane_dn(q0, 1), qp2 = lane_dn(qp1, 1);
+      T s0 = T(kB2) * (qm2 + qp1) + T(kB1) * (qm1 + q0);
+      if (form != 0) {
+        // the outer form at point p = i, i - 1 (inner west) or i + 1 (inner east)
+        const T b0 = form == 1 ? q0 : west ? qm1 : qp1, b1 = form == 1 ? qp1 : west ? q0 : qp2;
+        const T a1 = form == 1 ? qm1 : west ? qm2 : q0, a2 = form == 1 ? qm2 : west ? qm3 : qm1;
+        const T outer = T(0.5) * (Divisor<T>(T(1) + g_in).quot((T(2) + g_in) * b0 - b1) +
+                                  Divisor<T>(T(1) + g_ou).quot((T(2) + g_ou) * a1 - a2));
+        if (form == 1) {
+          s0 = outer;
+        } else {
+          // qx_edge_west2, or qx_edge_east2 with q[k] -> q[-1-k]
+          const T g = west ? g_in : g_ou;
+          const T w0 = west ? q0 : qm1, w1 = west ? qp1 : qm2, wm = west ? qm1 : q0,
+                  w2 = west ? qp2 : qm3;
+          const T inner = T(kB2) * (wm + w2) + T(kB1) * (w0 + w1);
+          s0 = Divisor<T>(T(2) + T(2) * g).quot(T(3) * (g * wm + w0) - (g * outer + inner));
+        }
+      }
+      // corners of row j
+      const int j = r - 2;
+      T y = T(kB2) * (q4 + q1) + T(kB1) * (q3 + q2);
+      if (j == d.js || j == d.js + 1 || j == d.je || j == d.je + 1) {
+        const T q7[7] = {q5, q4, q3, q2, q1, q0, T(0)};
+        T dy7[7];
+#pragma unroll
+        for (int u = 0; u < 6; ++u) dy7[u] = col.m(m.dya + o2, j + u - 3);
+        dy7[6] = T(1);
+        y = volume_mean(q7, dy7, j, d.js, d.je);
+      }
+      const T ym1 = lane_up(y, 1), ym2 = lane_up(ym1, 1), ym3 = lane_up(ym2, 1);
+      const T yp1 = lane_dn(y, 1), yp2 = lane_dn(yp1, 1);
+      T qxx = T(kA2) * (s4 + s1) + T(kA1) * (s3 + s2);
+      if (j == d.js + 1) {
+        const T up = T(kA2) * (s3 + s0) + T(kA1) * (s2 + s1);
+        qxx = T(kCc1) * (s3 + s2) + T(kCc2) * (col.f(qout, j - 1) + up);
+      }
+      if (j == d.je) {
+        const T lo = T(kA2) * (s5 + s2) + T(kA1) * (s4 + s3);
+        qxx = T(kCc1) * (s3 + s2) + T(kCc2) * (col.f(qout, j + 1) + lo);
+      }
+      T qyy = T(kA2) * (ym2 + yp1) + T(kA1) * (ym1 + y);
+      if (i == d.is + 1) {
+        const T rr = T(kA2) * (ym1 + yp2) + T(kA1) * (y + yp1);
+        qyy = T(kCc1) * (ym1 + y) + T(kCc2) * (ev + rr);
+      }
+      if (i == d.ie) {
+        const T l = T(kA2) * (ym3 + y) + T(kA1) * (ym2 + ym1);
+        qyy = T(kCc1) * (ym1 + y) + T(kCc2) * (ev + l);
+      }
+      col.store(qout, j, T(0.5) * (qxx + qyy), out && j >= j0 && j <= last);
+      q5 = q4;
+      q4 = q3;
+      q3 = q2;
+      q2 = q1;
+      q1 = q0;
+      s5 = s4;
+      s4 = s3;
+      s3 = s2;
+      s2 = s1;
+      s1 = s0;
+    };
+    // rows r0 .. last + 2 in blocks of KR
+    const int r0 = j0 - 3, blocks = (rows + 5 + KR - 1) / KR;
+    strip_march(0, blocks - 1, load(r0), [&](int b, const Rows& w, Rows& nx) {
+      const int r = r0 + b * KR;
+      nx = load(r + KR);
+#pragma unroll
+      for (int u = 0; u < KR; ++u) row(r + u, w.q[u], w.e[u], w.gi[u], w.go[u]);
+    });
+  }
+};
 
 }  // namespace
 
 template <typename T>
-int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m, int k0, int nk,
-                    const T* qin, T* qout, T* qx, T* edges, int replace, T* qin_w,
-                    const char* who) {
+int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
+                    const A2BFields<T>& f, T* weights, const char* who) {
+  int nk = 0;
+  for (int n = 0; n < f.n; ++n) nk += f.nk[n];
   if (nk <= 0) return FV3_OK;
   Dom d = to_dom(dom);
   const bool w = has_edge(dom->i_start), e = has_edge(dom->i_end);
   const bool so = has_edge(dom->j_start), no = has_edge(dom->j_end);
   const int js2 = so ? d.jsc + 1 : d.jsc, je1 = no ? d.jec : d.jec + 1;
   const int is2 = w ? d.isc + 1 : d.isc, ie1 = e ? d.iec : d.iec + 1;
-  // 0: corner extrapolation weights, 12 per tile, into the head of the qx
-  // slab, and the x volume means' edge ratios after them (nothing else
-  // writes that slab during the call)
-  T* const cw = qx;
-  T* const xr = qx + 12 * (int64_t)d.ntiles;
+  // 0: corner extrapolation weights, 12 per tile, into the head of the slab,
+  // and the x volume means' edge ratios after them
+  T* const cw = weights;
+  T* const xr = weights + 12 * (int64_t)d.ntiles;
   const int nrow = d.jec - d.jsc + 5;
   hipLaunchKernelGGL((corner_weights_kernel<T>), dim3((unsigned)d.ntiles), dim3(64), 0, s, m, d,
                      cw, xr, nrow);
   FV3_HIP_CHECK_LAUNCH(who);
   // 1: corners and edge lines: only the perimeter of [isc, iec+1]^2 can hold them
   const Box bx{d.isc, d.iec + 1, d.jsc, d.jec + 1};
-  launch_perimeter(s, d, bx, k0, nk, [=] __device__(int i, int j, int k, int t) {
+  launch_perimeter(s, d, bx, 0, nk, [=] __device__(int i, int j, int k, int t) {
+    const int n = a2b_field(f, k);
+    const T* const qin = f.qin[n];
     const int64_t o = at3(d, i, j, k, t);
     const int64_t o2 = at2(d, i, j, t);
     T val;
@@ -379,47 +414,24 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m, int k
     } else {
       return;
     }
-    qout[o] = val;
-    edges[o] = val;
+    f.qout[n][o] = val;
   });
   FV3_HIP_CHECK_LAUNCH(who);
-  // 2 + 3: volume means and interpolation off the tile-edge lines
-  {
-    A2BArgs a;
-    a.ci0 = w ? d.isc + 1 : d.isc;
-    a.cj0 = so ? d.jsc + 1 : d.jsc;
-    a.nci = (e ? d.iec : d.iec + 1) - a.ci0 + 1;
-    a.ncj = (no ? d.jec : d.jec + 1) - a.cj0 + 1;
-    a.k0 = k0;
-    a.nrow = nrow;
-    if (a.nci > 0 && a.ncj > 0) {
-      a.nbi = (a.nci + AB_TI - 1) / AB_TI;
-      const int nbj = (a.ncj + AB_TJ - 1) / AB_TJ;
-      dim3 grid((unsigned)(a.nbi * nbj), (unsigned)nk, (unsigned)d.ntiles);
-      // q read, qout written (per corner-level)
-      TimedLaunch timed("a2b_interp_kernel", s,
-                        2.0 * sizeof(T) * (double)a.nci * a.ncj * nk * d.ntiles);
-      hipLaunchKernelGGL((a2b_interp_kernel<T>), grid, dim3(AB_W, AB_NY), 0, s, d, m, a, qin,
-                         edges, xr, qout);
-      FV3_HIP_CHECK_LAUNCH(who);
-    }
-  }
-  if (replace && qin_w) {
-    launch_box(s, d, bx, k0, nk, [=] __device__(int i, int j, int k, int t) {
-      const int64_t o = at3(d, i, j, k, t);
-      qin_w[o] = qout[o];
-    });
-    FV3_HIP_CHECK_LAUNCH(who);
-  }
-  return FV3_OK;
+  // 2: volume means and interpolation off the tile-edge lines
+  const A2BInterp<T> interp{m, f, xr, nrow, is2, ie1, js2, je1};
+  if (is2 > ie1 || js2 > je1) return FV3_OK;
+  Dom dk = d;
+  dk.nk = nk;
+  // q read, qout written (per corner-level)
+  TimedLaunch timed("a2b_interp_kernel", s,
+                    2.0 * sizeof(T) * (double)(ie1 - is2 + 1) * (je1 - js2 + 1) * nk * d.ntiles);
+  return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, 5, interp, who, FV3_AB_TJ);
 }
 
-template int launch_a2b_ord4<double>(hipStream_t, const fv3_domain*, const Met<double>&, int, int,
-                                     const double*, double*, double*, double*, int, double*,
-                                     const char*);
-template int launch_a2b_ord4<float>(hipStream_t, const fv3_domain*, const Met<float>&, int, int,
-                                    const float*, float*, float*, float*, int, float*,
-                                    const char*);
+template int launch_a2b_ord4<double>(hipStream_t, const fv3_domain*, const Met<double>&,
+                                     const A2BFields<double>&, double*, const char*);
+template int launch_a2b_ord4<float>(hipStream_t, const fv3_domain*, const Met<float>&,
+                                    const A2BFields<float>&, float*, const char*);
 
 int check_a2b_metrics(const fv3_metrics* g, const char* who) {
   FV3_REQUIRE(g && g->dxa && g->dya && g->agrid1 && g->agrid2 && g->bgrid1 && g->bgrid2 &&
@@ -445,6 +457,16 @@ extern "C" int32_t fv3_a2b_ord4_f64(const fv3_domain* dom, const fv3_metrics* g,
   FV3_REQUIRE(work_slab >= (int64_t)(dom->ntiles - 1) * dom->st + (int64_t)dom->nk * dom->sk,
               FV3_E_ARG, "%s: work_slab too small", who);
   const Met<double> m = to_met<double>(g);
-  return launch_a2b_ord4<double>(as_stream(stream), dom, m, 0, dom->nk, qin, qout, work,
-                                 work + 2 * work_slab, replace, qin, who);
+  const hipStream_t s = as_stream(stream);
+  rc = launch_a2b_ord4<double>(s, dom, m, A2BFields<double>{1, {qin}, {qout}, {0}, {dom->nk}}, work,
+                               who);
+  if (rc || !replace) return rc;
+  const Dom d = to_dom(dom);
+  launch_box(s, d, Box{d.isc, d.iec + 1, d.jsc, d.jec + 1}, 0, d.nk,
+             [=] __device__(int i, int j, int k, int t) {
+               const int64_t o = at3(d, i, j, k, t);
+               qin[o] = qout[o];
+             });
+  FV3_HIP_CHECK_LAUNCH(who);
+  return FV3_OK;
 }

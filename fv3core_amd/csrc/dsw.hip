@@ -906,7 +906,7 @@ void append_rotation_fill(FillTable* tab, const fv3_domain* dom, int kind, int f
 template <typename T>
 int run_div_high(hipStream_t s, const fv3_domain* dom, const Met<T>& m, const fv3_dsw_params* p,
                  const DswCols<T>& cols, T dt, const T* wk, T* divg, T* vc, T* uc, T* delpc,
-                 T* vort, T* ke, T* a2b_qx, T* a2b_edges, T* dg_last, const char* who) {
+                 T* vort, T* ke, T* a2b_qx, T* dg_last, const char* who) {
   const int k0 = p->div_k0;
   fv3_domain hd = *dom;
   hd.nk = dom->nk - k0;
@@ -1044,8 +1044,8 @@ int run_div_high(hipStream_t s, const fv3_domain* dom, const Met<T>& m, const fv
   // _vorticity_calc
   const T dddmp = (T)p->dddmp;
   if (!(dddmp < T(1e-5))) {
-    int rc = launch_a2b_ord4<T>(s, &hd, m, 0, hd.nk, wkh, vo, a2b_qx + ko, a2b_edges + ko, 0,
-                                nullptr, who);
+    const int rc =
+        launch_a2b_ord4<T>(s, &hd, m, A2BFields<T>{1, {wkh}, {vo}, {0}, {hd.nk}}, a2b_qx + ko, who);
     if (rc) return rc;
   }
   const T adt = fabs(dt), da_min_c = (T)p->da_min_c;
@@ -1154,7 +1154,7 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
   T *wgx = W[6], *wgy = W[7], *dw = W[8], *heat_s = W[9], *wk = W[10], *vort = W[11];
   T *ke = W[12], *delpn = W[13], *ptn = W[14], *qcn = W[15], *qy = W[17];
   T *us = W[4], *vs = W[5];  // the winds before their damping (gx, gy are free by then)
-  T *a2x = W[18], *a2e = W[20], *vort2 = W[21];  // W[19]: the last divergence pass
+  T *a2x = W[18], *vort2 = W[21];  // W[19]: the last divergence pass
   const T* area = m.area;
   const T* dxa = m.dxa;
   const T* dya = m.dya;
@@ -1232,7 +1232,7 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
     FV3_HIP_CHECK_LAUNCH(who);
   }
   rc = run_div_high<T>(s, dom, m, p, cols, dt, wk, st.divgd, st.vc, st.uc, st.delpc, vort, ke,
-                       a2x, a2e, W[19], who);
+                       a2x, W[19], who);
   if (rc) return rc;
   launch_absolute_vort<T>(s, d, m, wk, vort2);
   FV3_HIP_CHECK_LAUNCH(who);

@@ -558,21 +558,16 @@ int nh_p_grad(const fv3_domain* dom, const fv3_metrics* g, S* u, S* v, double* p
               FV3_E_ARG, "%s: work_slab too small", who);
   hipStream_t s = as_stream(stream);
   const Met<double> m = to_met<double>(g);
-  // slabs: B-grid pp, delp's B-grid values (wk1), the a2b scratch (corner
-  // weights, edges), B-grid pk3 and gz
+  // slabs: B-grid pp, delp's B-grid values (wk1), the a2b weights, B-grid pk3
+  // and gz
   double *ppb = work, *wk1 = work + work_slab, *qx = work + 2 * work_slab;
-  double *pk3b = work + 3 * work_slab, *edges = work + 4 * work_slab;
-  double* gzb = work + 5 * work_slab;
+  double *pk3b = work + 3 * work_slab, *gzb = work + 5 * work_slab;
   // a2b_k1 on pp and pk3 (levels 1..nz), a2b_kbuffer on gz (0..nz), into
   // the slabs; the u/v update below writes them back into pp, pk3 and gz
   // (the reference's replace), so no separate copies are launched
-  rc = launch_a2b_ord4<double>(s, dom, m, 1, nz, pp, ppb, qx, edges, 0, nullptr, who);
-  if (rc) return rc;
-  rc = launch_a2b_ord4<double>(s, dom, m, 1, nz, pk3, pk3b, qx, edges, 0, nullptr, who);
-  if (rc) return rc;
-  rc = launch_a2b_ord4<double>(s, dom, m, 0, nz + 1, gz, gzb, qx, edges, 0, nullptr, who);
-  if (rc) return rc;
-  rc = launch_a2b_ord4<double>(s, dom, m, 0, nz, delp, wk1, qx, edges, 0, nullptr, who);
+  const A2BFields<double> bf{
+      4, {pp, pk3, gz, delp}, {ppb, pk3b, gzb, wk1}, {1, 1, 0, 0}, {nz, nz, nz + 1, nz}};
+  rc = launch_a2b_ord4<double>(s, dom, m, bf, qx, who);
   if (rc) return rc;
   Dom d = to_dom(dom);
   // set_k0_and_calc_wk, calc_u and calc_v on [isc, iec+1]^2 in one pass:

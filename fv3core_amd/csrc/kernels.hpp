@@ -5,15 +5,24 @@
 
 namespace fv3 {
 
-// AGrid2BGridFourthOrder.__call__ (a2b_ord4.py:617-695) on levels
-// [k0, k0 + nk): qout on the corners [isc, iec+1]^2; qx (whose head holds
-// the 12 corner extrapolation weights per tile) and edges are scratch slabs
-// laid out like the fields.  With replace set, qin_w (the writable qin)
-// receives qout as well.
+// Up to four fields to interpolate at once, field n on levels
+// [k0[n], k0[n] + nk[n]).
+constexpr int kMaxA2B = 4;
 template <typename T>
-int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m, int k0, int nk,
-                    const T* qin, T* qout, T* qx, T* edges, int replace, T* qin_w,
-                    const char* who);
+struct A2BFields {
+  int n;
+  const T* qin[kMaxA2B];
+  T* qout[kMaxA2B];
+  int k0[kMaxA2B], nk[kMaxA2B];
+};
+
+// AGrid2BGridFourthOrder.__call__ (a2b_ord4.py:617-695) on the fields f: qout
+// on the corners [isc, iec+1]^2.  weights is a scratch slab laid out like the
+// fields (its head holds 12 corner extrapolation weights a tile and the edge
+// ratios).
+template <typename T>
+int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
+                    const A2BFields<T>& f, T* weights, const char* who);
 
 int check_a2b_metrics(const fv3_metrics* g, const char* who);
 

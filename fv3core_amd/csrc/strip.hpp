@@ -2,6 +2,8 @@
 // of columns and marches up its rows, neighbours across i by lane shifts.
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace fv3 {
@@ -114,16 +116,13 @@ struct StripPlan {
   int i0, j0, j1, width, nbi, nbj, seg;
 };
 
-constexpr int kStripWaves = 4;  // waves (strips) per workgroup
-
 // Runs body(d, i, j, rows, k, t) for every strip (first column i), segment
-// (first row j), level and tile, one wave each.
-template <typename F>
-__global__ void __launch_bounds__(64 * kStripWaves) strip_kernel(Dom d, StripPlan p, F body) {
+// (first row j), level and tile, one wave each, NW waves to a workgroup.
+template <int NW, typename F>
+__global__ void __launch_bounds__(64 * NW) strip_kernel(Dom d, StripPlan p, F body) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const int per_plane = p.nbi * p.nbj, total = per_plane * d.nk * d.ntiles;
-  const int unit =
-      xcd_logical_block(blockIdx.x, (total + kStripWaves - 1) / kStripWaves) * kStripWaves + wave;
+  const int unit = xcd_logical_block(blockIdx.x, (total + NW - 1) / NW) * NW + wave;
   if (unit >= total) return;
   const int plane = unit / per_plane, within = unit % per_plane;
   const int j = p.j0 + within / p.nbi * p.seg;
@@ -134,19 +133,20 @@ __global__ void __launch_bounds__(64 * kStripWaves) strip_kernel(Dom d, StripPla
 // of `planes` strips.
 int strip_segment_rows(int rows, int extra, int64_t planes);
 
-// Strips over columns [i0, i1] and rows [j0, j1] of every level and tile.
-template <typename F>
+// Strips over columns [i0, i1] and rows [j0, j1] of every level and tile, in
+// segments of at most `most` rows.
+template <int NW = 4, typename F>
 inline int launch_strips(hipStream_t s, const Dom& d, int i0, int i1, int j0, int j1, int width,
-                         int extra, const F& body, const char* who) {
+                         int extra, const F& body, const char* who, int most = 1 << 30) {
   StripPlan p{i0, j0, j1, width, (i1 - i0 + width) / width, 1, j1 - j0 + 1};
-  p.seg = strip_segment_rows(p.seg, extra, (int64_t)p.nbi * d.nk * d.ntiles);
+  p.seg = std::min(most, strip_segment_rows(p.seg, extra, (int64_t)p.nbi * d.nk * d.ntiles));
   p.nbj = (j1 - j0 + p.seg) / p.seg;
   const int64_t total = (int64_t)p.nbi * p.nbj * d.nk * d.ntiles;
   FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);
-  const int64_t blocks = (total + kStripWaves - 1) / kStripWaves;
+  const int64_t blocks = (total + NW - 1) / NW;
   const int64_t launched = (blocks + kNumXcd - 1) / kNumXcd * kNumXcd;
-  hipLaunchKernelGGL((strip_kernel<F>), dim3((unsigned)launched), dim3(64, kStripWaves), 0, s, d,
-                     p, body);
+  hipLaunchKernelGGL((strip_kernel<NW, F>), dim3((unsigned)launched), dim3(64, NW), 0, s, d, p,
+                     body);
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }

@@ -1,4 +1,4 @@
-// Workgroup shapes of the strip and LDS-tiled stencil kernels, as chosen by
+// Workgroup shapes of the strip stencil kernels, as chosen by
 // fv3core_amd/autotune.py on one MI355X (six C96 tiles x 79 levels, the
 // acoustic step).  A shape changes only how the work is split, never the
 // arithmetic, so every choice returns the same bits.  The tuner builds
@@ -15,10 +15,11 @@
 #define FV3_DN_NY 4
 #endif
 
-// a2b_interp_kernel: corner rows per block, waves per block
+// a2b_interp_kernel: most corner rows per strip segment, strips (waves) per
+// workgroup
 #ifndef FV3_AB_TJ
-#define FV3_AB_TJ 16
+#define FV3_AB_TJ 33
 #endif
 #ifndef FV3_AB_NY
-#define FV3_AB_NY 8
+#define FV3_AB_NY 4
 #endif

@@ -412,8 +412,8 @@ int32_t fv3_c_sw_f32(const fv3_domain* d, const fv3_metrics* g, int32_t nord, fl
 /*
  * AGrid2BGridFourthOrder.__call__ (fv3core/stencils/a2b_ord4.py:617-695):
  * qout <- qin interpolated from cell centres to the corners [isc, iec+1]^2
- * (and qin <- qout there when replace != 0).  work: 3 slabs (qx, qy, edge
- * values).  Needs dxa, dya, agrid1/2, bgrid1/2 and edge_w/e/s/n.
+ * (and qin <- qout there when replace != 0).  work: 3 slabs (the head of the
+ * first holds the corner weights).  Needs dxa, dya, agrid1/2, bgrid1/2 and edge_w/e/s/n.
  */
 int32_t fv3_a2b_ord4_f64(const fv3_domain* d, const fv3_metrics* g, int32_t replace, double* qin,
                          double* qout, double* work, int64_t work_slab, void* stream);

@@ -205,6 +205,33 @@ def test_gpu_a2b_ord4_matches_oracle(cube_tiles):
         assert_close(got[full], ref[full], 1e-12, near_zero=1e-300, what=f"tile {ti} qout")
 
 
+# Corner boxes of one column and more up to one and two strips of 58 columns,
+# row counts at the edges of a block of rows, segments of several heights.
+@pytest.mark.gpu
+@pytest.mark.parametrize("cube_tiles", [False, True])
+@pytest.mark.parametrize("n,nz", [(4, 3), (5, 3), (6, 4), (7, 3), (57, 3), (58, 3), (59, 3),
+                                  (60, 3), (24, 90)])
+def test_gpu_a2b_ord4_strips_and_segments(n, nz, cube_tiles):
+    from fv3core_amd.stencils.a2b_ord4 import AGrid2BGridFourthOrder
+
+    case = Case(n, nz, cube_tiles, seed=33 + n)
+    q, out0 = case.field(1.0, 3.0), case.field(0.0, 1.0)
+    tq, to = case.dev(q), case.dev(out0)
+    AGrid2BGridFourthOrder(case.factory, case.grid_data(), 0, replace=True)(tq, to)
+    torch.cuda.synchronize()
+    t = case.tile
+    corners = (slice(t.isc, t.iec + 2), slice(t.jsc, t.jec + 2))
+    for ti in range(case.ntiles):
+        ref = out0[ti][..., :nz].copy()
+        ods.a2b_ord4(q[ti][..., :nz].copy(), ref, case.metric[ti], t)
+        got, qin = case.host(to)[ti][..., :nz], case.host(tq)[ti][..., :nz]
+        # sums of a few field values: rounded on the field's scale
+        assert np.abs(got - ref).max() <= 1e-13 * np.abs(q[ti]).max(), ti
+        want = q[ti][..., :nz].copy()
+        want[corners] = got[corners]
+        assert np.array_equal(qin, want)
+
+
 def _dsw_config(nord=3, hord=6, dddmp=0.5):
     from fv3core_amd._config import DynamicalCoreConfig
 
