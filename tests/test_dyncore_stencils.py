@@ -208,6 +208,57 @@ def test_gpu_update_dz_c_and_d(cube_tiles):
         assert_close(ws2g[c], ws2r[c], 1e-10, near_zero=1e-10, what=f"tile {ti} ws (d)")
 
 
+# Interface counts of one level per wave, at the edges of a chunk of 80 and past
+# two of them, layers thin enough for the floor to run through whole columns,
+# column counts beside a workgroup's 64.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nz", [(6, 4), (6, 8), (8, 79), (7, 80), (6, 81), (5, 162)])
+def test_gpu_update_dz_level_chunks(n, nz):
+    from fv3core_amd.stencils.updatedzc import UpdateGeopotentialHeightOnCGrid
+    from fv3core_amd.stencils.updatedzd import UpdateHeightOnDGrid
+    from fv3core_amd.utils.grid import DampingCoefficients
+
+    case = Case(n, nz, True, seed=57)
+    grid = case.grid_data()
+    zh = [np.cumsum(case.rng.uniform(0.5, 4.0, case.shape)[..., ::-1], axis=2)[..., ::-1].copy()
+          for _ in range(case.ntiles)]
+    ut, vt = case.field(0.0, 2e7), case.field(0.0, 2e7)
+    zs = [np.full(case.shape[:2], 30.0) for _ in range(case.ntiles)]
+    ws = [np.zeros(case.shape[:2]) for _ in range(case.ntiles)]
+    dp0 = np.linspace(300.0, 900.0, nz + 1)
+    gz_d, ws_d = _dev(case, zh), _dev2(case, ws)
+    UpdateGeopotentialHeightOnCGrid(case.factory, grid.area)(
+        dp0, _dev2(case, zs), _dev(case, ut), _dev(case, vt), gz_d, ws_d, 18.75)
+    crx, cry = case.field(0.0, 0.15), case.field(0.0, 0.15)
+    xfx = [c * m["dy"][..., None] * 2e4 for c, m in zip(crx, case.metric)]
+    yfx = [c * m["dx"][..., None] * 2e4 for c, m in zip(cry, case.metric)]
+    col = {"damp_vt": np.full(nz + 1, 0.06), "nord_v": np.array([0, 0, 2] + [2] * (nz - 2))}
+    damp = DampingCoefficients(grid.del6_u, grid.del6_v, case.scalars["da_min"],
+                               case.scalars["da_min_c"])
+    udd = UpdateHeightOnDGrid(case.factory, damp, grid, 0, 6, dp0, col,
+                              [[0, 1], [1, 1], [2, 1], [3, 1]])
+    h_d, ws2_d = _dev(case, zh), _dev2(case, ws)
+    udd(_dev2(case, zs), h_d, _dev(case, crx), _dev(case, cry), _dev(case, xfx), _dev(case, yfx),
+        ws2_d, 37.5)
+    torch.cuda.synchronize()
+    t = case.tile
+    for ti in range(case.ntiles):
+        g = case.metric[ti]
+        gz, h = zh[ti].copy(), zh[ti].copy()
+        wsr, ws2r = np.zeros(case.shape[:2]), np.zeros(case.shape[:2])
+        odc.update_dz_c(dp0, zs[ti], g["area"], ut[ti], vt[ti], gz, wsr, 18.75, t)
+        odc.update_dz_d(zs[ti], h, crx[ti], cry[ti], xfx[ti], yfx[ti], ws2r, 37.5, g, t, 6,
+                        col["nord_v"], col["damp_vt"], dp0)
+        box = (slice(t.isc - 1, t.iec + 2), slice(t.jsc - 1, t.jec + 2))
+        c = (slice(t.isc, t.iec + 1), slice(t.jsc, t.jec + 1))
+        # a column's sums of up to nz values: nz roundings of the highest
+        for got, want, b in ((gz_d, gz, box), (h_d, h, c)):
+            scale = np.abs(want[b]).max()
+            assert np.abs(case.host(got)[ti][b] - want[b]).max() <= (nz + 32) * 2.0 ** -52 * scale
+        assert np.abs(ws_d.cpu().numpy()[ti][box] - wsr[box]).max() <= 1e-12 * np.abs(wsr).max()
+        assert np.abs(ws2_d.cpu().numpy()[ti][c] - ws2r[c]).max() <= 1e-10 * np.abs(ws2r).max()
+
+
 @pytest.mark.gpu
 def test_gpu_update_dz_mixed_inputs_equal_the_fp64_entry():
     """fv3_update_dz_c_mixed / fv3_update_dz_d_mixed take FP32 winds, Courant
