@@ -415,6 +415,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV
       g[u] = last ? 0.0 : dm[u] / dm1;
       p[u] = last ? (pa + 2.0 * pb) * 1.0 / 3.0
                   : (pa + 2.0 * (1.0 + g[u]) * pb + g[u] * pc) * 1.0 / 3.0;
+      // layers past the bottom hand up 0: their value times the bottom layer's
+      // gr = 0 is NaN where pe is infinite
+      if (k0 + u >= nz) p[u] = 0.0;
       pa = pb;
     }
   }

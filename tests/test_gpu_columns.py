@@ -199,6 +199,46 @@ def test_riem_solvers_level_counts(nz, n, monkeypatch):
         assert np.array_equal(a, was)
 
 
+# Layer counts with and without layers past the bottom in the last set of 5 or 8.
+@pytest.mark.parametrize("nz", [3, 5, 10, 12, 79, 81, 127])
+def test_riem_solver3_infinite_wind_in_the_lowest_layer(nz, monkeypatch):
+    """An infinite w in the lowest layer, under a layer hot enough for its
+    change of w to be infinite and not NaN: pe is -inf there, the pressure
+    limit p_fac takes over and the layer keeps a finite height, as in the oracle."""
+    from fv3core_amd import workloads
+
+    monkeypatch.setattr(workloads, "hybrid_coefficients", workloads.synthetic_hybrid)
+    r = riemann_inputs(5, nz, workload=1)
+    factory, gi = _factory(5, nz)
+    c = gi.isc
+    for j, wind in ((c, np.inf), (c + 1, -np.inf)):
+        r["w"][c + 1, j, nz - 1] = wind
+        r["pt"][c + 1, j, nz - 2] = 3e38
+    t = {k: to_storage(v) for k, v in r.items() if isinstance(v, np.ndarray) and v.ndim >= 2}
+    wsd = np.full(r["zs"].shape, 0.01)
+    ppe, pk3, pk, peln = (utils.zeros(gi.max_shape) for _ in range(4))
+    RiemannSolver3(factory, RiemannConfig(p_fac=0.05, a_imp=1.0, use_logp=False, beta=0.0))(
+        True, r["dt"], t["cappa"], r["ptop"], t["zs"], to_storage(wsd), t["delz"], t["q_con"],
+        t["delp"], t["pt"], t["zh"], t["pe"], ppe, pk3, pk, peln, t["w"])
+    torch.cuda.synchronize()
+    sl = (slice(gi.isc, gi.iec + 1), slice(gi.jsc, gi.jec + 1))
+    z = np.zeros(r["pe"].shape)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = ori.riem_solver3(True, r["dt"], r["cappa"][sl], r["ptop"], r["zs"][sl], wsd[sl],
+                               r["delz"][sl], r["q_con"][sl], r["delp"][sl], r["pt"][sl],
+                               r["zh"][sl], r["pe"][sl], z[sl], z[sl], z[sl], z[sl],
+                               r["w"][sl], 0.05)
+    assert np.isfinite(ref[7][1, 0, nz - 1]) and not np.isfinite(ref[7][1, 0, 0])
+    for name, got, want in zip(["zh", "pe", "ppe", "pk3", "pk", "peln", "w", "delz"],
+                               [t["zh"], t["pe"], ppe, pk3, pk, peln, t["w"], t["delz"]], ref):
+        g = to_np(got)[sl]
+        np.testing.assert_array_equal(np.isfinite(g), np.isfinite(want), err_msg=name)
+        if name in ("zh", "delz"):
+            fin = np.isfinite(want)
+            assert_close(np.where(fin, g, 0.0), np.where(fin, want, 0.0), 1e-11, near_zero=1e-12,
+                         what=name)
+
+
 def test_riem_solver_c_wide_offsets():
     """Storages whose levels lie more than 4 GiB apart: 64-bit offsets, the
     same results as on dense storages."""
