@@ -11,6 +11,7 @@
 //             a strip marches up the rows, and a2b_interpolation on the corners
 //             off the tile-edge lines;
 // and the optional copy back into qin.
+#include "divide.hpp"
 #include "kernels.hpp"
 #include "strip.hpp"
 #include "tile_config.hpp"
@@ -170,30 +171,6 @@ __device__ __forceinline__ T volume_mean(const T (&q7)[7], const T (&dx7)[7], in
   if (a == s) return qx_edge_west(q, dx);
   return T(kB2) * (q[-2] + q[1]) + T(kB1) * (q[-1] + q[0]);
 }
-
-// A quotient by a divisor that several share: the division's own steps
-// (reciprocal, Newton, residual correction, fix-up of zeros, infinities and
-// NaN), so the bits are those of a / b but where a quotient is near the ends of
-// the exponent range.
-template <typename T>
-struct Divisor {
-  T b;
-  __device__ __forceinline__ explicit Divisor(T v) : b(v) {}
-  __device__ __forceinline__ T quot(T a) const { return a / b; }
-};
-template <>
-struct Divisor<double> {
-  double b, y;
-  __device__ __forceinline__ explicit Divisor(double v) : b(v) {
-    y = __builtin_amdgcn_rcp(v);
-    y = fma(y, fma(-v, y, 1.0), y);
-    y = fma(y, fma(-v, y, 1.0), y);
-  }
-  __device__ __forceinline__ double quot(double a) const {
-    const double q = a * y;
-    return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), y, q), b, a);
-  }
-};
 
 // The field and level of level kk of a set.
 template <typename T>

@@ -2,6 +2,7 @@
 // (fv3core/stencils/remap_profile.py:119-638, map_single.py:12-173): the kernel,
 // its launcher and the C entry points.
 #include "common.hpp"
+#include "divide.hpp"
 #include "remap_profile.hpp"
 #include "timing.hpp"
 
@@ -11,22 +12,6 @@ namespace fv3 {
 
 // Layers of the tallest column that map_layers_kernel takes.
 constexpr int kMapMaxLayers = 128;
-// Two quotients by one divisor: the division's own steps (reciprocal, Newton,
-// residual correction, fix-up of zeros, infinities and NaN) with the reciprocal
-// shared, so the bits are those of a / b but where a quotient is near the ends
-// of the exponent range.
-__device__ __forceinline__ void quot2(double a0, double a1, double b, double& q0, double& q1) {
-  double y = __builtin_amdgcn_rcp(b);
-  y = fma(y, fma(-b, y, 1.0), y);
-  y = fma(y, fma(-b, y, 1.0), y);
-  const double r0 = a0 * y, r1 = a1 * y;
-  q0 = __builtin_amdgcn_div_fixup(fma(fma(-b, r0, a0), y, r0), b, a0);
-  q1 = __builtin_amdgcn_div_fixup(fma(fma(-b, r1, a1), y, r1), b, a1);
-}
-__device__ __forceinline__ void quot2(float a0, float a1, float b, float& q0, float& q1) {
-  q0 = a0 / b;
-  q1 = a1 / b;
-}
 
 // The same remap with a column's layers spread over a workgroup.
 //
@@ -177,7 +162,9 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int u = 0; u < LV; ++u) {
         const T bet = s[u] - gam;
-        quot2(r[u] - ev, g[u], bet, ev, gam);
+        const Divisor<T> by(bet);
+        ev = by.quot(r[u] - ev);
+        gam = by.quot(g[u]);
         r[u] = ev;
         g[u] = gam;
       }

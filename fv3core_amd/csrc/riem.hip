@@ -29,6 +29,7 @@
 // independent parts.  64 columns by 10 levels (a whole wave per set, one
 // workgroup per CU) measured 342 us on six C96 tiles.
 #include "common.hpp"
+#include "divide.hpp"
 #include "timing.hpp"
 
 namespace fv3 {
@@ -39,24 +40,6 @@ constexpr double kCpAir = 1004.6;
 constexpr int RC = 32;      // columns per workgroup (half a wave)
 
 __device__ __forceinline__ double gm_of(double cp3) { return 1.0 / (1.0 - cp3); }
-
-// A refined reciprocal and the quotients by it: the Newton steps and the
-// final residual correction (Markstein) of the compiler's own division, so a
-// quotient has the bits of a / b wherever neither operand nor quotient is
-// near the ends of the exponent range (here: ratios of layer masses and
-// pressures).  Chains that divide twice by one value share the reciprocal.
-struct Recip {
-  double b, y;
-  __device__ __forceinline__ explicit Recip(double v) : b(v) {
-    const double y0 = __builtin_amdgcn_rcp(v);
-    const double y1 = fma(y0, fma(-v, y0, 1.0), y0);
-    y = fma(y1, fma(-v, y1, 1.0), y1);
-  }
-  __device__ __forceinline__ double quot(double a) const {
-    const double q = a * y;
-    return fma(fma(-b, q, a), y, q);
-  }
-};
 
 // The low (hi = false) or high half-wave's value in both halves.
 __device__ __forceinline__ double half_bcast(double v, bool hi) {
@@ -256,7 +239,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV
         const double gr = g[u], dd = p[u];
         g[u] = gk;
         p[u] = pk;
-        const Recip r(2.0 * (1.0 + gr) - gk);  // gr = 0 in the bottom layer
+        const Divisor<double> r(2.0 * (1.0 + gr) - gk);  // gr = 0 in the bottom layer
         pk = r.quot(dd - pk);
         gk = r.quot(gr);  // the next layer's gam = gr_k / bet_k
         if (k0 + u == nz - 1) bot[col] = pk;
@@ -323,7 +306,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV
 #pragma unroll
     for (int u = 0; u < LV; ++u) {
       const double an = u + 1 < LV && k0 + u != nz - 1 ? g[u + 1 < LV ? u + 1 : u] : ab;
-      const Recip r(bet);
+      const Divisor<double> r(bet);
       const double gam = r.quot(g[u]);
       bet = dm[u] - (g[u] + an + g[u] * gam);
       wp = (p[u] - g[u] * wp) / bet;

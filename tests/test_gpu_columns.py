@@ -239,6 +239,43 @@ def test_riem_solver3_infinite_wind_in_the_lowest_layer(nz, monkeypatch):
                          what=name)
 
 
+# 10^e m: where the factor of w's lowest layer overflows while the terms it sums
+# and every output stay finite.
+@pytest.mark.parametrize("nz,e", [(6, -299.05), (12, -299.45), (41, -300.15), (79, -300.55),
+                                  (127, -300.82)])
+def test_riem_solver3_overflowing_divisor(nz, e, monkeypatch):
+    """A quotient by an infinite divisor is 0, as IEEE division has it: three
+    layers so thin that the lowest one's divisor overflows leave a finite
+    column, as in the oracle."""
+    from fv3core_amd import workloads
+
+    monkeypatch.setattr(workloads, "hybrid_coefficients", workloads.synthetic_hybrid)
+    r = riemann_inputs(5, nz, workload=1)
+    factory, gi = _factory(5, nz)
+    sl = (slice(gi.isc, gi.iec + 1), slice(gi.jsc, gi.jec + 1))
+    for l, height in enumerate((2.0, 3.0, 4.0)):
+        r["zh"][..., nz - 1 - l] = height * 10.0 ** e
+        r["pt"][..., nz - 1 - l] = 0.02 * (r["zh"][..., nz - 1 - l] - r["zh"][..., nz - l])
+    t = {k: to_storage(v) for k, v in r.items() if isinstance(v, np.ndarray) and v.ndim >= 2}
+    wsd = np.full(r["zs"].shape, 0.01)
+    ppe, pk3, pk, peln = (utils.zeros(gi.max_shape) for _ in range(4))
+    RiemannSolver3(factory, RiemannConfig(p_fac=0.05, a_imp=1.0, use_logp=False, beta=0.0))(
+        True, r["dt"], t["cappa"], r["ptop"], t["zs"], to_storage(wsd), t["delz"], t["q_con"],
+        t["delp"], t["pt"], t["zh"], t["pe"], ppe, pk3, pk, peln, t["w"])
+    torch.cuda.synchronize()
+    z = np.zeros(r["pe"].shape)
+    with np.errstate(over="ignore"):
+        ref = ori.riem_solver3(True, r["dt"], r["cappa"][sl], r["ptop"], r["zs"][sl], wsd[sl],
+                               r["delz"][sl], r["q_con"][sl], r["delp"][sl], r["pt"][sl],
+                               r["zh"][sl], r["pe"][sl], z[sl], z[sl], z[sl], z[sl],
+                               r["w"][sl], 0.05)
+    for name, got, want in zip(["zh", "pe", "ppe", "pk3", "pk", "peln", "w", "delz"],
+                               [t["zh"], t["pe"], ppe, pk3, pk, peln, t["w"], t["delz"]], ref):
+        g = to_np(got)[sl]
+        assert np.isfinite(want).all() and np.isfinite(g).all(), name
+        assert_close(g, want, 1e-9, what=name, scale_floor=1.0)
+
+
 def test_riem_solver_c_wide_offsets():
     """Storages whose levels lie more than 4 GiB apart: 64-bit offsets, the
     same results as on dense storages."""
