@@ -652,11 +652,11 @@ template <typename T>
 struct VortDampEpilogue {
   const T *us, *vs, *vort, *delp, *heat_s;
   const T *rdx, *rdy, *rsin2, *cosa_s;
-  const T *kef, *damp_vt;
+  const T *kef, *damp_vt, *damp_w;  // damp_w: nullptr when heat_diss does not run
   T *u, *v, *heat_total;
   int d_con_on;
   T kefk;
-  bool heat, damp;
+  bool heat, damp, diss;
   int64_t sj;
 
   struct In {
@@ -666,6 +666,7 @@ struct VortDampEpilogue {
     kefk = kef[k];
     heat = kefk > T(kDconThreshold);
     damp = damp_vt[k] > T(1e-5);
+    diss = damp_w && damp_w[k] > T(1e-5);  // heat_s holds this level's dissipation
     us += off3;
     vs += off3;
     vort += off3;
@@ -686,7 +687,7 @@ struct VortDampEpilogue {
     n.u0 = c.f(us, j);
     n.v0 = c.f(vs, j);
     if (d_con_on) {
-      n.hs = c.f(heat_s, j);
+      n.hs = diss ? c.f(heat_s, j) : T(0);
       n.ht = c.f(heat_total, j);
       if (heat) {
         n.u1 = c.f(us, j + 1);
@@ -754,7 +755,7 @@ void launch_vorticity_adjust(hipStream_t s, const Dom& d, const Met<T>& m, int n
     T wn = w[o];
     if (nonhydro) wn = wn * delp[o] + (wgx[o] - wgx[o + 1] + wgy[o] - wgy[o + d.sj]) * ra;
     wn = wn / dpn;
-    if (damp_w[k] > T(1e-5)) wn = wn + dw[o];
+    if (nonhydro && damp_w[k] > T(1e-5)) wn = wn + dw[o];
     w[o] = wn;
     q_con[o] = qcn[o] / dpn;
     delp[o] = dpn;
@@ -1253,6 +1254,7 @@ int run_d_sw(const fv3_domain* dom, const fv3_metrics* g, const fv3_dsw_params* 
     epi.cosa_s = m.cosa_s;
     epi.kef = cols.d_con_col;
     epi.damp_vt = cols.damp_vt;
+    epi.damp_w = nonhydro ? cols.damp_w : nullptr;
     epi.u = st.u;
     epi.v = st.v;
     epi.heat_total = st.heat_source;

@@ -284,5 +284,54 @@ def test_gpu_d_sw_matches_oracle(cube_tiles, nord, hord, dddmp):
                          what=f"tile {ti} {name}")
 
 
+def _run_d_sw(case, st, nord, hord, dddmp, hydrostatic=False, dt=37.5):
+    """The device fields after one D-grid step from st, its workspace full of NaN
+    before the call, and the oracle's result of each tile."""
+    from fv3core_amd._config import DynamicalCoreConfig
+    from fv3core_amd.stencils.d_sw import DGridShallowWaterLagrangianDynamics, get_column_namelist
+    from fv3core_amd.utils.grid import DampingCoefficients
+
+    config = DynamicalCoreConfig(nord=nord, hord_dp=hord, hord_tm=hord, hord_mt=hord,
+                                 hord_vt=hord, dddmp=dddmp,
+                                 hydrostatic=hydrostatic).d_grid_shallow_water
+    grid = case.grid_data()
+    damp = DampingCoefficients(grid.del6_u, grid.del6_v, case.scalars["da_min"],
+                               case.scalars["da_min_c"])
+    col = get_column_namelist(config, case.nz)
+    dsw = DGridShallowWaterLagrangianDynamics(case.factory, grid, damp, col, False, False, config)
+    dev = {k: case.dev(v) for k, v in st.items()}
+    dsw._work.get(dev["delp"], case.nz + 1)[0].fill_(float("nan"))
+    dsw(*(dev[k] for k in ("delpc", "delp", "ptc", "pt", "u", "v", "w", "uc", "vc", "ua", "va",
+                           "divgd", "mfx", "mfy", "cx", "cy", "crx", "cry", "xfx", "yfx", "q_con",
+                           "zh", "heat_source", "diss_est")), dt)
+    torch.cuda.synchronize()
+    cfg = dict(hord_dp=hord, hord_tm=hord, hord_mt=hord, hord_vt=hord, dddmp=dddmp, d4_bg=0.15,
+               nord=nord, d_con=1.0, do_f3d=False, hydrostatic=hydrostatic, do_skeb=False)
+    refs = []
+    for ti in range(case.ntiles):
+        g = case.metric[ti]
+        damp_d = dict(del6_u=g["del6_u"], del6_v=g["del6_v"], da_min=case.scalars["da_min"],
+                      da_min_c=case.scalars["da_min_c"])
+        stt = {k: v[ti][..., :case.nz] for k, v in st.items()}
+        refs.append(ods.d_sw(stt, dt, g, case.tile, cfg, col, damp_d))
+    return dev, refs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cube_tiles", [False, True])
+def test_gpu_d_sw_hydrostatic(cube_tiles):
+    """Without the nonhydrostatic terms the dissipation of w neither enters w nor
+    the heat source."""
+    case = Case(12, 5, cube_tiles, seed=47)
+    dev, refs = _run_d_sw(case, dsw_state(case), 3, 6, 0.5, hydrostatic=True)
+    full = (slice(0, case.n + 6), slice(0, case.n + 6))
+    for ti, ref in enumerate(refs):
+        for name in _STATE_OUT:
+            got = case.host(dev[name])[ti][..., :case.nz]
+            assert np.isfinite(got[full]).all(), name
+            assert_close(got[full], ref[name][full], 1e-11, near_zero=1e-300,
+                         what=f"tile {ti} {name}")
+
+
 _STATE_OUT = ("delp", "pt", "u", "v", "w", "q_con", "uc", "vc", "divgd", "delpc", "ptc", "mfx",
               "mfy", "cx", "cy", "crx", "cry", "xfx", "yfx", "heat_source", "diss_est")
