@@ -992,6 +992,10 @@ int fvtp2d_corner_fill_f32(const fv3_domain* dom, int hord, float* q, float* qy_
 
 extern "C" {
 
+int32_t fv3_plan_fvtp2d_rows(int32_t rows, int64_t planes, int32_t fp32) {
+  return fv3::segment_rows(rows, planes, fp32 != 0);
+}
+
 int32_t fv3_fvtp2d_f64(const fv3_domain* d, int32_t hord, const double* q_x, const double* q_y,
                        const double* crx, const double* cry, const double* x_area_flux,
                        const double* y_area_flux, const double* x_mass_flux,

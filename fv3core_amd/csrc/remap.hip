@@ -6,6 +6,7 @@
 #include "remap_profile.hpp"
 #include "timing.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace fv3 {
@@ -315,6 +316,46 @@ static int map_layers_launch(const Dom& d, const RemapArgs& a, T* q1, const T* p
   return FV3_OK;
 }
 
+// The forms of the remap, which give the same bits: one thread per column in
+// four sweeps or with the limiter fused into the walk, and layers spread over a
+// workgroup (up to kMapMaxLayers).
+enum MapForm { kMapSweeps = 0, kMapFused = 1, kMapLayers = 2 };
+
+// The form with the least time on `waves` waves of columns (64 each).  Sets of 5
+// layers and 16 columns up to 80 layers (10 layers: 259 us, 8 layers by 8
+// columns: 287 us, 5 by 32: 245 us, against 178 us on six C128 tiles) take
+// 0.030 us per wave of columns and 20 layers, 8 by 8 above them 0.272 us per
+// wave, where 16 columns leave one workgroup to a CU (127 layers on six C96
+// tiles: 322 against 254 us).  One thread per column takes 2.3 us a layer at its
+// latency (less in launches of a few workgroups) and more once memory bounds it,
+// so few layers on many columns are its: 10 layers on six C128 tiles 34 against
+// 58 us, 81 layers 309 against 435 us.  Its fused form moves fewer bytes over a
+// longer dependent chain: it wins where two waves a SIMD cover the chain, or
+// where the nine column arrays of the sweeps (from 280 MB) do not fit the last-level
+// cache (137 layers, six C128 tiles: 531 against 597 us; 96 C48 tiles 1204
+// against 1698 us).  In FP32 the lines lie where its own times put them.
+static MapForm map_form(int km, int64_t waves, bool fp32) {
+  const double w = (double)waves;
+  const bool fused = waves >= 2 * kSimdsPerGpu ||
+                     9.0 * 64.0 * w * km * (fp32 ? 4 : 8) >= 280e6;
+  const MapForm column = fused ? kMapFused : kMapSweeps;
+  if (km > kMapMaxLayers) return column;
+  double layers, busy;
+  if (km <= 80) {
+    const double n = (km + 19) / 20;  // waves of a workgroup
+    layers = fp32 ? std::max(14.4, 11.0 + 0.0175 * n * w) : std::max(15.0, 12.0 + 0.030 * n * w);
+  } else {
+    layers = fp32 ? 18.0 + 0.134 * w : 20.0 + 0.272 * w;
+  }
+  // up to 32 layers a column's arrays stay in the caches
+  if (km <= 32)
+    busy = fp32 ? 0.25 + 0.00108 * w : 0.21 + 0.00185 * w;
+  else
+    busy = fp32 ? 0.35 + 0.0013 * w : 0.7 + 0.0021 * w;
+  const double lone = fp32 ? std::min(1.75, 1.35 + 0.008 * w) : std::min(2.3, 1.5 + 0.01 * w);
+  return 3.0 + km * std::max(lone, busy) < layers ? column : kMapLayers;
+}
+
 template <typename T>
 static int map_single_launch(const fv3_domain* dom, int kord, int iv, int i1, int i2, int j1,
                              int j2, T* q1, const T* pe1, const T* pe2, const T* qs, double qmin,
@@ -345,16 +386,18 @@ static int map_single_launch(const fv3_domain* dom, int kord, int iv, int i1, in
   // q1, pe1, pe2 read and q1 written once per cell-level of the box
   TimedLaunch timed("map_single_kernel", as_stream(stream),
                     4.0 * sizeof(T) * (double)nib * njb * km * d.ntiles);
-  // Sets of 5 layers and 16 columns up to 80 layers (10 layers: 259 us, 8
-  // layers by 8 columns: 287 us, 5 by 32: 245 us, against 178 us on six C128
-  // tiles), 8 by 8 above them, where 16 columns leave one workgroup to a CU
-  // (127 layers on six C96 tiles: 322 against 254 us).  Columns of more layers
-  // than the four waves hold run in one thread each.
-  if (km <= 80) return map_layers_launch<T, 5, 16>(d, a, q1, pe1, pe2, qs, stream, who);
-  if (km <= kMapMaxLayers)
-    return map_layers_launch<T, 8, 8>(d, a, q1, pe1, pe2, qs, stream, who);
-  hipLaunchKernelGGL((map_single_kernel<T>), grid, dim3(256), 0, as_stream(stream), d, a, q1, pe1,
-                     pe2, qs, work);
+  switch (map_form(km, ((int64_t)nib * njb + 63) / 64 * d.ntiles, sizeof(T) == 4)) {
+    case kMapLayers:
+      return km <= 80 ? map_layers_launch<T, 5, 16>(d, a, q1, pe1, pe2, qs, stream, who)
+                      : map_layers_launch<T, 8, 8>(d, a, q1, pe1, pe2, qs, stream, who);
+    case kMapFused:
+      hipLaunchKernelGGL((map_single_kernel<T, true>), grid, dim3(256), 0, as_stream(stream), d, a,
+                         q1, pe1, pe2, qs, work);
+      break;
+    default:
+      hipLaunchKernelGGL((map_single_kernel<T, false>), grid, dim3(256), 0, as_stream(stream), d, a,
+                         q1, pe1, pe2, qs, work);
+  }
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }
@@ -418,6 +461,10 @@ static int map_single_noalloc(const fv3_domain* dom, int kord, int iv, int i1, i
 }  // namespace fv3
 
 extern "C" {
+
+int32_t fv3_plan_map_single(int32_t km, int64_t waves, int32_t fp32) {
+  return fv3::map_form(km, waves, fp32 != 0);
+}
 
 int32_t fv3_map_single_noalloc_f64(const fv3_domain* d, int32_t kord, int32_t mode, int32_t i1,
                                    int32_t i2, int32_t j1, int32_t j2, double* q1,

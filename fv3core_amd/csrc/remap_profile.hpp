@@ -1,7 +1,7 @@
 // RemapProfile (cs_profile) + MapSingle: the limiter's steps, and the column
 // kernel that the derivative code (remap_adjoint.hip) instantiates on
-// derivative-carrying numbers and the forward entry points (remap.hip) take for
-// columns of more layers than their own kernel holds on chip.
+// derivative-carrying numbers and the forward entry points (remap.hip) take
+// where it beats the one that spreads a column's layers over a workgroup.
 //
 // Reference: fv3core/stencils/remap_profile.py:119-638 (three stencils:
 // tridiagonal edge values, monotonicity constraints, kord 9/10 limiters) and
@@ -126,8 +126,8 @@ struct RemapCoef {
 // level s-1) over a register window of the column: a4_1 of levels s-3 .. s+2,
 // the clamped edges of level s-1 and the flags (extm | ext5 << 1 | ext6 << 2)
 // of levels s-2 .. s.  Steps run for s = 0 .. km in order, or from two levels
-// above the first wanted one: both column kernels drive the same steps, so
-// they give the same bits.
+// above the first wanted one: the forms of map_single_kernel and
+// map_layers_kernel drive the same steps, so they give the same bits.
 template <typename T>
 struct RemapLimiter {
   int kord, iv, km;
@@ -325,17 +325,21 @@ struct RemapLimiter {
   }
 };
 
-// slabs: 0 edge values (km+1), 1 gam (km+1), 2 a4_2, 3 a4_3, 4 a4_4, 5 copy
-//        of a4_1 (read after the walk has started overwriting q1)
+// slabs: 0 edge values (km+1), 1 gam (km+1), 2 a4_2, 3 a4_3, 4 a4_4 (not
+//        with FUSED), 5 copy of a4_1 (read after the walk has started
+//        overwriting q1)
 //
 // Sweeps: (1) upward forward elimination of the edge-value system with the
 // running values in registers; (2) downward back substitution; (3) one
 // upward sweep that clamps the edge values and forms the interpolation
 // coefficients, with a register window over the layer means, the clamped
 // edges and the extremum flags of the neighbouring levels; (4) the overlap
-// walk, which prefetches the next source layer.  Every value is formed by the
-// same operations in the same order as the stencils.
-template <typename T>
+// walk, which prefetches the next source layer.  FUSED runs (3) as a
+// producer one source layer ahead of the walk instead, so the coefficients
+// never go through memory: fewer bytes, but a longer dependent chain per
+// column, which pays only when the launch has waves enough to cover it.  Every value is
+// formed by the same operations in the same order as the stencils.
+template <typename T, bool FUSED>
 __global__ void __launch_bounds__(256)
     map_single_kernel(Dom d, RemapArgs a, T* __restrict__ q1, const T* __restrict__ pe1,
                       const T* __restrict__ pe2, const T* __restrict__ qs,
@@ -499,6 +503,7 @@ __global__ void __launch_bounds__(256)
     }
   }
 
+  if constexpr (!FUSED) {
   // ---- (3) one upward sweep of limiter steps; step s writes level s-1's
   // a4_2 .. a4_4
   {
@@ -584,6 +589,99 @@ __global__ void __launch_bounds__(256)
         }
       }
     }
+  }
+  } else {
+  // ---- (3) + (4): the limiter steps run as a producer one source layer
+  // ahead of the overlap walk that consumes them, so the limited coefficients
+  // never go through memory; a step's two loads are issued one step ahead.
+  {
+    RemapLimiter<T> lim(kord, iv, km, a.qmin, q_0, q_1, EV[0]);
+    int s = 0;
+    T nx_a = A1[2], nx_e = EV[1];
+    // producer step s; for s >= 1 it returns level s-1's a4_1 .. a4_4
+    auto produce = [&]() __attribute__((always_inline)) -> RemapCoef<T> {
+      RemapCoef<T> o{T(0), T(0), T(0), T(0)};
+      const T ap2 = nx_a, wp1 = nx_e;
+      nx_a = A1[min(s + 3, km - 1)];
+      nx_e = EV[min(s + 2, km)];
+      lim.step(s, ap2, wp1, o);
+      ++s;
+      return o;
+    };
+    // overlap walk (map_single.py:19-66) over source layers L, with layer L's
+    // coefficients in registers and layer L+1's produced as soon as L moves
+    produce();  // step 0: no level yet
+    T c1, c2, c3, c4, n1, n2, n3, n4;
+    {
+      const RemapCoef<T> a = produce();  // level 0
+      c1 = a.a1;
+      c2 = a.a2;
+      c3 = a.a3;
+      c4 = a.a4;
+      const RemapCoef<T> b = produce();  // level 1
+      n1 = b.a1;
+      n2 = b.a2;
+      n3 = b.a3;
+      n4 = b.a4;
+    }
+    int L = 0;
+    T pL = p_0, pR = p_1, nR = p_2;
+    auto advance = [&]() __attribute__((always_inline)) {  // L -> L + 1, for L < km - 1
+      L += 1;
+      pL = pR;
+      pR = nR;
+      c1 = n1;
+      c2 = n2;
+      c3 = n3;
+      c4 = n4;
+      if (L + 1 < km) {
+        nR = P1[L + 2];
+        const RemapCoef<T> b = produce();  // level L + 1
+        n1 = b.a1;
+        n2 = b.a2;
+        n3 = b.a3;
+        n4 = b.a4;
+      }
+    };
+    T p2k = P2[0];
+    for (int k0 = 0; k0 < km; k0 += KC) {
+      T p2v[KC];
+#pragma unroll
+      for (int u = 0; u < KC; ++u) p2v[u] = P2[min(k0 + u + 1, km)];
+#pragma unroll
+      for (int u = 0; u < KC; ++u) {
+        const int k = k0 + u;
+        if (k < km) {
+          const T p2n = p2v[u];
+          const T dpl = pR - pL;
+          const T pl = (p2k - pL) / dpl;
+          T out;
+          if (p2n <= pR) {
+            const T pr = (p2n - pL) / dpl;
+            out = c2 + T(0.5) * (c4 + c3 - c2) * (pr + pl) -
+                  (c4 * T(1) / T(3)) * (pr * (pr + pl) + pl * pl);
+          } else {
+            T qsum = (pR - p2k) * (c2 + T(0.5) * (c4 + c3 - c2) * (T(1) + pl) -
+                                   (c4 * T(1) / T(3)) * (T(1) + pl * (T(1) + pl)));
+            // valid columns (pe1 bottom at or below pe2 bottom) never pass the
+            // last layer; the bound only keeps a malformed column inside its
+            // storage
+            if (L < km - 1) advance();
+            while (L < km - 1 && pR < p2n) {
+              qsum += (pR - pL) * c1;
+              advance();
+            }
+            const T dpx = p2n - pL;
+            const T esl = dpx / (pR - pL);
+            qsum += dpx * (c2 + T(0.5) * esl * (c3 - c2 + c4 * (T(1) - T(2.0 / 3.0) * esl)));
+            out = qsum / (p2n - p2k);
+          }
+          Q[k] = out;
+          p2k = p2n;
+        }
+      }
+    }
+  }
   }
 }
 

@@ -211,8 +211,8 @@ int32_t fv3_delnflux_f32(const fv3_domain* d, int32_t mode, const int32_t nord4[
  * kord <= 10 (its magnitude selects the limiter), mode = iv in {-2,...,2};
  * qs (IJ, bottom value for iv = -2) may be NULL (then 0); qmin is the
  * kord-9 floor.  work: 7 slabs, each of work_slab elements laid out like the
- * fields (work_slab >= (ntiles-1)*st + (km+1)*sk); left alone for km <= 128,
- * where a column's intermediates stay on chip.
+ * fields (work_slab >= (ntiles-1)*st + (km+1)*sk); left alone where layers are
+ * spread over a workgroup and their intermediates stay on chip.
  */
 int32_t fv3_map_single_f64(const fv3_domain* d, int32_t kord, int32_t mode, int32_t i1,
                            int32_t i2, int32_t j1, int32_t j2, double* q1, const double* pe1,
@@ -742,6 +742,20 @@ int32_t fv3_cubed_to_latlon_f64(const fv3_domain* d, int32_t order, const double
                                 const double* v, const double* dx, const double* dy,
                                 const double* a11, const double* a12, const double* a21,
                                 const double* a22, double* ua, double* va, void* stream);
+
+/* ---- launch plans ------------------------------------------------------ */
+
+/*
+ * What a launcher chooses for a launch of this size (no counterpart in the
+ * reference; for tests and tuning).  Nothing is launched.  waves: columns / 64,
+ * rounded up in each tile; planes: strips along i times levels, tiles and
+ * scalars.
+ *   fv3_plan_map_single: 0 one thread per column, 1 the same with the limiter
+ *     fused into the walk, 2 layers spread over a workgroup.
+ *   fv3_plan_fvtp2d_rows: output rows of a segment of fv_tp_2d's march.
+ */
+int32_t fv3_plan_map_single(int32_t km, int64_t waves, int32_t fp32);
+int32_t fv3_plan_fvtp2d_rows(int32_t rows, int64_t planes, int32_t fp32);
 
 #ifdef __cplusplus
 }

@@ -3,15 +3,16 @@
 * fv3_fvtp2d_corner_fill: CopyCornersXY(q, q_x = q, q_y) + fv_tp_2d in one
   call (the y corner fill applied as the transport reads q) against the two
   calls, on domains with all four and with two cube corners.
-* fv_tp_2d segment height: the launcher takes 51-row segments for large
-  batches of narrow tiles and 33-row segments otherwise; columns of output
-  rows are computed the same way in either, so one call on 64 C48 tiles
-  (51-row segments) must equal eight calls on 8 tiles each (33-row
-  segments) bit for bit, FP64 and FP32.
-* map_single: the launcher takes the fused producer/walk form from 1024
-  waves of columns up and the four-sweep form below; columns are
-  independent, so one call on six 128 x 128 tiles (fused form) must equal
-  four calls on its quadrants (four-sweep form) bit for bit.
+* fv_tp_2d segment height: the rows of a segment follow from the launch's size;
+  output rows are computed the same way in any, so one call on 64 C48 tiles must
+  equal eight calls on 8 tiles each, which take segments of another height, bit
+  for bit, FP64 and FP32.
+* map_single: the launcher chooses between one thread per column (four sweeps,
+  or fused) and layers spread over a workgroup by layer count and columns.
+  Columns are independent, so one call on six 128 x 128 tiles must equal four
+  calls on its quadrants, which take another form, bit for bit; and the value
+  of the tangent-linear call, which runs one thread per column, must be that of
+  the spread form at the edges of its layer counts.
 """
 import ctypes
 
@@ -100,6 +101,10 @@ def test_fvtp2d_tall_segments_equal_regular_segments(dtype, hord):
                       _lib.ptr(fx), _lib.ptr(fy), s))
         return fx, fy
 
+    # the heights of the one call and of a part's, 49 rows of one strip a level
+    rows = [_lib.lib().fv3_plan_fvtp2d_rows(n + 1, ctypes.c_int64(t * nz),
+                                            int(dtype == torch.float32)) for t in (nt, chunk)]
+    assert rows[0] != rows[1], rows
     fx_all, fy_all = run(slice(0, nt))
     for c in range(0, nt, chunk):
         fx_c, fy_c = run(slice(c, c + chunk))
@@ -108,26 +113,42 @@ def test_fvtp2d_tall_segments_equal_regular_segments(dtype, hord):
     assert float(fx_all.abs().max()) > 0.0
 
 
+SWEEPS, FUSED, LAYERS = 0, 1, 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("nz,whole_form,part_form", [(10, SWEEPS, LAYERS), (81, FUSED, LAYERS),
+                                                     (137, FUSED, SWEEPS)])
 @pytest.mark.parametrize("kord,mode", [(9, 1), (10, 0), (10, -2), (9, -1)])
-def test_map_single_fused_form_equals_four_sweep_form(kord, mode):
-    n, nz, nt = 128, 79, 6
+def test_map_single_forms_equal(kord, mode, nz, whole_form, part_form, dtype):
+    n, nt, h = 128, 6, 64
     gi = GridIndexing((n, n, nz), 3, True, True, True, True)
     factory = StencilFactory(StencilConfig(), gi)
-    ins = [remap_inputs(n, nz, workload=90 + t) for t in range(nt)]
 
-    def batch(name):
-        b = utils.empty((nt,) + tuple(ins[0][name].shape), batch_dims=1)
-        for t in range(nt):
-            b[t].copy_(torch.as_tensor(ins[t][name]))
+    def plan(columns):
+        waves = (columns + 63) // 64 * nt
+        return _lib.lib().fv3_plan_map_single(nz, ctypes.c_int64(waves),
+                                              int(dtype == torch.float32))
+
+    assert (plan(n * n), plan(h * h)) == (whole_form, part_form)
+    g = torch.Generator(device="cuda").manual_seed(nz)
+    shape = (nt,) + gi.max_shape
+
+    def field(t):
+        b = utils.empty(shape, dtype=dtype, batch_dims=1)
+        b.copy_(t)
         return b
 
-    field = "q" if mode == 0 else ("w" if mode in (-2, -1) else "pt")
-    src, pe1, pe2, qs = batch(field), batch("pe1"), batch("pe2"), batch("qs")
-    qs = qs if mode == -2 else None
-    whole = _like(src)
+    def interfaces():
+        dp = 500.0 + 1000.0 * torch.rand(shape, generator=g, device="cuda", dtype=torch.float64)
+        return field(100.0 + 1e5 * dp.cumsum(-1) / dp.sum(-1, keepdim=True))
+
+    pe1, pe2 = interfaces(), interfaces()
+    pe2[..., 0], pe2[..., nz] = pe1[..., 0], pe1[..., nz]
+    src = field(torch.rand(shape, generator=g, device="cuda", dtype=torch.float64))
+    qs = field(torch.rand(shape, generator=g, device="cuda"))[..., 0] if mode == -2 else None
+    whole, parts = _like(src).to(dtype), _like(src).to(dtype)
     MapSingle(factory, kord, mode, gi.isc, gi.iec, gi.jsc, gi.jec)(whole, pe1, pe2, qs=qs)
-    parts = _like(src)
-    h = n // 2
     for i1 in (gi.isc, gi.isc + h):
         for j1 in (gi.jsc, gi.jsc + h):
             MapSingle(factory, kord, mode, i1, i1 + h - 1, j1, j1 + h - 1)(parts, pe1, pe2,
@@ -135,3 +156,26 @@ def test_map_single_fused_form_equals_four_sweep_form(kord, mode):
     torch.cuda.synchronize()
     assert torch.equal(whole, parts)
     assert not torch.equal(whole, src)
+
+
+@pytest.mark.parametrize("nz", [79, 80, 81, 127, 128])
+@pytest.mark.parametrize("mode", [-2, -1, 0, 1, 2])
+def test_map_single_spread_layers_equal_the_tangent_linear_value(mode, nz, monkeypatch):
+    from fv3core_amd import workloads
+    from fv3core_amd.adjoint import RemapLinearization
+
+    monkeypatch.setattr(workloads, "hybrid_coefficients", workloads.synthetic_hybrid)
+    n = 7
+    d = remap_inputs(n, nz, workload=91)
+    gi = GridIndexing((n, n, nz), 3, True, True, True, True)
+    box = (gi.isc, gi.iec, gi.jsc, gi.jec)
+    assert _lib.lib().fv3_plan_map_single(nz, ctypes.c_int64(1), 0) == LAYERS
+    src = to_storage(d["q"] if mode == 0 else d["w"] if mode in (-2, -1) else d["pt"])
+    pe1, pe2 = to_storage(d["pe1"]), to_storage(d["pe2"])
+    qs = to_storage(d["qs"]) if mode == -2 else None
+    spread = _like(src)
+    MapSingle(StencilFactory(StencilConfig(), gi), 9, mode, *box)(spread, pe1, pe2, qs=qs)
+    value, _ = RemapLinearization(gi, mode).tlm(src, _like(src), pe1, pe2, qs)
+    torch.cuda.synchronize()
+    assert torch.equal(spread[..., :nz], value[..., :nz])
+    assert not torch.equal(spread, src)
