@@ -4,42 +4,44 @@
 // Reference: fv3core/stencils/sim1_solver.py:11-101 (two tridiagonal
 // solves, for the pressure perturbation and for w, plus the dz update),
 // riem_solver_c.py:13-165 and riem_solver3.py:24-242 (precompute / sim1 /
-// finalize stencils).  Each solver is one kernel, always in FP64, that reads
-// every input level once (pt, cappa and w a second time at the end, which
-// frees their registers in between) and keeps all intermediates on chip.
+// finalize stencils).  Each solver is one kernel, always in FP64.  Two are
+// here for each: this file's, which spreads a column's levels over a workgroup
+// and reads every input level once (pt, cappa and w a second time at the end,
+// which frees their registers in between), and riem_column.hpp's, which runs a
+// column in one thread, where that is the faster one (riem_form).
 //
 // What bounds it: nearly all of the ~1000 instructions a column-level takes
 // are the logs, exps and divisions of pressures and coefficients, which
 // depend on their own level only; what one level hands to the next is two
-// division chains and a few sums.  One thread per column (as these kernels
-// were) runs everything in sequence, at less than one wave per SIMD on a C96
-// cube, and reads the inputs again in each of six sweeps.  Here a column's
-// levels are spread over a workgroup: RC columns by sets of LV levels, two
-// sets to a wave.  Every thread forms the independent part of its levels in
-// registers, and the recurrences run as chains: the waves take turns, each
-// carrying the running values through its levels and handing them on through
-// LDS.  Sums and recurrences keep the order of the stencils' sweeps, so the
-// results are those of the one-thread form bit for bit.
+// division chains and a few sums.  One thread per column runs everything in
+// sequence, at less than one wave per SIMD on a C96 cube, and reads the inputs
+// again in each of six sweeps.  Here a column's levels are spread over a
+// workgroup: RC columns by sets of LV levels, two sets to a wave.  Every thread
+// forms the independent part of its levels in registers, and the recurrences
+// run as eight chains (A to H): the waves take turns, each carrying the running
+// values through its levels and handing them on through LDS.  Sums and
+// recurrences keep the order of the stencils' sweeps, so the results are those
+// of the one-thread form bit for bit.  Intermediates stay on chip but for what
+// five levels a thread spill: 28 to 68 bytes a lane.
 //
 // Measured (RiemannSolver3, last call, 79 levels, one MI355X; one thread per
-// column -> levels spread): six C12 tiles 224 -> 45 us, six C51 193 -> 66 us,
-// six C96 303 -> 240 us, six C128 628 -> 404 us, 96 C48 tiles with FP32
-// inputs 1246 -> 1013 us.  One workgroup takes about 104 k cycles, of which
+// column -> levels spread): six C12 tiles 224 -> 46 us, six C51 193 -> 66 us,
+// six C96 311 -> 242 us, six C128 628 -> 406 us, 96 C48 tiles with FP32
+// inputs 1242 -> 1014 us.  One workgroup takes about 104 k cycles, of which
 // the chains take 60 k; with two to a CU one's chains run beside the other's
 // independent parts.  64 columns by 10 levels (a whole wave per set, one
 // workgroup per CU) measured 342 us on six C96 tiles.
+#include <algorithm>
+#include <cmath>
+
 #include "common.hpp"
 #include "divide.hpp"
+#include "riem_column.hpp"
 #include "timing.hpp"
 
 namespace fv3 {
 
-constexpr double kRdgas = 287.05;
-constexpr double kGrav = 9.80665;
-constexpr double kCpAir = 1004.6;
 constexpr int RC = 32;      // columns per workgroup (half a wave)
-
-__device__ __forceinline__ double gm_of(double cp3) { return 1.0 / (1.0 - cp3); }
 
 // The low (hi = false) or high half-wave's value in both halves.
 __device__ __forceinline__ double half_bcast(double v, bool hi) {
@@ -50,33 +52,6 @@ __device__ __forceinline__ double half_bcast(double v, bool hi) {
   return __builtin_bit_cast(double, hi ? ((unsigned long long)b[1] << 32) | a[1]
                                        : ((unsigned long long)b[0] << 32) | a[0]);
 }
-
-struct Box2 {
-  int i1, j1, nib, njb;
-};
-
-struct Riem3Opts {
-  int last_call, use_logp;
-  double beta, dt, ptop, p_fac, peln1, ptk, kappa, rgrav;
-};
-
-// Fields of one solver call.  RiemannSolverC: dp = delpc, qc = q_con,
-// z = gz (geopotential, written at the end), pt = ptc, w = w3 (read only);
-// RiemannSolver3: dp = delp, z = zh (height, written at the end), w in/out,
-// plus the pressure outputs.
-// S is the storage type of cappa, q_con, delp, pt and w: FP64, or FP32 in
-// the mixed-precision acoustic step (loaded into FP64, w stored back
-// rounded); the solve itself is always FP64.
-template <typename S>
-struct RiemFields {
-  const S *cappa, *qc, *dp, *pt;
-  const double* surf;  // hs (C) or zs (3), IJ
-  const double* wsd;   // ws (C) or wsd (3), IJ
-  double* z;
-  S* w;
-  double* pef;                                  // C only
-  double *delz, *pe, *ppe, *pk3, *pk, *peln;    // 3 only
-};
 
 constexpr int kRiemMaxLevels = 128;
 
@@ -91,7 +66,7 @@ constexpr int kRiemMaxLevels = 128;
 // neighbours.  At most five column arrays are alive at a time (2 LV registers
 // each), so that two workgroups fit a CU: gm, gr and w are formed or loaded a
 // second time instead of kept.
-template <bool C, typename S, typename OFF, int LV, int NW>
+template <bool C, typename S, int LV, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV <= 5 ? 4 : 2)))
     riem_kernel(Dom d, Box2 bx, Riem3Opts o, double dt, double p_fac, RiemFields<S> f) {
   extern __shared__ double lds[];
@@ -118,6 +93,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(LV
   // fields are addressed as a tile's uniform base plus the lane's offset in
   // elements, layers past the bottom clamped to it
   const int64_t tb = (int64_t)t * d.st;
+  typedef uint32_t OFF;
   const OFF sk = (OFF)d.sk;
   const OFF c = (OFF)j * (OFF)d.sj + (OFF)i;
   auto ptr = [tb](auto* base, OFF e) {
@@ -455,31 +431,95 @@ static bool riem_narrow(const fv3_domain* dom) {
   return ((int64_t)dom->nk * dom->sk) * (int64_t)sizeof(double) < (int64_t)1 << 32;
 }
 
-template <bool C, typename S, typename OFF, int LV, int NW>
+// Microseconds of a launch on `waves` waves of columns (64 each), by the forms
+// below.  Measured over 3 .. 127 layers on 18 to 3840 waves, FP64 and FP32
+// inputs; the estimates hold within about 15 %.
+//
+// One thread per column: 2.1 us a layer (RiemannSolver3 2.5) at the latency of
+// its sweeps, more where memory bounds them, in rounds of the workgroups whose
+// column array fits the LDS (1024 up to 80 interfaces, 512 from 106 on).
+static double riem_column_us(int nz, int64_t waves, bool c, bool fp32) {
+  const int64_t lds = ((int64_t)(nz + 1) * RW * 8 + 1279) / 1280 * 1280;  // as allocated
+  const int64_t round = 256 * std::min<int64_t>(16, 160 * 1024 / lds);
+  const bool small = c ? waves < 2000 : nz <= 40 && waves < 2000;
+  const double rate = c ? (fp32 ? (small ? 2.75 : 2.8) : (small ? 3.05 : 3.1))
+                        : (fp32 ? (small ? 3.5 : 4.1) : (small ? 3.9 : 4.6));
+  auto layer = [&](int64_t w) {
+    return w == 0 ? 0.0 : std::max((c ? 2.1 : 2.5) + 0.6e-3 * w, rate * 1e-3 * w);
+  };
+  double t = (waves / round) * layer(round) + layer(waves % round);
+  if (waves > round && round <= 1024)
+    t = std::max(t, (c ? 3.9 : fp32 ? 4.8 : 5.1) * 1e-3 * waves);
+  return nz * t + 4.5;
+}
+
+// Levels over a workgroup, lv to a thread: up to four waves (two of lv 8) a
+// latency and a time per wave of columns; more of them in rounds of the
+// workgroups whose registers fit the chip (16 waves to a CU at lv 5, 8 at lv 8).
+static double riem_levels_us(int lv, int nz, int64_t waves, bool c) {
+  const int nw = (nz + 2 * lv - 1) / (2 * lv);
+  if (nw > 8) return 1e30;
+  static const double few5[5][3] = {{}, {14, 6, 18}, {25, 8, 38}, {33, 10, 66}, {41, 15, 91}};
+  static const double few8[3][3] = {{}, {19, 6, 30}, {36, 12, 76}};
+  if (nw <= (lv == 5 ? 4 : 2)) {
+    const double* f = lv == 5 ? few5[nw] : few8[nw];
+    return std::max(f[0], (f[1] + f[2] * 1e-3 * waves) * (c ? 1.0 : 1.1));
+  }
+  // alone, per round of RiemannSolverC, of RiemannSolver3
+  static const double round5[4][3] = {{51, 65, 80}, {58, 57.5, 59}, {66, 62, 63}, {74, 64, 68}};
+  static const double round8[6][3] = {{48, 44, 47}, {58, 53, 57}, {52, 53, 53},
+                                      {60, 60, 60}, {68, 68, 67}, {76, 76, 75}};
+  const double* r = lv == 5 ? round5[nw - 5] : round8[nw - 3];
+  const int per_cu = (lv == 5 ? 16 : 8) / nw;
+  const double rounds = 2.0 * waves / (256.0 * per_cu);
+  if (rounds <= 1.0) return r[0];
+  return c || per_cu == 1 ? (c ? r[1] : r[2]) * std::ceil(rounds) : r[2] * (rounds + 0.35);
+}
+
+// The form with the least time: one thread per column (0), or 5 or 8 levels a
+// thread.  Few layers and launches of one full round of columns take the
+// column form (RiemannSolverC on six C96 tiles, 79 layers: 242 against 261 us;
+// 4 layers: 17 against 22 us), which spreads nothing where every SIMD already
+// has a wave; 100 layers on six C128 tiles 722 against 887 us, since 8 levels
+// a thread leave one workgroup to a CU.  Below half a workgroup a CU the
+// levels' latency alone counts.
+static int riem_form(int nz, int64_t waves, bool c, bool fp32) {
+  if (waves >= 100 && nz <= (waves < 500 ? 4 : fp32 ? 7 : 6)) return 0;
+  if (waves <= 128) return nz <= 80 ? 5 : 8;
+  const double t0 = riem_column_us(nz, waves, c, fp32);
+  const double t5 = riem_levels_us(5, nz, waves, c), t8 = riem_levels_us(8, nz, waves, c);
+  if (t0 <= t5 && t0 <= t8) return 0;
+  return t5 <= t8 ? 5 : 8;
+}
+
+template <bool C, typename S, int LV, int NW>
 void riem_launch_as(const fv3_domain* dom, hipStream_t s, const Dom& d, Box2 bx,
                     const Riem3Opts& o, double dt, double p_fac, const RiemFields<S>& f) {
   const dim3 grid((unsigned)((bx.nib * bx.njb + RC - 1) / RC), (unsigned)d.ntiles);
-  hipLaunchKernelGGL((riem_kernel<C, S, OFF, LV, NW>), grid, dim3(64, riem_waves<LV>(dom->nk)),
+  hipLaunchKernelGGL((riem_kernel<C, S, LV, NW>), grid, dim3(64, riem_waves<LV>(dom->nk)),
                      riem_lds_bytes<LV>(dom->nk), s, d, bx, o, dt, p_fac, f);
 }
 
 template <bool C, typename S>
 void riem_launch(const fv3_domain* dom, hipStream_t s, const Dom& d, Box2 bx, const Riem3Opts& o,
                  double dt, double p_fac, const RiemFields<S>& f) {
-  // 5 levels a thread up to 80 layers: 8 waves of 128 registers, two
-  // workgroups to a CU.  Above that 8 levels a thread (up to 128 layers), one
-  // workgroup to a CU: 100 layers on six C96 tiles 594 us with one thread per
-  // column, 454 us so, 639 us squeezed into 128 registers.
-  if (!riem_narrow(dom))
-    riem_launch_as<C, S, int64_t, 8, 8>(dom, s, d, bx, o, dt, p_fac, f);
-  else if (riem_waves<5>(dom->nk) <= 8)
-    riem_launch_as<C, S, uint32_t, 5, 8>(dom, s, d, bx, o, dt, p_fac, f);
-  else
-    riem_launch_as<C, S, uint32_t, 8, 8>(dom, s, d, bx, o, dt, p_fac, f);
+  const int64_t waves = ((int64_t)bx.nib * bx.njb + RW - 1) / RW * d.ntiles;
+  // the level kernels' byte offsets in a tile are 32 bits wide
+  const int form =
+      riem_narrow(dom) ? riem_form(dom->nk - 1, waves, C, sizeof(S) == 4) : 0;
+  if (form == 5) {
+    riem_launch_as<C, S, 5, 8>(dom, s, d, bx, o, dt, p_fac, f);
+  } else if (form == 8) {
+    riem_launch_as<C, S, 8, 8>(dom, s, d, bx, o, dt, p_fac, f);
+  } else {
+    const dim3 grid((unsigned)(((int64_t)bx.nib * bx.njb + RW - 1) / RW), (unsigned)d.ntiles);
+    hipLaunchKernelGGL((riem_column_kernel<C, S>), grid, dim3(RW),
+                       (size_t)dom->nk * RW * sizeof(double), s, d, bx, o, dt, p_fac, f);
+  }
 }
 
 static int check_riem(const fv3_domain* dom, const char* who, int i1, int i2, int j1, int j2,
-                      int64_t slab, int nslabs) {
+                      int64_t slab) {
   int rc = check_domain(dom, who);
   if (rc) return rc;
   FV3_REQUIRE(dom->nk >= 4, FV3_E_ARG, "%s: need at least 4 levels", who);
@@ -489,7 +529,6 @@ static int check_riem(const fv3_domain* dom, const char* who, int i1, int i2, in
               "%s: box outside the storage", who);
   FV3_REQUIRE(slab >= (int64_t)(dom->ntiles - 1) * dom->st + dom->sk * dom->nk, FV3_E_ARG,
               "%s: workspace slab too small", who);
-  (void)nslabs;
   return FV3_OK;
 }
 
@@ -504,7 +543,7 @@ int riem_solver_c(const fv3_domain* dom, double dt2, double ptop, double p_fac, 
     return FV3_E_ARG;
   }
   const int i1 = dom->isc - 1, i2 = dom->iec + 1, j1 = dom->jsc - 1, j2 = dom->jec + 1;
-  int rc = check_riem(dom, who, i1, i2, j1, j2, work_slab, 3);
+  int rc = check_riem(dom, who, i1, i2, j1, j2, work_slab);
   if (rc) return rc;
   FV3_REQUIRE(cappa && hs && ws && ptc && q_con && delpc && gz && pef && w3 && work, FV3_E_ARG,
               "%s: NULL pointer", who);
@@ -523,6 +562,8 @@ int riem_solver_c(const fv3_domain* dom, double dt2, double ptop, double p_fac, 
   f.z = gz;
   f.w = const_cast<S*>(w3);  // read only in this solver
   f.pef = pef;
+  f.work = work;
+  f.slab = work_slab;
   // cappa, ptc, q_con, delpc, gz, w3 read; gz, pef written (per cell-level)
   TimedLaunch timed("riem_c_kernel", as_stream(stream),
                     (4.0 * sizeof(S) + 4.0 * sizeof(double)) * bx.nib * bx.njb *
@@ -544,7 +585,7 @@ int riem_solver3(const fv3_domain* dom, int last_call, double dt, double ptop, d
     return FV3_E_ARG;
   }
   const int i1 = dom->isc, i2 = dom->iec, j1 = dom->jsc, j2 = dom->jec;
-  int rc = check_riem(dom, who, i1, i2, j1, j2, work_slab, 3);
+  int rc = check_riem(dom, who, i1, i2, j1, j2, work_slab);
   if (rc) return rc;
   FV3_REQUIRE(cappa && zs && wsd && delz && q_con && delp && pt && zh && pe && ppe && pk3 &&
                   pk && peln && w && work,
@@ -579,6 +620,8 @@ int riem_solver3(const fv3_domain* dom, int last_call, double dt, double ptop, d
   f.pk3 = pk3;
   f.pk = pk;
   f.peln = peln;
+  f.work = work;
+  f.slab = work_slab;
   // cappa, q_con, delp, pt, zh, w read; zh, ppe, pk3, delz, w written, plus
   // pe, pk and peln on the last call (per cell-level)
   TimedLaunch timed("riem3_kernel", as_stream(stream),
@@ -591,6 +634,10 @@ int riem_solver3(const fv3_domain* dom, int last_call, double dt, double ptop, d
 }  // namespace fv3
 
 extern "C" {
+
+int32_t fv3_plan_riem(int32_t nz, int64_t waves, int32_t solver_c, int32_t fp32) {
+  return fv3::riem_form(nz, waves, solver_c != 0, fp32 != 0);
+}
 
 int32_t fv3_riem_solver_c_f64(const fv3_domain* dom, double dt2, double ptop, double p_fac,
                               const double* cappa, const double* hs, const double* ws,

@@ -273,8 +273,8 @@ int32_t fv3_map_single_adjoint_f64(const fv3_domain* d, int32_t kord, int32_t mo
  * RiemannSolverC.__call__ (fv3core/stencils/riem_solver_c.py:119-165):
  * precompute + sim1_solver + finalize on [isc-1, iec+1] x [jsc-1, jec+1],
  * d->nk = nz + 1 levels (4 .. 128), FP64.  Outputs gz and pef; w3 is read
- * only.  work: 3 slabs of work_slab elements (>= (ntiles-1)*st + nk*sk),
- * which the present kernel leaves alone (its intermediates stay on chip).
+ * only.  work: 3 slabs of work_slab elements (>= (ntiles-1)*st + nk*sk), used
+ * where a thread runs a whole column.
  */
 int32_t fv3_riem_solver_c_f64(const fv3_domain* d, double dt2, double ptop, double p_fac,
                               const double* cappa, const double* hs, const double* ws,
@@ -286,7 +286,7 @@ int32_t fv3_riem_solver_c_f64(const fv3_domain* d, double dt2, double ptop, doub
  * RiemannSolver3.__call__ (fv3core/stencils/riem_solver3.py:145-242) on the
  * compute domain, d->nk = nz + 1 levels (4 .. 128), FP64 (a_imp > 0.999
  * path).  In/out: delz, zh, pe, ppe, pk3, pk, peln, w; pe is written only
- * on the last call.  work: 3 slabs, left alone like RiemannSolverC's.
+ * on the last call.  work: 3 slabs, used as RiemannSolverC's.
  */
 int32_t fv3_riem_solver3_f64(const fv3_domain* d, int32_t last_call, double dt, double ptop,
                              double p_fac, int32_t use_logp, double beta, const double* cappa,
@@ -752,9 +752,11 @@ int32_t fv3_cubed_to_latlon_f64(const fv3_domain* d, int32_t order, const double
  * scalars.
  *   fv3_plan_map_single: 0 one thread per column, 1 the same with the limiter
  *     fused into the walk, 2 layers spread over a workgroup.
+ *   fv3_plan_riem: 0 one thread per column, else the levels a thread holds.
  *   fv3_plan_fvtp2d_rows: output rows of a segment of fv_tp_2d's march.
  */
 int32_t fv3_plan_map_single(int32_t km, int64_t waves, int32_t fp32);
+int32_t fv3_plan_riem(int32_t nz, int64_t waves, int32_t solver_c, int32_t fp32);
 int32_t fv3_plan_fvtp2d_rows(int32_t rows, int64_t planes, int32_t fp32);
 
 #ifdef __cplusplus

@@ -13,6 +13,8 @@
   calls on its quadrants, which take another form, bit for bit; and the value
   of the tangent-linear call, which runs one thread per column, must be that of
   the spread form at the edges of its layer counts.
+* The Riemann solvers: one thread per column and both level counts a thread
+  holds must return the same bits, on one call and on calls of its parts.
 """
 import ctypes
 
@@ -179,3 +181,63 @@ def test_map_single_spread_layers_equal_the_tangent_linear_value(mode, nz, monke
     torch.cuda.synchronize()
     assert torch.equal(spread[..., :nz], value[..., :nz])
     assert not torch.equal(spread, src)
+
+
+COLUMN = 0  # the other forms of the Riemann solvers go by the levels a thread holds
+
+
+# Every pair of forms: few layers, 16 layers (one wave of 8 levels a thread), a
+# full round of columns, above the reach of 5 levels a thread.
+@pytest.mark.parametrize("solver_c,nz,tiles,whole_form,part_form", [
+    (True, 4, 8, COLUMN, 5), (True, 16, 16, 8, 5), (True, 79, 56, COLUMN, 5),
+    (True, 90, 40, COLUMN, 8), (False, 4, 8, COLUMN, 5), (False, 16, 16, 8, 5),
+    (False, 64, 16, 8, 5), (False, 90, 40, COLUMN, 8)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_riemann_forms_equal(solver_c, nz, tiles, whole_form, part_form, dtype, monkeypatch):
+    from fv3core_amd import workloads
+    from fv3core_amd._config import RiemannConfig
+    from fv3core_amd.stencils.riem_solver3 import RiemannSolver3
+    from fv3core_amd.stencils.riem_solver_c import RiemannSolverC
+
+    monkeypatch.setattr(workloads, "hybrid_coefficients", workloads.synthetic_hybrid)
+    n = 30 if solver_c else 32  # 1024 columns a tile
+    for waves, form in ((16 * tiles, whole_form), (16, part_form)):
+        assert _lib.lib().fv3_plan_riem(nz, ctypes.c_int64(waves), int(solver_c),
+                                        int(dtype == torch.float32)) == form
+    r = workloads.riemann_inputs(n, nz, workload=7)
+    gi = GridIndexing((n, n, nz), 3, True, True, True, True)
+    factory = StencilFactory(StencilConfig(), gi)
+    bulk = ("cappa", "pt", "q_con", "delp", "w")
+
+    def batch(name):
+        a = torch.as_tensor(np.ascontiguousarray(r[name]), device="cuda")
+        b = utils.empty((tiles,) + tuple(a.shape), batch_dims=1,
+                        dtype=dtype if name in bulk else torch.float64)
+        b.copy_(a.expand(b.shape))
+        if name == "pt":  # tiles that differ
+            b.mul_(1.0 + 1e-3 * torch.arange(tiles, device="cuda").view(-1, 1, 1, 1))
+        return b
+
+    out = []
+    for parts in (False, True):
+        t = {k: batch(k) for k in bulk + ("gz", "zh", "delz", "pe", "hs", "ws", "zs")}
+        o = [batch("pe").zero_() for _ in range(4)]
+        for sl in ([slice(k, k + 1) for k in range(tiles)] if parts else [slice(0, tiles)]):
+            f = {k: v[sl] for k, v in t.items()}
+            p = [v[sl] for v in o]
+            if solver_c:
+                RiemannSolverC(factory, 0.05)(18.75, f["cappa"], r["ptop"], f["hs"], f["ws"],
+                                              f["pt"], f["q_con"], f["delp"], f["gz"], p[0],
+                                              f["w"])
+            else:
+                RiemannSolver3(factory, RiemannConfig(p_fac=0.05, a_imp=1.0, use_logp=False,
+                                                      beta=0.0))(
+                    True, 37.5, f["cappa"], r["ptop"], f["zs"], f["ws"], f["delz"], f["q_con"],
+                    f["delp"], f["pt"], f["zh"], f["pe"], *p, f["w"])
+        out.append(list(t.values()) + o)
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    changed = out[0][5 if solver_c else 6]
+    assert not torch.equal(changed, batch("gz" if solver_c else "zh"))
+    assert bool(torch.isfinite(changed).all())
