@@ -329,6 +329,139 @@ struct A2BInterp {
   }
 };
 
+// The same means and interpolation in LDS blocks, for small launches: one
+// workgroup owns AB_TI x AB_TJ corners of one level.  It stages q over the block
+// plus a 3-cell halo, forms the x means on the rows j - 3 .. j + 2 and the y
+// means on the columns i - 3 .. i + 2 of its corners there, and interpolates.
+// Lane x of every wave owns LDS column x; wave y owns rows y, y + AB_NY, ...
+// Six more rows are read per block and both means pass through LDS behind two
+// barriers, but a block's rows run side by side where the march runs them one
+// after the other.  Measured on 12 to 192 cells a side, 4 to 127 levels, one to
+// 96 tiles, one field or the pressure gradient's four, the march overtakes it
+// between 3000 and 4500 blocks.  One field of 79 levels, block and march: one
+// C12 tile 13.7 and 16.3 us, six 15.2 and 21.0, six C48 29.4 and 32.3, six C96
+// 64.0 and 61.3, 96 C48 274 and 208 us.
+constexpr int64_t kA2BMarchBlocks = 3500;
+constexpr int AB_W = 64;         // LDS columns = TI + 6
+constexpr int AB_TI = AB_W - 6;  // corners per block in i
+constexpr int AB_TJ = 16;        // corners per block in j
+constexpr int AB_H = AB_TJ + 6;  // q rows: j0-3 .. j0+TJ+2
+constexpr int AB_NY = 8;         // waves per block
+
+template <typename T>
+__global__ void __launch_bounds__(AB_W * AB_NY)
+    a2b_block_kernel(Dom d, A2BInterp<T> p, int nbi) {
+  __shared__ T sq[AB_H][AB_W];
+  __shared__ T sx[AB_H - 1][AB_W];  // x means on rows j0-3 .. j0+TJ+1
+  __shared__ T sy[AB_TJ][AB_W];     // y means on rows j0 .. j0+TJ-1
+  const int li = threadIdx.x, ty = threadIdx.y;
+  const int bi = blockIdx.x % nbi, bj = blockIdx.x / nbi;
+  int k = (int)blockIdx.y;
+  const int n = a2b_field(p.f, k), t = blockIdx.z;
+  const int i0 = p.ci0 + bi * AB_TI, j0 = p.cj0 + bj * AB_TJ;
+  const int i = i0 - 3 + li;  // absolute column of this lane
+  const int jb = j0 - 3;      // absolute row of LDS row 0
+  const bool col_ok = i >= 0 && i < d.ni;
+  const int64_t off3 = (int64_t)t * d.st + (int64_t)k * d.sk;
+  const int64_t off2 = (int64_t)t * d.st2;
+  const T* const qin = p.f.qin[n] + off3;
+  T* const qout = p.f.qout[n] + off3;  // holds the tile-edge lines
+  for (int r = ty; r < AB_H; r += AB_NY) {
+    const int j = jb + r;
+    sq[r][li] = (col_ok && j >= 0 && j < d.nj) ? qin[(int64_t)j * d.sj + i] : T(0);
+  }
+  __syncthreads();
+  // x means, i in [isc, iec+1], j in [jsc-2, jec+2], in the march's forms
+  if (li >= 3 && li < AB_W - 3 && i >= d.isc && i <= d.iec + 1) {
+    int form = 0, sh = 0;  // sh: the outer form's point, relative to i
+    if (i == d.ie) {
+      form = 3;
+      sh = 1;
+    } else if (i == d.ie + 1) {
+      form = 1;
+    } else if (i == d.is + 1) {
+      form = 2;
+      sh = -1;
+    } else if (i == d.is) {
+      form = 1;
+    }
+    const bool west = form == 2;
+    for (int r = ty; r < AB_H - 1; r += AB_NY) {
+      const int j = jb + r;
+      if (j < d.jsc - 2 || j > d.jec + 2) continue;
+      const T* q = &sq[r][li];
+      T v = T(kB2) * (q[-2] + q[1]) + T(kB1) * (q[-1] + q[0]);
+      if (form != 0) {
+        const T* gr = p.xr + ((int64_t)t * p.nrow + (j - (d.jsc - 2))) * 4;
+        const bool wside = i <= d.is + 1;
+        const T g_in = wside ? gr[0] : gr[2], g_ou = wside ? gr[1] : gr[3];
+        const T* qb = q + sh;
+        const T outer = T(0.5) * (((T(2) + g_in) * qb[0] - qb[1]) / (T(1) + g_in) +
+                                  ((T(2) + g_ou) * qb[-1] - qb[-2]) / (T(1) + g_ou));
+        if (form == 1) {
+          v = outer;
+        } else {
+          auto qm = [&](int m) { return west ? q[m] : q[-1 - m]; };
+          const T g = west ? g_in : g_ou;
+          const T inner = T(kB2) * (qm(-1) + qm(2)) + T(kB1) * (qm(0) + qm(1));
+          v = (T(3) * (g * qm(-1) + qm(0)) - (g * outer + inner)) / (T(2) + T(2) * g);
+        }
+      }
+      sx[r][li] = v;
+    }
+  }
+  // y means, i in [isc-2, iec+2], j in [jsc, jec+1]; only the rows on the
+  // tile-edge interfaces read the cell lengths
+  if (li < AB_W - 1 && i >= d.isc - 2 && i <= d.iec + 2) {
+    for (int r = ty; r < AB_TJ; r += AB_NY) {
+      const int j = j0 + r;
+      if (j >= d.jsc && j <= d.jec + 1) {
+        T v = T(kB2) * (sq[r + 1][li] + sq[r + 4][li]) + T(kB1) * (sq[r + 2][li] + sq[r + 3][li]);
+        if (j == d.js || j == d.js + 1 || j == d.je || j == d.je + 1) {
+          const int64_t o2 = off2 + (int64_t)j * d.sj2 + i;
+          T q7[7], dy7[7];
+#pragma unroll
+          for (int u = 0; u < 7; ++u) {
+            q7[u] = sq[r + u][li];
+            dy7[u] = p.m.dya[o2 + (int64_t)(u - 3) * d.sj2];
+          }
+          v = volume_mean(q7, dy7, j, d.js, d.je);
+        }
+        sy[r][li] = v;
+      }
+    }
+  }
+  __syncthreads();
+  // a2b_interpolation on the block's corners (qx rows and qy columns -3 .. +2)
+  if (li < 3 || li >= 3 + AB_TI || i > p.ci1) return;
+  const int64_t sj = d.sj;
+  for (int r = ty; r < AB_TJ; r += AB_NY) {
+    const int j = j0 + r;
+    if (j > p.cj1) break;
+    const int x = r + 3;  // sx row of j
+    T* const o = qout + (int64_t)j * sj + i;
+    T qxx = T(kA2) * (sx[x - 2][li] + sx[x + 1][li]) + T(kA1) * (sx[x - 1][li] + sx[x][li]);
+    T qyy = T(kA2) * (sy[r][li - 2] + sy[r][li + 1]) + T(kA1) * (sy[r][li - 1] + sy[r][li]);
+    if (j == d.js + 1) {
+      const T up = T(kA2) * (sx[x - 1][li] + sx[x + 2][li]) + T(kA1) * (sx[x][li] + sx[x + 1][li]);
+      qxx = T(kCc1) * (sx[x - 1][li] + sx[x][li]) + T(kCc2) * (o[-sj] + up);
+    }
+    if (j == d.je) {
+      const T lo = T(kA2) * (sx[x - 3][li] + sx[x][li]) + T(kA1) * (sx[x - 2][li] + sx[x - 1][li]);
+      qxx = T(kCc1) * (sx[x - 1][li] + sx[x][li]) + T(kCc2) * (o[sj] + lo);
+    }
+    if (i == d.is + 1) {
+      const T rr = T(kA2) * (sy[r][li - 1] + sy[r][li + 2]) + T(kA1) * (sy[r][li] + sy[r][li + 1]);
+      qyy = T(kCc1) * (sy[r][li - 1] + sy[r][li]) + T(kCc2) * (o[-1] + rr);
+    }
+    if (i == d.ie) {
+      const T l = T(kA2) * (sy[r][li - 3] + sy[r][li]) + T(kA1) * (sy[r][li - 2] + sy[r][li - 1]);
+      qyy = T(kCc1) * (sy[r][li - 1] + sy[r][li]) + T(kCc2) * (o[1] + l);
+    }
+    *o = T(0.5) * (qxx + qyy);
+  }
+}
+
 }  // namespace
 
 template <typename T>
@@ -402,6 +535,14 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
   // q read, qout written (per corner-level)
   TimedLaunch timed("a2b_interp_kernel", s,
                     2.0 * sizeof(T) * (double)(ie1 - is2 + 1) * (je1 - js2 + 1) * nk * d.ntiles);
+  const int nbi = (ie1 - is2 + AB_TI) / AB_TI, nbj = (je1 - js2 + AB_TJ) / AB_TJ;
+  if ((int64_t)nbi * nbj * nk * d.ntiles < kA2BMarchBlocks) {
+    hipLaunchKernelGGL((a2b_block_kernel<T>),
+                       dim3((unsigned)(nbi * nbj), (unsigned)nk, (unsigned)d.ntiles),
+                       dim3(AB_W, AB_NY), 0, s, d, interp, nbi);
+    FV3_HIP_CHECK_LAUNCH(who);
+    return FV3_OK;
+  }
   return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, 5, interp, who, FV3_AB_TJ);
 }
 

@@ -206,12 +206,15 @@ def test_gpu_a2b_ord4_matches_oracle(cube_tiles):
 
 
 # Corner boxes of one column and more up to one and two strips of 58 columns,
-# row counts at the edges of a block of rows, segments of several heights.
+# row counts at the edges of a block of rows; few levels, which run in LDS blocks,
+# and enough of them for the march, with segments of several heights.
 @pytest.mark.gpu
-@pytest.mark.parametrize("cube_tiles", [False, True])
-@pytest.mark.parametrize("n,nz", [(4, 3), (5, 3), (6, 4), (7, 3), (57, 3), (58, 3), (59, 3),
-                                  (60, 3), (24, 90)])
-def test_gpu_a2b_ord4_strips_and_segments(n, nz, cube_tiles):
+@pytest.mark.parametrize("cube_tiles,n,nz", [
+    (c, n, nz) for c in (False, True) for n, nz in
+    [(4, 3), (5, 3), (6, 4), (7, 3), (57, 3), (58, 3), (59, 3), (60, 3), (24, 90)]] + [
+    (True, 4, 600), (True, 5, 600), (True, 7, 600), (True, 57, 150), (True, 58, 150),
+    (True, 59, 75), (True, 60, 75), (False, 5, 3600)])
+def test_gpu_a2b_ord4_strips_and_segments(cube_tiles, n, nz):
     from fv3core_amd.stencils.a2b_ord4 import AGrid2BGridFourthOrder
 
     case = Case(n, nz, cube_tiles, seed=33 + n)
