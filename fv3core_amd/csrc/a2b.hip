@@ -543,7 +543,8 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
     FV3_HIP_CHECK_LAUNCH(who);
     return FV3_OK;
   }
-  return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, 5, interp, who, FV3_AB_TJ);
+  const StripCost cost{0.65, 0.28, 0.75, 0.37, false, 5, 4.0, 3, FV3_AB_TJ};
+  return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, cost, interp, who);
 }
 
 template int launch_a2b_ord4<double>(hipStream_t, const fv3_domain*, const Met<double>&,

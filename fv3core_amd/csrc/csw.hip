@@ -76,6 +76,20 @@ __device__ __forceinline__ T contravariant(T v1, T v2, T cosa, T rsin2) {
   return (v1 - v2 * cosa) * rsin2;
 }
 
+// The marches' cost, measured on the launches alone: rows per segment of c_sw and
+// of d2a2c_vect on 12 to 128 cells a side, one to 96 tiles.  By the del-n march's
+// figures six C12 tiles, 79 levels, took 53.2 us in FP64 and 39.6 in FP32, six
+// C24 71.8 and 50.9; by these 46.8 and 36.9, 65.5 and 48.5.  Above three waves
+// the heights differ little.
+inline StripCost csw_cost(bool fp32) {
+  return fp32 ? StripCost{0.62, 0.27, 0.75, 0.37, true, 2, 3.5, 2, 33}
+              : StripCost{0.7, 0.53, 1.2, 0.52, true, 2, 3.5, 2, 33};
+}
+inline StripCost d2a2c_cost(bool fp32) {
+  return fp32 ? StripCost{0.62, 0.27, 0.75, 0.37, true, 3, 3.5, 2, 33}
+              : StripCost{0.78, 0.39, 1.0, 0.44, true, 3, 3.5, 2, 33};
+}
+
 // ---------------------------------------------------------------- d2a2c_vect
 // set_tmps, lagrange_interpolation_y_p1/x_p1, avg_box, contravariant_components,
 // ut_main + east_west_edges, north_south_edges + vt_main and, when geo != 0,
@@ -263,7 +277,8 @@ int run_d2a2c(hipStream_t s, const fv3_domain* dom, const Met<T>& m, int geo, T 
               T* vc, const T* u, const T* v, T* ua, T* va, T* utc, T* vtc, const char* who) {
   const Dom d = to_dom(dom);
   const D2A2C<T> f{d2a2c_bounds(dom), m, geo, dt2, u, v, ua, va, uc, vc, utc, vtc};
-  return launch_strips(s, d, d.isc - 2, d.iec + 2, d.jsc - 2, d.jec + 3, 60, 3, f, who);
+  return launch_strips(s, d, d.isc - 2, d.iec + 2, d.jsc - 2, d.jec + 3, 60,
+                       d2a2c_cost(sizeof(T) == 4), f, who);
 }
 
 // ----------------------------------------------------------------------- c_sw
@@ -606,10 +621,11 @@ int run_c_sw(const fv3_domain* dom, const fv3_metrics* g, int32_t nord, T dt2, T
   const CswTransport<T> transport{m,  dt2, delp, pt, w,     ut,  vt, ua, va,
                                   uc0, vc0, u,   v,  delpc, ptc, omga, ke,
                                   nord > 0 ? divgd : nullptr};
-  rc = launch_strips(s, d, d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3, 62, 2, transport, who);
+  const StripCost cost = csw_cost(sizeof(T) == 4);
+  rc = launch_strips(s, d, d.isc - 3, d.iec + 3, d.jsc - 3, d.jec + 3, 62, cost, transport, who);
   if (rc) return rc;
   const CswUpdate<T> update{m, dt2, uc0, vc0, ke, u, v, uc, vc};
-  return launch_strips(s, d, d.isc - 1, d.iec + 2, d.jsc - 1, d.jec + 2, 62, 2, update, who);
+  return launch_strips(s, d, d.isc - 1, d.iec + 2, d.jsc - 1, d.jec + 2, 62, cost, update, who);
 }
 
 }  // namespace
@@ -617,6 +633,14 @@ int run_c_sw(const fv3_domain* dom, const fv3_metrics* g, int32_t nord, T dt2, T
 }  // namespace fv3
 
 extern "C" {
+
+int32_t fv3_plan_c_sw_rows(int32_t rows, int64_t planes, int32_t fp32) {
+  return fv3::strip_segment_rows(rows, planes, fv3::csw_cost(fp32 != 0));
+}
+
+int32_t fv3_plan_d2a2c_rows(int32_t rows, int64_t planes, int32_t fp32) {
+  return fv3::strip_segment_rows(rows, planes, fv3::d2a2c_cost(fp32 != 0));
+}
 
 int32_t fv3_d2a2c_vect_f64(const fv3_domain* dom, const fv3_metrics* g, double* uc, double* vc,
                            const double* u, const double* v, double* ua, double* va,

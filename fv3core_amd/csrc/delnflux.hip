@@ -2,28 +2,25 @@
 // as, the caller's fluxes.
 #include "delnflux.hpp"
 
+#include <cmath>
+
 namespace fv3 {
 
-// Measured on the del-n march in the acoustic call (FP64, two extra passes, 6
-// rows beside a segment's own): a step takes 0.65 us plus 0.28 us per wave on a
-// SIMD up to three waves, about 0.75 us plus 0.37 us per wave above that, and a
-// launch adds about four steps; the segment count with the least time by these
-// figures is taken, of heights up to DN_TJ rows where there are more than
-// three waves (96 C48 tiles in FP32: one 49-row segment 266 us, two of 25 rows
-// 230 us).
-int strip_segment_rows(int rows, int extra, int64_t planes) {
+int strip_segment_rows(int rows, int64_t planes, const StripCost& cost) {
   int best = 0;
   double least = 0.0;
   for (int nb = 1; nb <= rows; ++nb) {
     const int seg = (rows + nb - 1) / nb;
     const double w = (double)planes * ((rows + seg - 1) / seg) / kSimdsPerGpu;
-    if (w > 3.0 && seg > FV3_DN_TJ) continue;
-    const double t = (w <= 3.0 ? 0.65 + 0.28 * w : 0.75 + 0.37 * w) * (seg + extra + 4);
+    if (w > 3.0 && seg > cost.most) continue;
+    const double n = cost.whole ? std::ceil(w) : w;
+    const double step = w <= 3.0 ? cost.lone + cost.wave * n : cost.lone3 + cost.wave3 * n;
+    const double t = step * (seg + cost.extra + cost.lead);
     if (best == 0 || t < least) {
       best = seg;
       least = t;
     }
-    if (seg <= 3) break;
+    if (seg <= cost.least) break;
   }
   return best;
 }
@@ -102,6 +99,12 @@ static int delnflux_launch(const fv3_domain* dom, int mode, const int32_t* nord4
 }  // namespace fv3
 
 extern "C" {
+
+int32_t fv3_plan_delnflux_rows(int32_t rows, int64_t planes, int32_t fp32, int32_t most) {
+  fv3::StripCost cost = fv3::deln_cost(fp32 != 0);
+  if (most > 0) cost.most = most;
+  return fv3::strip_segment_rows(rows, planes, cost);
+}
 
 int32_t fv3_delnflux_f64(const fv3_domain* d, int32_t mode, const int32_t nord4[4],
                          const double* q, const double* mass, const double* damp,

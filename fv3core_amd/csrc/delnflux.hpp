@@ -40,6 +40,17 @@ constexpr int DN_TI = DN_W - 6;     // interfaces per strip in i
 constexpr int DN_NY = FV3_DN_NY;    // strips (waves) per workgroup
 constexpr int DN_WIN = 100;         // cells of a corner window (at most 10 x 10)
 
+// The march's cost.  FP64 (two extra passes) measured in the acoustic call, FP32
+// on the launch alone: [1, 1, 1, 1] on six C48 tiles, 79 levels, 19.4 us by the
+// FP64 figures, 17.4 by its own (17.7 in LDS blocks); six C128 72.2 and 60.7; in
+// the mixed acoustic call on 96 C48 tiles the same.  Segments of more than 33
+// rows where there are more than three waves measured slower (96 C48 tiles in
+// FP32: one 49-row segment 266 us, two of 25 rows 230 us).
+inline StripCost deln_cost(bool fp32) {
+  return fp32 ? StripCost{0.62, 0.18, 0.62, 0.18, true, 6, 4.0, 3, FV3_DN_TJ}
+              : StripCost{0.65, 0.28, 0.75, 0.37, false, 6, 4.0, 3, FV3_DN_TJ};
+}
+
 // Launch-wide arguments of the passes.
 template <typename T>
 struct DelnArgs {
@@ -345,7 +356,7 @@ int deln_launch(const fv3_domain* dom, const int32_t* nord4, int use_damp, const
     a.wi = d.ie - d.is + 1 < 4 ? 1 : 2;
     a.wj = d.je - d.js + 1 < 4 ? 1 : 2;
   }
-  a.seg = strip_segment_rows(nfj, 6, (int64_t)a.nbi * d.nk * d.ntiles);
+  a.seg = strip_segment_rows(nfj, (int64_t)a.nbi * d.nk * d.ntiles, deln_cost(sizeof(T) == 4));
   a.nbj = (nfj + a.seg - 1) / a.seg;
   const int64_t total = (int64_t)(a.nbi * a.nbj + a.wi * a.wj) * d.nk * d.ntiles;
   FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);

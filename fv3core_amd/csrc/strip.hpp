@@ -129,17 +129,31 @@ __global__ void __launch_bounds__(64 * NW) strip_kernel(Dom d, StripPlan p, F bo
   body(d, p.i0 + within % p.nbi * p.width, j, min(p.seg, p.j1 + 1 - j), plane % d.nk, plane / d.nk);
 }
 
-// Rows per segment of a march of `extra` rows beside its own, over `rows` rows
-// of `planes` strips.
-int strip_segment_rows(int rows, int extra, int64_t planes);
+// What a march costs, for the choice of its segments: a step takes lone us plus
+// wave us for each wave on its SIMD up to three, lone3 plus wave3 above that
+// (whole waves where `whole`); a segment marches its rows, `extra` rows beside
+// them and `lead` steps' worth of launch and first loads.  No more segments are
+// tried once they have `least` rows, and where a SIMD has more than three waves
+// they are at most `most` rows.
+struct StripCost {
+  double lone, wave, lone3, wave3;
+  bool whole;
+  int extra;
+  double lead;
+  int least, most;
+};
+
+// Rows per segment over `rows` rows of `planes` strips: the segment count with
+// the least time by the march's cost.
+int strip_segment_rows(int rows, int64_t planes, const StripCost& cost);
 
 // Strips over columns [i0, i1] and rows [j0, j1] of every level and tile, in
-// segments of at most `most` rows.
+// segments by the march's cost.
 template <int NW = 4, typename F>
 inline int launch_strips(hipStream_t s, const Dom& d, int i0, int i1, int j0, int j1, int width,
-                         int extra, const F& body, const char* who, int most = 1 << 30) {
+                         const StripCost& cost, const F& body, const char* who) {
   StripPlan p{i0, j0, j1, width, (i1 - i0 + width) / width, 1, j1 - j0 + 1};
-  p.seg = std::min(most, strip_segment_rows(p.seg, extra, (int64_t)p.nbi * d.nk * d.ntiles));
+  p.seg = strip_segment_rows(p.seg, (int64_t)p.nbi * d.nk * d.ntiles, cost);
   p.nbj = (j1 - j0 + p.seg) / p.seg;
   const int64_t total = (int64_t)p.nbi * p.nbj * d.nk * d.ntiles;
   FV3_REQUIRE(total < (int64_t)1 << 30, FV3_E_ARG, "%s: grid too large", who);
