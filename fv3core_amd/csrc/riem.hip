@@ -477,16 +477,22 @@ static double riem_levels_us(int lv, int nz, int64_t waves, bool c) {
 }
 
 // The form with the least time: one thread per column (0), or 5 or 8 levels a
-// thread.  Few layers and launches of one full round of columns take the
-// column form (RiemannSolverC on six C96 tiles, 79 layers: 242 against 261 us;
-// 4 layers: 17 against 22 us), which spreads nothing where every SIMD already
-// has a wave; 100 layers on six C128 tiles 722 against 887 us, since 8 levels
-// a thread leave one workgroup to a CU.  Below half a workgroup a CU the
-// levels' latency alone counts.
+// thread.  Few layers take the column form (RiemannSolverC on six C96 tiles, 4
+// layers: 17 against 22 us), as do layer counts that fill the levels' waves
+// badly on many columns (50 layers: 147 against 200 us) and those above 80,
+// where 8 levels a thread leave one workgroup to a CU (100 layers on six C128
+// tiles: 722 against 887 us).  Below half a workgroup a CU the levels' latency
+// alone counts.  The rates are those of calls alone; inside the acoustic call,
+// among a gigabyte of other fields, RiemannSolverC's column form, which reads its
+// inputs in six sweeps, takes more (79 layers, six C96 tiles: 236 us alone and
+// 285 us there, 5 levels a thread 258 and 259 us), hence kColumnInCall between
+// the few layers that fit the caches and the many where 8 levels lose by more.
+constexpr double kColumnInCall = 1.16;
 static int riem_form(int nz, int64_t waves, bool c, bool fp32) {
   if (waves >= 100 && nz <= (waves < 500 ? 4 : fp32 ? 7 : 6)) return 0;
   if (waves <= 128) return nz <= 80 ? 5 : 8;
-  const double t0 = riem_column_us(nz, waves, c, fp32);
+  const double t0 = riem_column_us(nz, waves, c, fp32) *
+                    (c && nz > 16 && nz <= 80 ? kColumnInCall : 1.0);
   const double t5 = riem_levels_us(5, nz, waves, c), t8 = riem_levels_us(8, nz, waves, c);
   if (t0 <= t5 && t0 <= t8) return 0;
   return t5 <= t8 ? 5 : 8;

@@ -189,7 +189,7 @@ COLUMN = 0  # the other forms of the Riemann solvers go by the levels a thread h
 # Every pair of forms: few layers, 16 layers (one wave of 8 levels a thread), a
 # full round of columns, above the reach of 5 levels a thread.
 @pytest.mark.parametrize("solver_c,nz,tiles,whole_form,part_form", [
-    (True, 4, 8, COLUMN, 5), (True, 16, 16, 8, 5), (True, 79, 56, COLUMN, 5),
+    (True, 4, 8, COLUMN, 5), (True, 16, 16, 8, 5), (True, 50, 56, COLUMN, 5),
     (True, 90, 40, COLUMN, 8), (False, 4, 8, COLUMN, 5), (False, 16, 16, 8, 5),
     (False, 64, 16, 8, 5), (False, 90, 40, COLUMN, 8)])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
