@@ -333,7 +333,11 @@ enum MapForm { kMapSweeps = 0, kMapFused = 1, kMapLayers = 2 };
 // longer dependent chain: it wins where two waves a SIMD cover the chain, or
 // where the nine column arrays of the sweeps (from 280 MB) do not fit the last-level
 // cache (137 layers, six C128 tiles: 531 against 597 us; 96 C48 tiles 1204
-// against 1698 us).  In FP32 the lines lie where its own times put them.
+// against 1698 us).  In FP32 the lines lie where its own times put them.  The
+// rates are those of calls on data that the last one left in the caches; on cold
+// data the one-thread forms, which read a column four times, take 5 to 25 % more
+// and the spread form the same, hence kColumnCold.
+constexpr double kColumnCold = 1.15;
 static MapForm map_form(int km, int64_t waves, bool fp32) {
   const double w = (double)waves;
   const bool fused = waves >= 2 * kSimdsPerGpu ||
@@ -343,7 +347,11 @@ static MapForm map_form(int km, int64_t waves, bool fp32) {
   double layers, busy;
   if (km <= 80) {
     const double n = (km + 19) / 20;  // waves of a workgroup
-    layers = fp32 ? std::max(14.4, 11.0 + 0.0175 * n * w) : std::max(15.0, 12.0 + 0.030 * n * w);
+    if (n == 1)
+      layers = fp32 ? 8.0 + 0.0175 * w : 6.0 + 0.034 * w;
+    else
+      layers = fp32 ? 11.0 + 0.0175 * n * w : 12.0 + 0.030 * n * w;
+    layers = std::max(fp32 ? 14.4 : 15.3, layers);
   } else {
     layers = fp32 ? 18.0 + 0.134 * w : 20.0 + 0.272 * w;
   }
@@ -353,7 +361,7 @@ static MapForm map_form(int km, int64_t waves, bool fp32) {
   else
     busy = fp32 ? 0.35 + 0.0013 * w : 0.7 + 0.0021 * w;
   const double lone = fp32 ? std::min(1.75, 1.35 + 0.008 * w) : std::min(2.3, 1.5 + 0.01 * w);
-  return 3.0 + km * std::max(lone, busy) < layers ? column : kMapLayers;
+  return kColumnCold * (3.0 + km * std::max(lone, busy)) < layers ? column : kMapLayers;
 }
 
 template <typename T>
