@@ -10,6 +10,8 @@
 // and dyn_core.py:47-145.  Vertical recurrences run one column per lane.
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace fv3 {
 
 namespace {
@@ -61,19 +63,33 @@ constexpr int KC = 8;
 // 79 layers, C-grid and D-grid heights: six C12 tiles 66 -> 19 us and 36 -> 14
 // us, six C96 tiles 83 -> 63 us and 78 -> 78 us, 96 C48 tiles mixed 221 -> 201
 // us and 346 -> 282 us.  Sixteen waves leave one workgroup to a CU (C96: 79 and
-// 90 us).
-constexpr int HW = 8;   // waves per workgroup
-constexpr int HK = 80;  // levels per chunk
+// 90 us).  The chunk is as high as the column and the waves as many as its
+// levels occupy, so that few levels on many columns fill the chip as one thread
+// per column did (C-grid, six C128 tiles: 4 layers, one thread per column 17.1
+// us, always eight waves and 80 levels 20.0, these 16.5; 10 layers 25.6, 28.2 and
+// 24.2).
+constexpr int HW = 8;   // most waves per workgroup
+constexpr int HK = 80;  // most levels per chunk
 
+// waves of a workgroup on nk levels: the fewest that HW waves do not outrun
+inline int floor_waves(int nk) {
+  const int each = (nk + HW - 1) / HW;
+  return (nk + each - 1) / each;
+}
+// bytes of a workgroup's chunk
+inline size_t floor_lds(int nk) { return (size_t)std::min(nk, HK) * 64 * sizeof(double); }
+
+// h: min(nk, HK) levels
 template <typename T, typename F>
-__device__ __forceinline__ T floor_columns(T (&h)[HK][64], int nk, int64_t sk, T* out, bool keep,
+__device__ __forceinline__ T floor_columns(T (*h)[64], int nk, int64_t sk, T* out, bool keep,
                                            F value) {
   const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int nw = (int)blockDim.y;
   T above = T(0), bottom = T(0);
   for (int k1 = nk; k1 > 0; k1 -= HK) {
     const int k0 = max(k1 - HK, 0);
 #pragma unroll 2
-    for (int k = k0 + wave; k < k1; k += HW) h[k - k0][lane] = value(k);
+    for (int k = k0 + wave; k < k1; k += nw) h[k - k0][lane] = value(k);
     __syncthreads();
     if (wave == 0) {
       for (int k = k1 - 1; k >= k0; k -= KC) {
@@ -96,7 +112,7 @@ __device__ __forceinline__ T floor_columns(T (&h)[HK][64], int nk, int64_t sk, T
     }
     __syncthreads();
     if (keep)
-      for (int k = k0 + wave; k < k1; k += HW) out[(int64_t)k * sk] = h[k - k0][lane];
+      for (int k = k0 + wave; k < k1; k += nw) out[(int64_t)k * sk] = h[k - k0][lane];
     if (k0 > 0) __syncthreads();
   }
   return bottom;
@@ -114,7 +130,8 @@ __global__ void __launch_bounds__(64 * HW)
                        const T* __restrict__ area, const U* __restrict__ ut,
                        const U* __restrict__ vt, const T* __restrict__ gz, T* __restrict__ gzn,
                        T* __restrict__ ws, T rdt) {
-  __shared__ T h[HK][64];
+  extern __shared__ double chunk[];
+  T(*const h)[64] = (T(*)[64])chunk;
   const int ni = d.iec - d.isc + 3, nj = d.jec - d.jsc + 3;
   const int n0 = (int)(blockIdx.x * 64 + threadIdx.x);
   const bool keep = n0 < ni * nj;
@@ -228,7 +245,8 @@ __global__ void __launch_bounds__(64 * HW)
                         const T* __restrict__ xfx, const T* __restrict__ yfx,
                         const T* __restrict__ gxd, const T* __restrict__ gyd, T* __restrict__ ws,
                         T dt) {
-  __shared__ T lds[HK][64];
+  extern __shared__ double chunk[];
+  T(*const lds)[64] = (T(*)[64])chunk;
   const int ni = d.iec - d.isc + 1, nj = d.jec - d.jsc + 1;
   const int n0 = (int)(blockIdx.x * 64 + threadIdx.x);
   const bool keep = n0 < ni * nj;
@@ -678,7 +696,8 @@ int update_dz_c(const fv3_domain* dom, const double* area, const double* zs,
   hipStream_t s = as_stream(stream);
   const int ncol = (d.iec - d.isc + 3) * (d.jec - d.jsc + 3);
   hipLaunchKernelGGL((update_dz_c_kernel<double, U>), dim3((ncol + 63) / 64, d.ntiles),
-                     dim3(64, HW), 0, s, d, dp_ref, zs, area, ut, vt, gz, work, ws, 1.0 / dt);
+                     dim3(64, floor_waves(dom->nk)), floor_lds(dom->nk), s, d, dp_ref, zs,
+                     area, ut, vt, gz, work, ws, 1.0 / dt);
   FV3_HIP_CHECK_LAUNCH(who);
   const Box bx{d.isc - 1, d.iec + 1, d.jsc - 1, d.jec + 1};
   const double* src = work;
@@ -734,8 +753,9 @@ int update_dz_d(const fv3_domain* dom, const fv3_metrics* g, int32_t hord_tm,
                         static_cast<const double*>(g->rarea), gxd, gyd, stream);
   if (rc) return rc;
   const int nc = (d.iec - d.isc + 1) * (d.jec - d.jsc + 1);
-  hipLaunchKernelGGL((apply_height_kernel<double>), dim3((nc + 63) / 64, d.ntiles), dim3(64, HW), 0,
-                     s, d, area, zs, height, fx, fy, xfx_i, yfx_i, gxd, gyd, ws, dt);
+  hipLaunchKernelGGL((apply_height_kernel<double>), dim3((nc + 63) / 64, d.ntiles),
+                     dim3(64, floor_waves(dom->nk)), floor_lds(dom->nk), s, d, area, zs, height,
+                     fx, fy, xfx_i, yfx_i, gxd, gyd, ws, dt);
   FV3_HIP_CHECK_LAUNCH(who);
   return FV3_OK;
 }

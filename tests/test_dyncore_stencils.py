@@ -208,11 +208,12 @@ def test_gpu_update_dz_c_and_d(cube_tiles):
         assert_close(ws2g[c], ws2r[c], 1e-10, near_zero=1e-10, what=f"tile {ti} ws (d)")
 
 
-# Interface counts of one level per wave, at the edges of a chunk of 80 and past
+# Interface counts of one level per wave and of two and three, at the edges of a chunk of 80 and past
 # two of them, layers thin enough for the floor to run through whole columns,
 # column counts beside a workgroup's 64.
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,nz", [(6, 4), (6, 8), (8, 79), (7, 80), (6, 81), (5, 162)])
+@pytest.mark.parametrize("n,nz", [(6, 3), (6, 4), (6, 8), (6, 16), (8, 79), (7, 80), (6, 81),
+                                  (5, 162)])
 def test_gpu_update_dz_level_chunks(n, nz):
     from fv3core_amd.stencils.updatedzc import UpdateGeopotentialHeightOnCGrid
     from fv3core_amd.stencils.updatedzd import UpdateHeightOnDGrid
