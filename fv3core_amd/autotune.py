@@ -1,18 +1,22 @@
-"""Offline tile-shape autotuner for the LDS-tiled stencil kernels.
+"""Offline shape autotuner for the del-n and a2b_ord4 row marches.
 
-The workgroup shapes of ``delnflux_kernel`` and ``a2b_interp_kernel`` are
-macros in ``csrc/tile_config.hpp``.  A shape only changes how the work is
+A march runs strips of columns in segments of rows, one wave to a segment.
+The segments follow from the launch's size by the march's cost
+(``csrc/strip.hpp``); the most rows a segment may have where a SIMD holds more
+than three waves, and the waves per workgroup, are macros in
+``csrc/tile_config.hpp``.  A shape only changes how the work is
 split, never the arithmetic, so every candidate returns the same bits; the
 tuner picks the fastest on the GPU it runs on:
 
-1. ``build``: for each candidate, compile the kernel's source with the
-   shape's ``-D`` flags and link it with the other objects of the in-tree
-   build into ``_tune/lib_<kernel>_<a>_<b>.so`` (CPU only: hipcc
+1. ``build``: for each candidate, compile every source that holds the kernel
+   with the shape's ``-D`` flags and link them with the other objects of the
+   in-tree build into ``_tune/lib_<kernel>_<a>_<b>.so`` (CPU only: hipcc
    cross-compiles for gfx950).
 2. ``measure``: run a benchmark workload once per library, each in its own
    process, timing the kernel with the library's HIP-event hooks
    (``bench.py --roofline-kernel <kernel>``), and write the mean launch
-   times to ``_tune/results.json``.  ``--workload ensemble`` (the default)
+   times to ``_tune/results.json``.  Candidates that split the workload's
+   launches as another does are left out.  ``--workload ensemble`` (the default)
    times the launches of the 32-member C48 batch in the mixed form;
    ``--workload dyncore`` those of the FP64 acoustic step on six C96 tiles.
 3. ``apply``: rewrite the defaults in ``tile_config.hpp`` with the fastest
@@ -25,6 +29,7 @@ tuner picks the fastest on the GPU it runs on:
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import pathlib
 import re
@@ -32,6 +37,7 @@ import subprocess
 import sys
 from typing import Dict, List, Tuple
 
+from . import _lib
 from . import build as _build
 
 HERE = pathlib.Path(__file__).resolve().parent
@@ -39,13 +45,60 @@ TUNE_DIR = HERE / "_tune"
 CONFIG = _build.CSRC / "tile_config.hpp"
 REPO = HERE.parent
 
-# kernel -> (source, timing name, macro names, candidate (rows, waves) pairs)
+# kernel -> (file that reads the macros, timing name, macro names, candidate
+# (most rows, waves) pairs)
 KERNELS: Dict[str, Tuple[str, str, Tuple[str, str], List[Tuple[int, int]]]] = {
-    "delnflux": ("delnflux.hip", "delnflux_kernel", ("FV3_DN_TJ", "FV3_DN_NY"),
+    "delnflux": ("delnflux.hpp", "delnflux_kernel", ("FV3_DN_TJ", "FV3_DN_NY"),
                  [(17, 4), (25, 4), (33, 1), (33, 2), (33, 4), (33, 8), (49, 4)]),
     "a2b": ("a2b.hip", "a2b_interp_kernel", ("FV3_AB_TJ", "FV3_AB_NY"),
             [(11, 4), (19, 4), (33, 1), (33, 2), (33, 4), (49, 4), (97, 4)]),
 }
+
+
+# workload -> its launches of the kernels: (cells a side, tiles, levels, FP32)
+_LAUNCHES = {"ensemble": [(48, 192, 79, True), (48, 192, 80, False)],
+             "dyncore": [(96, 6, 79, False), (96, 6, 80, False)]}
+
+
+def sources(kernel: str) -> List[pathlib.Path]:
+    """The HIP sources that compile the kernel: the file itself or its includers."""
+    name = KERNELS[kernel][0]
+    if name.endswith(".hip"):
+        return [_build.CSRC / name]
+    return [s for s in sorted(_build.CSRC.glob("*.hip")) if f'#include "{name}"' in s.read_text()]
+
+
+def default_shape(kernel: str) -> Tuple[int, int]:
+    text = CONFIG.read_text()
+    rows, waves = (int(re.search(rf"#define {m} (\d+)", text).group(1))
+                   for m in KERNELS[kernel][2])
+    return rows, waves
+
+
+def plan(kernel: str, shape: Tuple[int, int], workload: str) -> tuple:
+    """How the shape splits the workload's launches: their segment rows, and the waves."""
+    lib = _lib.lib()
+    segments = []
+    for n, tiles, levels, fp32 in _LAUNCHES[workload]:
+        if kernel == "delnflux":  # interfaces, 58 a strip
+            rows = n + 1
+            planes = -(-rows // 58) * levels * tiles
+            segments.append(lib.fv3_plan_delnflux_rows(rows, ctypes.c_int64(planes), int(fp32),
+                                                       shape[0]))
+        else:  # the corners off the tile edges
+            rows = n - 1
+            planes = -(-rows // 58) * levels * tiles
+            segments.append(lib.fv3_plan_a2b_rows(rows, ctypes.c_int64(planes), shape[0]))
+    return tuple(segments) + (shape[1],)
+
+
+def distinct_shapes(kernel: str, workload: str) -> List[Tuple[int, int]]:
+    """The candidates whose plans differ on the workload, the default before the others."""
+    shapes, first = KERNELS[kernel][3], default_shape(kernel)
+    kept = {}
+    for shape in sorted(shapes, key=lambda s: s != first):
+        kept.setdefault(plan(kernel, shape, workload), shape)
+    return [s for s in shapes if s in kept.values()]
 
 
 def variant_lib(kernel: str, shape: Tuple[int, int]) -> pathlib.Path:
@@ -59,23 +112,30 @@ def build_variants(kernels=None) -> List[pathlib.Path]:
     TUNE_DIR.mkdir(exist_ok=True)
     made = []
     for kernel in kernels or KERNELS:
-        src, _, macros, shapes = KERNELS[kernel]
-        others = [str(o) for o in sorted(objdir.glob("*.o")) if o.stem != pathlib.Path(src).stem]
+        _, _, macros, shapes = KERNELS[kernel]
+        srcs = sources(kernel)
+        others = [str(o) for o in sorted(objdir.glob("*.o"))
+                  if o.stem not in [s.stem for s in srcs]]
         for shape in shapes:
-            obj = TUNE_DIR / f"{kernel}_{shape[0]}_{shape[1]}.o"
             defs = [f"-D{macros[0]}={shape[0]}", f"-D{macros[1]}={shape[1]}"]
-            cmd = [_build.hipcc()] + _build.COMMON_FLAGS + defs + ["-c", str(_build.CSRC / src),
-                                                                 "-o", str(obj)]
-            res = subprocess.run(cmd, capture_output=True, text=True)
-            if res.returncode != 0:
-                raise RuntimeError(f"hipcc failed for {kernel} {shape}:\n{res.stderr}")
+            objs = []
+            for src in srcs:
+                obj = TUNE_DIR / f"{src.stem}_{shape[0]}_{shape[1]}.o"
+                cmd = [_build.hipcc()] + _build.COMMON_FLAGS + defs + ["-c", str(src),
+                                                                     "-o", str(obj)]
+                res = subprocess.run(cmd, capture_output=True, text=True)
+                if res.returncode != 0:
+                    raise RuntimeError(f"hipcc failed for {kernel} {shape}:\n{res.stderr}")
+                objs.append(obj)
             out = variant_lib(kernel, shape)
             res = subprocess.run([_build.hipcc(), "-shared", "-fPIC",
                                   f"--offload-arch={_build.OFFLOAD_ARCH}"] + others +
-                                 [str(obj), "-o", str(out)], capture_output=True, text=True)
+                                 [str(o) for o in objs] + ["-o", str(out)],
+                                 capture_output=True, text=True)
             if res.returncode != 0:
                 raise RuntimeError(f"link failed for {kernel} {shape}:\n{res.stderr}")
-            obj.unlink()
+            for obj in objs:
+                obj.unlink()
             made.append(out)
     return made
 
@@ -102,8 +162,8 @@ def measure(kernels=None, steps: int = 3, timeout: int = 300,
         raise ValueError(f"unknown workload {workload}")
     results = {}
     for kernel in kernels or KERNELS:
-        _, name, _, shapes = KERNELS[kernel]
-        for shape in shapes:
+        name = KERNELS[kernel][1]
+        for shape in distinct_shapes(kernel, workload):
             lib = variant_lib(kernel, shape)
             if not lib.exists():
                 raise FileNotFoundError(f"{lib} is missing: run the build step first")

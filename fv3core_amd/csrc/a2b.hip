@@ -342,6 +342,9 @@ struct A2BInterp {
 // C12 tile 13.7 and 16.3 us, six 15.2 and 21.0, six C48 29.4 and 32.3, six C96
 // 64.0 and 61.3, 96 C48 274 and 208 us.
 constexpr int64_t kA2BMarchBlocks = 3500;
+// The march's cost is the del-n march's (delnflux.hpp), with five rows beside a
+// segment's own.
+constexpr StripCost kA2BCost{0.65, 0.28, 0.75, 0.37, false, 5, 4.0, 3, FV3_AB_TJ};
 constexpr int AB_W = 64;         // LDS columns = TI + 6
 constexpr int AB_TI = AB_W - 6;  // corners per block in i
 constexpr int AB_TJ = 16;        // corners per block in j
@@ -543,8 +546,7 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
     FV3_HIP_CHECK_LAUNCH(who);
     return FV3_OK;
   }
-  const StripCost cost{0.65, 0.28, 0.75, 0.37, false, 5, 4.0, 3, FV3_AB_TJ};
-  return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, cost, interp, who);
+  return launch_strips<FV3_AB_NY>(s, dk, is2, ie1, js2, je1, 58, kA2BCost, interp, who);
 }
 
 template int launch_a2b_ord4<double>(hipStream_t, const fv3_domain*, const Met<double>&,
@@ -561,6 +563,12 @@ int check_a2b_metrics(const fv3_metrics* g, const char* who) {
 }
 
 }  // namespace fv3
+
+extern "C" int32_t fv3_plan_a2b_rows(int32_t rows, int64_t planes, int32_t most) {
+  fv3::StripCost cost = fv3::kA2BCost;
+  if (most > 0) cost.most = most;
+  return fv3::strip_segment_rows(rows, planes, cost);
+}
 
 extern "C" int32_t fv3_a2b_ord4_f64(const fv3_domain* dom, const fv3_metrics* g, int32_t replace,
                                     double* qin, double* qout, double* work, int64_t work_slab,

@@ -1,5 +1,7 @@
 """The tile-shape autotuner's host logic (no GPU): candidate bookkeeping and
 the rewrite of tile_config.hpp."""
+import pytest
+
 from fv3core_amd import autotune
 
 
@@ -32,3 +34,25 @@ def test_best_shape_is_the_fastest_and_rewrite_touches_only_its_macros():
 def _default(text, macro):
     import re
     return int(re.search(rf"#define {macro} (\d+)", text).group(1))
+
+
+@pytest.mark.parametrize("kernel", sorted(autotune.KERNELS))
+def test_every_source_of_the_kernel_is_rebuilt(kernel):
+    macros = autotune.KERNELS[kernel][2]
+    csrc = autotune._build.CSRC
+    readers = {p.name for p in csrc.iterdir() if p.suffix in (".hip", ".hpp")
+               and p.name != "tile_config.hpp" and any(m in p.read_text() for m in macros)}
+    reached = {s.name for s in csrc.glob("*.hip")
+               if s.name in readers or any(f'#include "{r}"' in s.read_text() for r in readers)}
+    assert {s.name for s in autotune.sources(kernel)} == reached
+
+
+@pytest.mark.parametrize("workload", sorted(autotune._WORKLOAD_ARGS))
+@pytest.mark.parametrize("kernel", sorted(autotune.KERNELS))
+def test_timed_candidates_split_the_workload_differently(kernel, workload):
+    shapes = autotune.distinct_shapes(kernel, workload)
+    plans = [autotune.plan(kernel, s, workload) for s in shapes]
+    assert len(set(plans)) == len(plans)
+    assert autotune.default_shape(kernel) in shapes
+    for s in autotune.KERNELS[kernel][3]:  # what is left out is a plan that is timed
+        assert autotune.plan(kernel, s, workload) in plans
