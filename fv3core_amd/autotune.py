@@ -2,8 +2,8 @@
 
 A march runs strips of columns in segments of rows, one wave to a segment.
 The segments follow from the launch's size by the march's cost
-(``csrc/strip.hpp``); the most rows a segment may have where a SIMD holds more
-than three waves, and the waves per workgroup, are macros in
+(``csrc/strip.hpp``); the most rows a segment may have (del-n: where a SIMD
+holds more than three waves), and the waves per workgroup, are macros in
 ``csrc/tile_config.hpp``.  A shape only changes how the work is
 split, never the arithmetic, so every candidate returns the same bits; the
 tuner picks the fastest on the GPU it runs on:

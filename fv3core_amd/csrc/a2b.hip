@@ -343,8 +343,9 @@ struct A2BInterp {
 // 64.0 and 61.3, 96 C48 274 and 208 us.
 constexpr int64_t kA2BMarchBlocks = 3500;
 // The march's cost is the del-n march's (delnflux.hpp), with five rows beside a
-// segment's own.
-constexpr StripCost kA2BCost{0.65, 0.28, 0.75, 0.37, false, 5, 4.0, 3, FV3_AB_TJ};
+// segment's own and the cap on every launch (six C128 tiles, 79 levels, 1.4 waves
+// a SIMD: 64 rows 99.5 us, 32 rows 94.8).
+constexpr StripCost kA2BCost{0.65, 0.28, 0.75, 0.37, false, 5, 4.0, 3, FV3_AB_TJ, 0.0};
 constexpr int AB_W = 64;         // LDS columns = TI + 6
 constexpr int AB_TI = AB_W - 6;  // corners per block in i
 constexpr int AB_TJ = 16;        // corners per block in j

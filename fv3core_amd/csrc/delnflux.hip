@@ -12,7 +12,7 @@ int strip_segment_rows(int rows, int64_t planes, const StripCost& cost) {
   for (int nb = 1; nb <= rows; ++nb) {
     const int seg = (rows + nb - 1) / nb;
     const double w = (double)planes * ((rows + seg - 1) / seg) / kSimdsPerGpu;
-    if (w > 3.0 && seg > cost.most) continue;
+    if (w > cost.free && seg > cost.most) continue;
     const double n = cost.whole ? std::ceil(w) : w;
     const double step = w <= 3.0 ? cost.lone + cost.wave * n : cost.lone3 + cost.wave3 * n;
     const double t = step * (seg + cost.extra + cost.lead);

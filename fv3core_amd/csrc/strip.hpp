@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(64 * NW) strip_kernel(Dom d, StripPlan p, F bo
 // wave us for each wave on its SIMD up to three, lone3 plus wave3 above that
 // (whole waves where `whole`); a segment marches its rows, `extra` rows beside
 // them and `lead` steps' worth of launch and first loads.  No more segments are
-// tried once they have `least` rows, and where a SIMD has more than three waves
+// tried once they have `least` rows, and where a SIMD has more than `free` waves
 // they are at most `most` rows.
 struct StripCost {
   double lone, wave, lone3, wave3;
@@ -141,6 +141,7 @@ struct StripCost {
   int extra;
   double lead;
   int least, most;
+  double free = 3.0;
 };
 
 // Rows per segment over `rows` rows of `planes` strips: the segment count with

@@ -14,8 +14,8 @@
 #define FV3_DN_NY 4
 #endif
 
-// a2b_ord4's march: most corner rows per strip segment in launches of more than
-// three waves a SIMD, strips (waves) per workgroup
+// a2b_ord4's march: most corner rows per strip segment, strips (waves) per
+// workgroup
 #ifndef FV3_AB_TJ
 #define FV3_AB_TJ 33
 #endif

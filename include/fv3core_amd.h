@@ -756,8 +756,8 @@ int32_t fv3_cubed_to_latlon_f64(const fv3_domain* d, int32_t order, const double
  *   fv3_plan_fvtp2d_rows: output rows of a segment of fv_tp_2d's march.
  *   fv3_plan_delnflux_rows, fv3_plan_a2b_rows, fv3_plan_c_sw_rows,
  *   fv3_plan_d2a2c_rows: the same of the del-n march and of those of a2b_ord4 (on
- *     launches that march), c_sw and d2a2c_vect.  most: the cap on the
- *     rows in launches of more than three waves a SIMD, 0 for the built one.
+ *     launches that march), c_sw and d2a2c_vect.  most: the cap on the rows (del-n:
+ *     where a SIMD has more than three waves), 0 for the built one.
  */
 int32_t fv3_plan_map_single(int32_t km, int64_t waves, int32_t fp32);
 int32_t fv3_plan_riem(int32_t nz, int64_t waves, int32_t solver_c, int32_t fp32);

@@ -36,3 +36,16 @@ def test_segments_stay_within_the_rows(march, fp32):
             assert 1 <= seg <= rows
             if planes > 3 * 1024:  # more than three waves a SIMD however they are cut
                 assert seg <= 33
+
+
+@pytest.mark.parametrize("n", [12, 48, 96, 128, 384])
+def test_a2b_segments_keep_the_cap_on_every_launch(n):
+    rows = n - 1
+    planes = -(-rows // 58) * 6 * 79
+    seg = rows_of_a2b(rows, planes, 0)
+    assert 1 <= seg <= 33
+    assert 1 <= rows_of_a2b(rows, planes, 17) <= 17
+
+
+def rows_of_a2b(rows, planes, most):
+    return _lib.lib().fv3_plan_a2b_rows(rows, ctypes.c_int64(planes), most)
