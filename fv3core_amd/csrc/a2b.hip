@@ -496,20 +496,8 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
     const int64_t o2 = at2(d, i, j, t);
     T val;
     const bool ci = i == d.isc || i == d.iec + 1, cj = j == d.jsc || j == d.jec + 1;
-    if (ci && cj) {
-      // _sw_corner at (isc, jsc), _nw_corner at (iec+1, jsc), _ne_corner at
-      // (iec+1, jec+1), _se_corner at (isc, jec+1) (a2b_ord4.py:617-658)
-      const int corner = j == d.jsc ? (i == d.isc ? 0 : 1) : (i == d.iec + 1 ? 2 : 3);
-      T ex[3];
-#pragma unroll
-      for (int tap = 0; tap < 3; ++tap) {
-        const int* tp = kCornerTaps[corner][tap];
-        const T qa = qin[o + tp[0] + (int64_t)tp[1] * d.sj];
-        const T qb = qin[o + tp[2] + (int64_t)tp[3] * d.sj];
-        ex[tap] = qa + cw[t * 12 + corner * 3 + tap] * (qa - qb);
-      }
-      val = (ex[0] + ex[1] + ex[2]) * (T(1) / T(3));
-    } else if (ci && ((i == d.isc && w) || (i == d.iec + 1 && e)) && j >= js2 && j <= je1) {
+    // a corner where the tile has one edge only lies on that edge's line
+    if (ci && ((i == d.isc && w) || (i == d.iec + 1 && e)) && j >= js2 && j <= je1) {
       // qout_x_edge (a2b_ord4.py:313-323): q2 at j and j - 1
       const T* dxa = m.dxa;
       const T q2 = (qin[o - 1] * dxa[o2] + qin[o] * dxa[o2 - 1]) / (dxa[o2 - 1] + dxa[o2]);
@@ -525,6 +513,19 @@ int launch_a2b_ord4(hipStream_t s, const fv3_domain* dom, const Met<T>& m,
                     (dya[o2 - 1 - sj2] + dya[o2 - 1]);
       const T wgt = (j == d.jsc ? m.edge_s : m.edge_n)[o2];
       val = wgt * q1m + (T(1) - wgt) * q1;
+    } else if (ci && cj) {
+      // _sw_corner at (isc, jsc), _nw_corner at (iec+1, jsc), _ne_corner at
+      // (iec+1, jec+1), _se_corner at (isc, jec+1) (a2b_ord4.py:617-658)
+      const int corner = j == d.jsc ? (i == d.isc ? 0 : 1) : (i == d.iec + 1 ? 2 : 3);
+      T ex[3];
+#pragma unroll
+      for (int tap = 0; tap < 3; ++tap) {
+        const int* tp = kCornerTaps[corner][tap];
+        const T qa = qin[o + tp[0] + (int64_t)tp[1] * d.sj];
+        const T qb = qin[o + tp[2] + (int64_t)tp[3] * d.sj];
+        ex[tap] = qa + cw[t * 12 + corner * 3 + tap] * (qa - qb);
+      }
+      val = (ex[0] + ex[1] + ex[2]) * (T(1) / T(3));
     } else {
       return;
     }

@@ -27,15 +27,16 @@ def smooth(rng, shape, mean, amp, modes=(1, 2, 3)):
 
 
 class Case:
-    """A single periodic plane tile (edges off) or the six cube tiles (edges on)."""
+    """A single periodic plane tile (edges off) or the six cube tiles (edges on:
+    all of them, or those of a tuple of south, north, west and east)."""
 
     def __init__(self, n, nz, cube_tiles, seed=0, f=1.0e-4):
         self.n, self.nz, self.cube = n, nz, cube_tiles
         self.ntiles = 6 if cube_tiles else 1
         self.rng = np.random.default_rng(seed)
-        edges = bool(cube_tiles)
-        self.tile = Tile(n, n, 3, edges, edges, edges, edges)
-        self.gi = GridIndexing((n, n, nz), 3, edges, edges, edges, edges)
+        edges = cube_tiles if isinstance(cube_tiles, tuple) else (bool(cube_tiles),) * 4
+        self.tile = Tile(n, n, 3, *edges)
+        self.gi = GridIndexing((n, n, nz), 3, *edges)
         self.factory = StencilFactory(StencilConfig(), self.gi)
         if cube_tiles:
             m = cube.tile_metrics(n)
@@ -83,6 +84,13 @@ class Case:
                 t.copy_(torch.as_tensor(np.stack([m[k] for m in self.metric])))
             fields[k] = t
         return GridData(fields)
+
+
+def to_fp32(case, fields):
+    """fields, and the case's metric terms, with every value rounded to FP32."""
+    r = lambda a: a.astype(np.float32).astype(np.float64)  # noqa: E731
+    case.metric = [{k: r(v) for k, v in m.items()} for m in case.metric]
+    return {k: [r(a) for a in v] for k, v in fields.items()}
 
 
 def oracle_acoustic_call(init, cfg, n, nz, pfull):
