@@ -6,7 +6,7 @@ import torch
 from fv3core_amd.workloads import fill_periodic, plane_metric
 from oracle import csw as ocs
 from oracle.fvtp2d import Tile
-from tests.dyn_helpers import Case
+from tests.dyn_helpers import Case, to_fp32
 from tests.helpers import assert_close
 
 N, NZ = 12, 4
@@ -242,10 +242,13 @@ def test_gpu_c_sw_matches_oracle(cube_tiles, nord):
 # one column past it (60 and 62 columns of n + 4 and n + 6), and batches whose
 # levels take segments of several heights.
 @pytest.mark.gpu
-@pytest.mark.parametrize("cube_tiles", [False, True])
+@pytest.mark.parametrize("cube_tiles", [False, True, (True, False, False, True),
+                                        (False, True, True, True)])
 @pytest.mark.parametrize("n,nz,nord", [(5, 4, 0), (6, 4, 2), (56, 3, 2), (57, 4, 2), (58, 3, 0),
                                        (59, 3, 2), (20, 90, 2)])
-def test_gpu_c_sw_strips_and_segments(n, nz, nord, cube_tiles):
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_gpu_c_sw_strips_and_segments(n, nz, nord, cube_tiles, dtype):
+    from fv3core_amd.mixed import _like, grid_fp32
     from fv3core_amd.stencils.c_sw import CGridShallowWaterDynamics
 
     case = Case(n, nz, cube_tiles, seed=31 + n)
@@ -253,8 +256,11 @@ def test_gpu_c_sw_strips_and_segments(n, nz, nord, cube_tiles):
     names = ("delp", "pt", "u", "v", "w", "uc", "vc", "ua", "va", "ut", "vt", "divgd", "omga")
     ins = dict(zip(names, [case.field(1000.0, 80.0), case.field(300.0, 15.0), u, v,
                            case.field(0.0, 0.8)] + [case.field(0.0, 5.0) for _ in range(8)]))
-    dev = {k: case.dev(a) for k, a in ins.items()}
-    csw = CGridShallowWaterDynamics(case.factory, case.grid_data(), False, 0, nord)
+    grid = case.grid_data()
+    if dtype == torch.float32:
+        ins, grid = to_fp32(case, ins), grid_fp32(grid)
+    dev = {k: _like(case.dev(a), dtype) for k, a in ins.items()}
+    csw = CGridShallowWaterDynamics(case.factory, grid, False, 0, nord)
     delpc, ptc = csw(*(dev[k] for k in names), 37.5)
     torch.cuda.synchronize()
     t = case.tile
@@ -265,6 +271,10 @@ def test_gpu_c_sw_strips_and_segments(n, nz, nord, cube_tiles):
         for name, got in list(dev.items()) + [("delpc", delpc), ("ptc", ptc)]:
             box = halo1 if name in ("delpc", "ptc", "omga") else full
             g, want = case.host(got)[ti][..., :nz][box], ref[name][box]
+            # the halo squares of corners with one edge hold the fill value's powers
+            g, want = g[np.abs(want) < 1e10], want[np.abs(want) < 1e10]
             # differences of neighbouring values: the fields' own scale bounds
-            # what a rounding in any term can move
-            assert np.abs(g - want).max() <= 1e-13 * np.abs(want).max(), (ti, name)
+            # what a rounding in any term can move, in FP32 by 2 ** 29 times as much
+            err = np.abs(g - want).max() / np.abs(want).max()
+            assert err <= (1e-13 if dtype == torch.float64 else 1e-13 * 2.0 ** 29), \
+                (ti, name, err)

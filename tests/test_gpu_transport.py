@@ -353,6 +353,41 @@ def test_fvtp2d_strips_and_segments(n, nz, tiles, hord, dtype):
     assert not a.any()
 
 
+# FP32 at the same sizes with every point bounded: hord 8, whose limiters choose
+# between values that meet where they switch.
+@pytest.mark.parametrize("n,nz,tiles", [(1, 2, 1), (3, 2, 1), (13, 2, 1), (58, 2, 1), (65, 2, 1),
+                                        (13, 79, 60), (59, 40, 48)])
+def test_fvtp2d_fp32_strips_and_segments(n, nz, tiles):
+    edges = (True, True, True, True)
+    d = {k: (v.astype(np.float32).astype(np.float64) if isinstance(v, np.ndarray) else v)
+         for k, v in transport_inputs(n, nz, workload=37).items()}
+    grid, damp = grid_from_numpy(d, dtype=torch.float32)
+    factory, gi = _factory(n, nz, edges)
+
+    def batch(a=None):
+        b = utils.zeros((tiles,) + gi.max_shape, dtype=torch.float32)
+        if a is not None:
+            b.copy_(torch.as_tensor(a, dtype=torch.float32))
+        return b
+
+    t = _tile(n, edges)
+    rqx, rqy = ofv.copy_corners_xy(d["q"], t)
+    fx, fy = batch(), batch()
+    FiniteVolumeTransport(factory, grid, damp, 0, 8)(
+        CopiedCorners(batch(d["q"]), batch(rqx), batch(rqy)), batch(d["crx"]), batch(d["cry"]),
+        batch(d["x_area_flux"]), batch(d["y_area_flux"]), fx, fy)
+    torch.cuda.synchronize()
+    rfx, rfy = ofv.fvtp2d(rqx, rqy, d["crx"], d["cry"], d["x_area_flux"], d["y_area_flux"],
+                          d["area"], d["dxa"], d["dya"], 8, t)
+    sx = (slice(3, n + 4), slice(3, n + 3))
+    sy = (slice(3, n + 3), slice(3, n + 4))
+    for tile in {0, tiles - 1}:
+        for got, ref, sl in ((fx, rfx, sx), (fy, rfy, sy)):
+            e = np.abs(to_np(got[tile])[sl].astype(np.float64) - ref[sl]).max()
+            e /= np.abs(ref[sl]).max()
+            assert e <= 16 * 2.0 ** -24, e * 2.0 ** 24
+
+
 # Tiles narrower than the corner windows (one to three cells, where one window
 # spans the tile) and as narrow as two windows, one and two strips along i, few
 # and many planes (short segments along j and one whole one), bands that mix
