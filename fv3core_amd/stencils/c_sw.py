@@ -48,7 +48,7 @@ class CGridShallowWaterDynamics:
         shape = batch_shape(self._grid_indexing, grid_data)
         self.delpc = utils.zeros(shape, dtype=grid_data.dx.dtype, device=grid_data.dx.device)
         self.ptc = utils.zeros(shape, dtype=grid_data.dx.dtype, device=grid_data.dx.device)
-        self._work = Workspace(7)
+        self._work = Workspace(3)
 
     def __call__(self, delp, pt, u, v, w, uc, vc, ua, va, ut, vt, divgd, omga, dt2: float):
         """Returns (delpc, ptc); uc, vc, ua, va, ut, vt, divgd, omga in place."""

@@ -32,7 +32,7 @@ class DGrid2AGrid2CGridVectors:
         self._grid_indexing = stencil_factory.grid_indexing
         self._grid_data = grid_data
         self._nk = self._grid_indexing.domain[2]
-        self._work = Workspace(2)
+        self._work = Workspace(1)
 
     def __call__(self, uc, vc, u, v, ua, va, utc, vtc):
         """uc, vc, ua, va, utc, vtc <- interpolations of the D-grid winds u, v."""

@@ -380,8 +380,8 @@ typedef struct fv3_metrics {
 /*
  * DGrid2AGrid2CGridVectors.__call__ (fv3core/stencils/d2a2c_vect.py:573-651):
  * D-grid winds u, v -> A-grid ua, va and C-grid uc, vc, utc, vtc, with the
- * tile-edge interpolations and corner fills.  work: 2 slabs of work_slab
- * elements, each addressed with the 3-D strides (left alone).
+ * tile-edge interpolations and corner fills.  work: 1 slab of work_slab
+ * elements (required, left alone).
  */
 int32_t fv3_d2a2c_vect_f64(const fv3_domain* d, const fv3_metrics* g, double* uc, double* vc,
                            const double* u, const double* v, double* ua, double* va,
@@ -394,7 +394,7 @@ int32_t fv3_d2a2c_vect_f64(const fv3_domain* d, const fv3_metrics* g, double* uc
  * pt in delpc, ptc (zero outside [isc-1, iec+1]^2 in the full domain).  delp,
  * pt and w get the reference's in-place corner fills; omga receives the
  * transported w; divgd is written on the compute corners when nord > 0.
- * work: 7 slabs (the first three hold uc and vc before the update, and ke).
+ * work: 3 slabs (uc and vc before the update, and ke).
  */
 int32_t fv3_c_sw_f64(const fv3_domain* d, const fv3_metrics* g, int32_t nord, double dt2,
                      double* delp, double* pt, const double* u, const double* v, double* w,
