@@ -19,9 +19,9 @@
 // waves a workgroup, tiles spread over the XCDs or kept on one and non-temporal
 // stores all measure within 10 %).  31 passes over full-size fields against 54
 // of one pointwise pass per stencil.  Measured, FP64, 79 levels: six C97 tiles
-// 593 -> 420 us (d2a2c 169 -> 126, transport with the divergence 301 -> 195,
+// 593 -> 423 us (d2a2c 169 -> 126, transport with the divergence 301 -> 195,
 // update with the vorticity 112 -> 97); 96 C48 tiles in FP32 1510 -> 975 us;
-// six C12 tiles, where a launch is its latency, 52 us as before.
+// six C12 tiles, where a launch is its latency, 52 -> 47 us.
 #include "strip.hpp"
 #include "stencil.hpp"
 

@@ -38,7 +38,7 @@ namespace fv3 {
 constexpr int DN_W = 64;            // lanes = strip columns
 constexpr int DN_TI = DN_W - 6;     // interfaces per strip in i
 constexpr int DN_NY = FV3_DN_NY;    // strips (waves) per workgroup
-constexpr int DN_WIN = 100;         // cells of a corner window (at most 10 x 10)
+constexpr int DN_WIN = 81;          // cells of a corner window (at most 9 x 9)
 
 // The march's cost.  FP64 (two extra passes) measured in the acoustic call, FP32
 // on the launch alone: [1, 1, 1, 1] on six C48 tiles, 79 levels, 19.4 us by the

@@ -7,7 +7,8 @@
 //
 // Reference: fv3core/stencils/updatedzc.py, updatedzd.py, nh_p_grad.py,
 // pk3_halo.py, pe_halo.py, ray_fast.py, del2cubed.py, temperature_adjust.py
-// and dyn_core.py:47-145.  Vertical recurrences run one column per lane.
+// and dyn_core.py:47-145.  Vertical recurrences run one column per
+// lane, or levels at once where only a floor passes between them.
 #include "kernels.hpp"
 
 #include <algorithm>

@@ -1,7 +1,8 @@
 """RiemannSolver3 (fv3core/stencils/riem_solver3.py:106-242) on the GPU.
 
 precompute, sim1_solver and finalize run as one FP64 kernel
-(``fv3_riem_solver3``), one column per lane.
+(``fv3_riem_solver3``): a column's levels over a workgroup, or one column per
+thread where that takes less time.
 """
 from __future__ import annotations
 

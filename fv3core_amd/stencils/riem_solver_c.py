@@ -1,7 +1,8 @@
 """RiemannSolverC (fv3core/stencils/riem_solver_c.py:67-165) on the GPU.
 
 precompute, sim1_solver and finalize run as one FP64 kernel
-(``fv3_riem_solver_c``), one column per lane.
+(``fv3_riem_solver_c``): a column's levels over a workgroup, or one column per
+thread where that takes less time.
 """
 from __future__ import annotations
 

@@ -1,7 +1,8 @@
 """UpdateGeopotentialHeightOnCGrid (fv3core/stencils/updatedzc.py:106-163) on the GPU.
 
 ``fv3_update_dz_c`` evaluates the corner-filled copies of gz on the fly,
-advances gz one column per lane and applies the DZ_MIN floor; a second
+advances gz with 64 columns and a chunk of their levels to a workgroup, and
+applies the DZ_MIN floor; a second
 launch copies the result back into gz (neighbouring columns read the old gz).
 """
 from __future__ import annotations
