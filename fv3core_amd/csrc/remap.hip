@@ -335,9 +335,11 @@ enum MapForm { kMapSweeps = 0, kMapFused = 1, kMapLayers = 2 };
 // cache (137 layers, six C128 tiles: 531 against 597 us; 96 C48 tiles 1204
 // against 1698 us).  In FP32 the lines lie where its own times put them.  The
 // rates are those of calls on data that the last one left in the caches; on cold
-// data the one-thread forms, which read a column four times, take 5 to 25 % more
-// and the spread form the same, hence kColumnCold.
-constexpr double kColumnCold = 1.15;
+// data the four sweeps, which read a column four times, take 5 to 25 % more, the
+// fused form up to 15 % and the spread form the same, hence the two factors (100
+// layers, six C128 tiles, fused against spread: 383 and 436 us warm, 389 and 437
+// cold; 32 layers on 96 C48 tiles in FP32 135 and 117, 151 and 118).
+constexpr double kSweepsCold = 1.15, kFusedCold = 1.06;
 static MapForm map_form(int km, int64_t waves, bool fp32) {
   const double w = (double)waves;
   const bool fused = waves >= 2 * kSimdsPerGpu ||
@@ -361,7 +363,8 @@ static MapForm map_form(int km, int64_t waves, bool fp32) {
   else
     busy = fp32 ? 0.35 + 0.0013 * w : 0.7 + 0.0021 * w;
   const double lone = fp32 ? std::min(1.75, 1.35 + 0.008 * w) : std::min(2.3, 1.5 + 0.01 * w);
-  return kColumnCold * (3.0 + km * std::max(lone, busy)) < layers ? column : kMapLayers;
+  const double cold = fused ? kFusedCold : kSweepsCold;
+  return cold * (3.0 + km * std::max(lone, busy)) < layers ? column : kMapLayers;
 }
 
 template <typename T>
